@@ -24,6 +24,8 @@ namespace exa {
 using C192 = GemmCfg<192, 192, 2, 4, 16>;
 using C128 = GemmCfg<128, 128, 2, 2, 16>;
 using CT64 = GemmCfg<64, 64, 2, 2, 16>;
+// The FP64 column stage's blocks (gemm_nt_pipe, two work-groups per CU).
+using CP192 = GemmCfg<96, 192, 2, 2, 16>;
 
 // P_j = L_jk X_kk for j in (k, mt), stored transposed (tile j of P holds
 // P_j^T, column-major), so the two consumers read it row-major.
@@ -91,34 +93,45 @@ __device__ __forceinline__ void takahashi_unit(const TileView& v, int k, const d
     if (nsplit == 1) acc32_store_t<C>(acc, tile_f64(U, m, k) + bj * C::BN + (long)bi * C::BM * ts, ts);
     return;
   }
+  double* out = nsplit > 1 ? W + ((long)sp * below + (m - k - 1)) * ts * ts : tile_f64(v, m, k);
+  out += bi * C::BM + (long)bj * C::BN * ts;
   dx4 acc[C::FM][C::FN];
   zero_acc<C>(acc);
+  if constexpr (HAS_U) {
+    // A(r, kk) = Z(m, j)[bi*BM + r, kk]: tile (m, j) of Z for j <= m, Z_jm^T
+    // from U for j > m; B(c, kk) = P_j^T[bj*BN + c, kk]
+    gemm_nt_pipe<C, 2>(
+        acc, j_hi - j_lo,
+        [&](int s, const double*& A, const double*& B) {
+          const int j = j_lo + s;
+          A = (j <= m ? tile_f64(v, m, j) : tile_f64(U, j, m)) + bi * C::BM;
+          B = P + (long)j * ts * ts + bj * C::BN;
+        },
+        ts, (int)ts, lds);
+    pipe_put_neg<C>(acc, out, ts);
+    if (nsplit == 1) pipe_put_neg_t<C>(acc, tile_f64(U, m, k) + bj * C::BN + (long)bi * C::BM * ts, ts);
+  } else {
 #pragma unroll 1
-  for (int j = j_lo; j < j_hi; ++j) {
-    const double* B = P + (long)j * ts * ts + bj * C::BN;  // B(c, kk) = P_j^T[bj*BN + c, kk]
-    if constexpr (HAS_U) {
-      // A(r, kk) = Z(m, j)[bi*BM + r, kk]: tile (m, j) of Z for j <= m, Z_jm^T from U for j > m
-      const double* A = (j <= m ? tile_f64(v, m, j) : tile_f64(U, j, m)) + bi * C::BM;
-      gemm_nt_ring<C>(acc, A, ts, B, ts, (int)ts, lds, -1.0);
-    } else if (j <= m) {
-      gemm_nt_acc<C>(acc, tile_f64(v, m, j) + bi * C::BM, ts, B, ts, (int)ts, lds, -1.0);
-    } else {
-      const double* A = tile_f64(v, j, m) + (long)bi * C::BM * ts;  // A(r, kk) = Z_jm[kk, bi*BM + r]
-      gemm_nt_acc<C, false, double, double, true>(acc, A, ts, B, ts, (int)ts, lds, -1.0);
+    for (int j = j_lo; j < j_hi; ++j) {
+      const double* B = P + (long)j * ts * ts + bj * C::BN;  // B(c, kk) = P_j^T[bj*BN + c, kk]
+      if (j <= m) {
+        gemm_nt_acc<C>(acc, tile_f64(v, m, j) + bi * C::BM, ts, B, ts, (int)ts, lds, -1.0);
+      } else {
+        const double* A = tile_f64(v, j, m) + (long)bi * C::BM * ts;  // A(r, kk) = Z_jm[kk, bi*BM + r]
+        gemm_nt_acc<C, false, double, double, true>(acc, A, ts, B, ts, (int)ts, lds, -1.0);
+      }
     }
+    acc_update<C>(acc, out, ts, 0.0);
   }
-  double* out = nsplit > 1 ? W + ((long)sp * below + (m - k - 1)) * ts * ts : tile_f64(v, m, k);
-  acc_update<C>(acc, out + bi * C::BM + (long)bj * C::BN * ts, ts, 0.0);
-  if constexpr (HAS_U)
-    if (nsplit == 1) acc_store_t<C>(acc, tile_f64(U, m, k) + bj * C::BN + (long)bi * C::BM * ts, ts);
 }
 
 template <class C, bool HAS_U, bool F32 = false>
-__global__ void __launch_bounds__(C::NT) k_takahashi_col(TileView v, int k, const double* P, double* W, int nsplit,
+__global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(HAS_U && !F32 ? 2 : 1)))
+    k_takahashi_col(TileView v, int k, const double* P, double* W, int nsplit,
                                                          TileView U, long units, int nx) {
   static_assert(!F32 || HAS_U, "the FP32 column stage reads the transposed copy");
   __shared__ __attribute__((aligned(16))) double lds[F32 ? C::LDS_DOUBLES / 2
-                                                         : (HAS_U ? RingLds<C>::DOUBLES : C::LDS_DOUBLES)];
+                                                         : (HAS_U ? PipeLds<C, 2>::DOUBLES : C::LDS_DOUBLES)];
   const int w = blockIdx.x;
   const int x = w % nx;
   const int gx = gridDim.x / nx;
@@ -201,14 +214,14 @@ __global__ void k_sum_tiles(const double* Q, int cnt, long len, double* out) {
 // one tile per range, and only as many as the slab buffer holds) whose work
 // units fill whole rounds of the concurrent work-groups best; each extra
 // range costs a write and a read of its slab, counted as 2% per range.
-template <class C, bool F32 = false>
+template <class C, bool HAS_U, bool F32>
 static int takahashi_splits(const TileView& v, int k, int max_split, int* slots_out) {
   static int slots = 0;
   if (!slots) {
     int dev = 0, cus = 0, occ = 1;
     EXA_HIP(hipGetDevice(&dev));
     EXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_takahashi_col<C, true, F32>, C::NT, 0));
+    EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_takahashi_col<C, HAS_U, F32>, C::NT, 0));
     slots = cus * (occ > 0 ? occ : 1);
     if (slots >= 8) slots -= slots % 8;
   }
@@ -230,7 +243,7 @@ static int takahashi_splits(const TileView& v, int k, int max_split, int* slots_
   return best;
 }
 
-template <class C>
+template <class C, class CP>
 static void takahashi_cfg(const TileView& v, int k, const double* X, double* P, double* Q, double* W, int max_split,
                           const TileView& U, int stage, hipStream_t s, bool f32) {
   const long per = (long)(v.ts / C::BM) * (v.ts / C::BN);
@@ -240,9 +253,13 @@ static void takahashi_cfg(const TileView& v, int k, const double* X, double* P, 
   if (stage == 1 && below > 0) {
     int slots = 0;
     const bool f32u = f32 && U.ptr;
-    const int ns = f32u ? takahashi_splits<C, true>(v, k, W ? max_split : 1, &slots)
-                        : takahashi_splits<C>(v, k, W ? max_split : 1, &slots);
-    const long units = below * per * ns;
+    const bool pipe = U.ptr && !f32;
+    const int ms = W ? max_split : 1;
+    const int ns = f32u ? takahashi_splits<C, true, true>(v, k, ms, &slots)
+                        : (pipe ? takahashi_splits<CP, true, false>(v, k, ms, &slots)
+                                : takahashi_splits<C, false, false>(v, k, ms, &slots));
+    const long per_col = pipe ? (long)(v.ts / CP::BM) * (v.ts / CP::BN) : per;
+    const long units = below * per_col * ns;
     // persistent grid: at most one round of resident work-groups, a
     // multiple of the 8 XCDs when it is that large
     long grid = units < slots ? units : slots;
@@ -253,7 +270,7 @@ static void takahashi_cfg(const TileView& v, int k, const double* X, double* P, 
       hipLaunchKernelGGL((k_takahashi_col<C, true, true>), dim3((unsigned)grid), dim3(C::NT), 0, s, v, k,
                          (const double*)P, W, ns, U, units, nx);
     else if (U.ptr)
-      hipLaunchKernelGGL((k_takahashi_col<C, true>), dim3((unsigned)grid), dim3(C::NT), 0, s, v, k,
+      hipLaunchKernelGGL((k_takahashi_col<CP, true>), dim3((unsigned)grid), dim3(CP::NT), 0, s, v, k,
                          (const double*)P, W, ns, U, units, nx);
     else
       hipLaunchKernelGGL((k_takahashi_col<C, false>), dim3((unsigned)grid), dim3(C::NT), 0, s, v, k,
@@ -274,9 +291,9 @@ void launch_takahashi_stage(const TileView& v, int k, const double* X, double* P
                             int stage, hipStream_t s, double* W, int max_split, const TileView* U, bool f32) {
   TileView u{};
   if (U) u = *U;
-  if (v.ts % 192 == 0) takahashi_cfg<C192>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
-  else if (v.ts % 128 == 0) takahashi_cfg<C128>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
-  else takahashi_cfg<CT64>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
+  if (v.ts % 192 == 0) takahashi_cfg<C192, CP192>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
+  else if (v.ts % 128 == 0) takahashi_cfg<C128, C128>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
+  else takahashi_cfg<CT64, CT64>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
   if (stage == 2) {
     const long len = (long)v.ts * v.ts;
     hipLaunchKernelGGL(k_sum_tiles, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, s, (const double*)Q,

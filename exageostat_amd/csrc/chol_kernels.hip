@@ -287,10 +287,7 @@ void launch_trtri_tiles(const TileView& v, const double* dinv, double* xinv, hip
 // CUs) loop over the block list.  Work-groups are dispatched round-robin
 // over the XCDs, so work-group w runs on XCD w % nx; each XCD gets a
 // contiguous slice of the block list and its work-groups walk it together,
-// which keeps the A/B row panels they share hot in that XCD's L2.  The
-// operands go through the three-stage direct-to-LDS ring (gemm_nt_ring):
-// 2.5% faster at n = 90,000 than register-staged double buffering, with
-// the same products in the same order.
+// which keeps the A/B row panels they share hot in that XCD's L2.
 template <class C>
 __device__ __forceinline__ void update_block(const TileView& v, int k, int np, int col_lo, int col_hi, long b,
                                              double* lds) {
@@ -317,19 +314,20 @@ __device__ __forceinline__ void update_block(const TileView& v, int k, int np, i
   double* Cp = tile_f64(v, m, n) + bi * C::BM + (long)bj * C::BN * v.ts;
   dx4 acc[C::FM][C::FN];
   zero_acc<C>(acc);
-#pragma unroll 1
-  for (int p = 0; p < np; ++p) {
-    const double* A = tile_f64(v, m, k + p) + bi * C::BM;
-    const double* B = tile_f64(v, n, k + p) + bj * C::BN;
-    gemm_nt_ring<C>(acc, A, v.ts, B, v.ts, v.ts, lds, -1.0);
-  }
-  acc_update<C>(acc, Cp, v.ts, 1.0);
+  gemm_nt_pipe<C, 2>(
+      acc, np,
+      [&](int s, const double*& A, const double*& B) {
+        A = tile_f64(v, m, k + s) + bi * C::BM;
+        B = tile_f64(v, n, k + s) + bj * C::BN;
+      },
+      v.ts, v.ts, lds);
+  pipe_sub<C>(acc, Cp, v.ts);
 }
 
 template <class C>
-__global__ void __launch_bounds__(C::NT) k_tile_update(TileView v, int k, int np, int col_lo, int col_hi,
+__global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2))) k_tile_update(TileView v, int k, int np, int col_lo, int col_hi,
                                                       long nblocks, int nx) {
-  __shared__ __attribute__((aligned(16))) double lds[RingLds<C>::DOUBLES];
+  __shared__ __attribute__((aligned(16))) double lds[PipeLds<C, 2>::DOUBLES];
   const int w = blockIdx.x;
   const int x = w % nx;
   const int gx = gridDim.x / nx;
@@ -384,7 +382,7 @@ void launch_tile_update(const TileView& v, int k, int np, int col_lo, int col_hi
   if (col_lo >= v.mt || col_hi < col_lo) return;
   if (np < 1 || np > 2 || col_lo < k + np) throw std::invalid_argument("tile_update: bad panel count or columns");
   if (v.ts % 192 == 0) {
-    launch_update_cfg<GemmCfg<192, 192, 2, 4, 16>>(v, k, np, col_lo, col_hi, s);
+    launch_update_cfg<GemmCfg<96, 192, 2, 2, 16>>(v, k, np, col_lo, col_hi, s);
   } else if (v.ts % 128 == 0) {
     launch_update_cfg<GemmCfg<128, 128, 2, 2, 16>>(v, k, np, col_lo, col_hi, s);
   } else {

@@ -4,8 +4,8 @@
 // memory.  A and B are staged through LDS in BK-deep slices, either with
 // register-staged double buffering (gemm_nt_acc: global loads of slice k+1
 // are in flight while slice k feeds the matrix cores; FP32 and K-major
-// operands) or with direct-to-LDS copies into a three-stage ring
-// (gemm_nt_ring: plain FP64 operands).  Each 64-lane wave owns a WM x WN
+// operands) or with direct-to-LDS copies into a ring and software-pipelined
+// fragments (gemm_nt_pipe: plain FP64 operands).  Each 64-lane wave owns a WM x WN
 // sub-block made of 16x16 fragments of v_mfma_f64_16x16x4f64.
 #pragma once
 
@@ -217,89 +217,210 @@ __device__ __forceinline__ void gemm_nt_acc(dx4 (&acc)[C::FM][C::FN], const TA* 
   }
 }
 
-// The same product with the operands copied straight into a three-stage LDS
-// ring by global_load_lds_dwordx4 (no staging registers, no LDS stores from
-// registers), as the BF16 classes do.  Stage layout: A as BK columns of BM
-// doubles (column-major, no padding: each 16-lane quarter of a fragment
-// read takes 16 consecutive doubles), then B likewise; a wave-wide copy
-// fills 1,024 contiguous LDS bytes, lane l taking the two doubles
-// 128 q + 2 l of its operand's stage array, gathered from their (row,
-// column) in the tile.  At step kc each wave waits for its own copies of
-// slice kc, a bare barrier makes every wave's copies visible and ends the
-// reads of slice kc-1, whose buffer then receives slice kc+2.  Plain FP64
-// operands (not K-major); K a multiple of BK; A, B 16-byte aligned, lda and
-// ldb even.
-template <class C>
-struct RingLds {
+// The same product for plain FP64 operands, software-pipelined, with the
+// fragments the other way round: acc[i][j] holds the block of rows
+// 16 i .. and columns 16 j .. with lane l, element v at row l%16, column
+// l/16 + 4 v (v_mfma_f64_16x16x4f64 with B's fragment as its first operand),
+// so 16 lanes of an access to a column-major block are 128 contiguous bytes.
+// The products and their order of summation are those of gemm_nt_acc.
+//
+// Bound by the FP64 matrix cores (64 cycles per instruction and SIMD).  What
+// keeps them fed, with 15,360 x 15,360 x 1,920 blocks over the whole card
+// (the same loop with 192 x 192 blocks, one work-group per CU, unpipelined
+// fragments: 62.7 TFLOP/s):
+//   * NST-stage LDS ring filled by global_load_lds_dwordx4 (no staging
+//     registers): slice kc + NST is requested as soon as slice kc is in
+//     registers;
+//   * the fragments of the next four k are read from LDS while the current
+//     four are multiplied, also across slices, so that no wave waits for LDS
+//     after a barrier (192 x 192: 67.7 TFLOP/s);
+//   * two 256-thread work-groups per CU, so that one multiplies while the
+//     other is at a barrier or writes its block out (96 x 192: 71.5,
+//     128 x 128: 68.4, 64 x 64: 60.9 TFLOP/s).
+// Stage layout: A as BK columns of BM doubles, then B; odd columns have
+// neighbouring groups of 16 rows exchanged (row ^ 16), so the two columns
+// that one LDS pass reads lie in different halves of the banks (5.6% of the
+// LDS cycles were conflicts without).  A wave-wide copy fills 1,024
+// contiguous LDS bytes, lane l taking elements 128 q + 2 l.
+// Operands: segment s (0 <= s < nseg) multiplies A_s B_s^T with K columns,
+// both from seg(s, A, B) with the leading dimension ld (even; pointers
+// 16-byte aligned); K a multiple of BK.
+template <class C, int NST>
+struct PipeLds {
   static constexpr int A_ST = C::BK * C::BM, B_ST = C::BK * C::BN;  // doubles per stage
   static constexpr int STAGE = A_ST + B_ST;
-  static constexpr int DOUBLES = 3 * STAGE;
+  static constexpr int DOUBLES = NST * STAGE;
   static constexpr int A_COPIES = A_ST / 128, B_COPIES = B_ST / 128;
   static constexpr int PER_WAVE = (A_COPIES + B_COPIES) / C::NW;
   static_assert(A_ST % 128 == 0 && B_ST % 128 == 0, "stage arrays must be whole 1 KB copies");
   static_assert(PER_WAVE * C::NW == A_COPIES + B_COPIES, "copies must split evenly over the waves");
-  static_assert(PER_WAVE < 32, "vmcnt range");
+  static_assert(C::BM % 32 == 0 && C::BN % 32 == 0, "row groups are exchanged in pairs");
+  static_assert(NST >= 2 && NST * PER_WAVE < 64, "vmcnt range");
 };
 
-template <class C>
-__device__ __forceinline__ void gemm_nt_ring(dx4 (&acc)[C::FM][C::FN], const double* __restrict__ A, long lda,
-                                             const double* __restrict__ B, long ldb, int K, double* lds,
-                                             double sign) {
-  using L = RingLds<C>;
+// Waits until at most n vector-memory operations and no LDS operation of
+// this wave are pending.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt_lgkm0() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4));
+}
+
+template <class C, int NST, class SEG>
+__device__ __forceinline__ void gemm_nt_pipe(dx4 (&acc)[C::FM][C::FN], int nseg, const SEG& seg, long ld, int K,
+                                             double* lds) {
+  using L = PipeLds<C, NST>;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / C::WGN;
   const int wn = wave - wm * C::WGN;
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);
-  auto issue = [&](int kc, int buf) {
-    const int k0 = kc * C::BK;
+  const int per_seg = K / C::BK;
+  const int nk = nseg * per_seg;
+  if (nk <= 0) return;
+  uint32_t off[L::PER_WAVE];  // byte offset of this lane's element in a slice of its operand
+#pragma unroll
+  for (int j = 0; j < L::PER_WAVE; ++j) {
+    int c = wave * L::PER_WAVE + j;
+    const bool is_b = c >= L::A_COPIES;
+    if (is_b) c -= L::A_COPIES;
+    const int rows = is_b ? C::BN : C::BM;
+    const int e = c * 128 + 2 * lane;
+    const int kk = e / rows;
+    const int r = (e - kk * rows) ^ ((kk & 1) * 16);
+    off[j] = (uint32_t)((r + kk * (int)ld) * 8);
+  }
+  const double *A, *B;
+  seg(0, A, B);
+  int s_next = 1, left = per_seg;  // next segment, slices left in the current one
+  auto issue = [&](int buf) {
+    if (left == 0) {
+      seg(s_next++, A, B);
+      left = per_seg;
+    }
 #pragma unroll
     for (int j = 0; j < L::PER_WAVE; ++j) {
-      int c = wave_s * L::PER_WAVE + j;
+      int c = wave * L::PER_WAVE + j;
       const bool is_b = c >= L::A_COPIES;
       if (is_b) c -= L::A_COPIES;
-      const int rows = is_b ? C::BN : C::BM;
-      const int e = c * 128 + 2 * lane;  // element of the operand's stage array
-      const int kk = e / rows;
-      const int r = e - kk * rows;
-      const double* src = is_b ? B + r + (long)(k0 + kk) * ldb : A + r + (long)(k0 + kk) * lda;
+      const char* src = reinterpret_cast<const char*>(is_b ? B : A) + off[j];
       double* dst = lds + buf * L::STAGE + (is_b ? L::A_ST : 0) + c * 128;
       __builtin_amdgcn_global_load_lds((glb_void_t*)(uintptr_t)src, (lds_void_t*)dst, 16, 0, 0);
     }
+    A += (long)C::BK * ld;
+    B += (long)C::BK * ld;
+    --left;
   };
-  auto compute = [&](int buf) {
-    const double* Ab = lds + buf * L::STAGE + wm * C::WM + (lane & 15);
-    const double* Bb = lds + buf * L::STAGE + L::A_ST + wn * C::WN + (lane & 15);
+  const int flip = ((lane >> 4) & 1) * 16;
+  const int a0 = wm * C::WM, b0 = wn * C::WN;
+  const int ao = (lane & 15) + (lane >> 4) * C::BM;
+  const int bo = (lane & 15) + (lane >> 4) * C::BN + L::A_ST;
+  double a[2][C::FM], b[2][C::FN];
+  auto frag = [&](int set, int buf, int kk) {
+    const double* Ab = lds + buf * L::STAGE + ao + kk * 4 * C::BM;
+    const double* Bb = lds + buf * L::STAGE + bo + kk * 4 * C::BN;
 #pragma unroll
-    for (int kk = 0; kk < C::BK; kk += 4) {
-      const int krow = kk + (lane >> 4);
-      double a[C::FM], b[C::FN];
+    for (int i = 0; i < C::FM; ++i) a[set][i] = Ab[(a0 + i * 16) ^ flip];
 #pragma unroll
-      for (int i = 0; i < C::FM; ++i) a[i] = sign * Ab[krow * C::BM + i * 16];
+    for (int j = 0; j < C::FN; ++j) b[set][j] = Bb[(b0 + j * 16) ^ flip];
+  };
+  constexpr int NK = C::BK / 4;
+  static_assert(NK % 2 == 0, "the two fragment sets alternate over a slice");
+  // The ring may still be read by the previous block's last steps.
+  __builtin_amdgcn_s_barrier();
 #pragma unroll
-      for (int j = 0; j < C::FN; ++j) b[j] = Bb[krow * C::BN + j * 16];
+  for (int st = 0; st < NST; ++st)
+    if (st < nk) issue(st);
+  if (nk >= NST) wait_vmcnt<(NST - 1) * L::PER_WAVE>();
+  else wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();
+  frag(0, 0, 0);
+  int buf = 0;
+#pragma unroll 1
+  for (int kc = 0; kc < nk; ++kc) {
+    const int nbuf = buf == NST - 1 ? 0 : buf + 1;
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+      const int cur = kk & 1, nxt = cur ^ 1;
+      if (kk + 1 < NK) {
+        frag(nxt, buf, kk + 1);
+      } else if (kc + 1 < nk) {
+        // Slice kc + 1 has landed, and every wave holds its last fragments
+        // of slice kc, whose buffer can be filled again.
+        __builtin_amdgcn_sched_barrier(0);
+        if (kc + NST - 1 < nk) wait_vmcnt_lgkm0<(NST - 2) * L::PER_WAVE>();
+        else wait_vmcnt_lgkm0<0>();
+        __builtin_amdgcn_s_barrier();
+        if (kc + NST < nk) issue(buf);
+        frag(nxt, nbuf, 0);
+      }
 #pragma unroll
       for (int i = 0; i < C::FM; ++i)
 #pragma unroll
-        for (int j = 0; j < C::FN; ++j) acc[i][j] = mfma_f64(a[i], b[j], acc[i][j]);
+        for (int j = 0; j < C::FN; ++j) acc[i][j] = mfma_f64(b[cur][j], a[cur][i], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  };
-  const int nk = K / C::BK;
-  if (nk <= 0) return;
-  // The ring may still be read by the previous block's last steps.
-  __builtin_amdgcn_s_barrier();
-  issue(0, 0);
-  if (nk > 1) issue(1, 1);
-  int buf = 0;
-  for (int kc = 0; kc < nk; ++kc) {
-    if (kc + 1 < nk) wait_vmcnt<L::PER_WAVE>();
-    else wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-    if (kc + 2 < nk) issue(kc + 2, buf == 0 ? 2 : buf - 1);
-    compute(buf);
-    buf = buf == 2 ? 0 : buf + 1;
+    buf = nbuf;
   }
+}
+
+// Base pointer of this lane's elements of a block in gemm_nt_pipe's layout.
+template <class C>
+__device__ __forceinline__ auto pipe_base(double* Cp, long ldc) {
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int wm = wave / C::WGN;
+  const int wn = wave - wm * C::WGN;
+  typedef __attribute__((address_space(1))) double gD;
+  return (gD*)(uintptr_t)(Cp + wm * C::WM + (lane & 15) + (long)(wn * C::WN + (lane >> 4)) * ldc);
+}
+
+// C -= acc, one fragment column at a time with all its reads before its
+// writes.
+template <class C>
+__device__ __forceinline__ void pipe_sub(const dx4 (&acc)[C::FM][C::FN], double* Cp, long ldc) {
+  auto* G = pipe_base<C>(Cp, ldc);
+#pragma unroll
+  for (int j = 0; j < C::FN; ++j) {
+    double cv[4][C::FM];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int i = 0; i < C::FM; ++i) cv[v][i] = G[i * 16 + (long)(j * 16 + 4 * v) * ldc];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int i = 0; i < C::FM; ++i) G[i * 16 + (long)(j * 16 + 4 * v) * ldc] = cv[v][i] - acc[i][j][v];
+  }
+}
+
+// C = -acc.
+template <class C>
+__device__ __forceinline__ void pipe_put_neg(const dx4 (&acc)[C::FM][C::FN], double* Cp, long ldc) {
+  auto* G = pipe_base<C>(Cp, ldc);
+#pragma unroll
+  for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int i = 0; i < C::FM; ++i) G[i * 16 + (long)(j * 16 + 4 * v) * ldc] = -acc[i][j][v];
+}
+
+// Cp[c + r*ldc] = -acc(r, c): the block stored transposed.
+template <class C>
+__device__ __forceinline__ void pipe_put_neg_t(const dx4 (&acc)[C::FM][C::FN], double* Cp, long ldc) {
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int wm = wave / C::WGN;
+  const int wn = wave - wm * C::WGN;
+  typedef __attribute__((address_space(1))) double gD;
+  gD* G = (gD*)(uintptr_t)(Cp + wn * C::WN + (lane >> 4) + (long)(wm * C::WM + (lane & 15)) * ldc);
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) G[j * 16 + 4 * v + (long)(i * 16) * ldc] = -acc[i][j][v];
 }
 
 // C[r + c*ldc] = beta*C + acc for the block owned by this work-group.
