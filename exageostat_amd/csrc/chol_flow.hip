@@ -1,0 +1,760 @@
+// Dataflow Cholesky: a whole range of 64-column blocks factored in one
+// launch, by work-groups that claim block tasks in order and wait on
+// per-row progress counters instead of on kernel boundaries.
+//
+// Replaces, for matrices whose factorisation is bound by its serial chain of
+// panels, CHAMELEON_dpotrf_Tile(ChamLower, C) as called from
+// EXAGEOSTAT_dmle_Tile (exageostat_exact/src/compute/MLE_dexact.c:372); the
+// same kernel factors one tile column (diagonal tile and panel) of the
+// larger matrices' right-looking tile Cholesky.
+//
+// Left-looking in blocks of 64: with L_il final for l < j,
+//   D_j  (one task per block column j): block (j, j-1) and the diagonal:
+//        L_{j,j-1} = (A_{j,j-1} - sum_l L_jl L_{j-1,l}^T) inv(L_{j-1,j-1})^T,
+//        L_jj = chol(A_jj - sum_l L_jl L_jl^T), and inv(L_jj);
+//   T_ij (block rows i > j+1, one or two of them per task):
+//        L_ij = (A_ij - sum_l L_il L_jl^T) inv(L_jj)^T.
+// The sums run as far as their operands are final and then wait for the
+// next ones, so the serial chain is, per 64 columns: one 64^3 product, one
+// symmetric 64^2 x 64 product, the factorisation and inverse of one 64 x 64
+// block, and the hand-over to the next D task.  Everything else runs beside
+// it on the other work-groups.
+//
+// Progress: tasks are claimed from one counter in an order in which every
+// task depends on earlier ones only (D_j first in its column), and a
+// work-group finishes its task before it claims another: the oldest
+// unfinished task never waits on an unclaimed one, so the launch drains
+// whatever share of its work-groups is resident, down to a single one.
+//
+// Memory: finished blocks are written through to the device's coherence
+// point (agent-scope stores), then the row's counter is released at agent
+// scope; a waiting work-group acquires at agent scope before it reads.
+#include "common.hpp"
+#include "besselk.hpp"
+#include "kernels.hpp"
+#include "mfma.hpp"
+
+namespace exa {
+
+namespace {
+
+// Counters, one per 64 bytes.
+constexpr int kClaim = 0, kExit = 16, kDiag = 32, kRows = 48;
+
+__device__ __forceinline__ int flag_get(const int* f) {
+  return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Every wave's stores have left the wave; to be called before the barrier
+// that precedes flag_set.
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void flag_set(int* f, int v) {
+  __hip_atomic_store(f, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void store_through(T* p, T v) {
+  typedef __attribute__((address_space(1))) T gT;
+  __hip_atomic_store((gT*)(uintptr_t)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ double lane_value(double x, int lane) {
+  const long u = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)u, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
+  return __longlong_as_double(((long)hi << 32) | (unsigned)lo);
+}
+
+// 1/sqrt(x) and sqrt(x) for normal x > 0: the hardware estimate refined by
+// two coupled Newton steps and one correction of the root.
+__device__ __forceinline__ void rsqrt_pair(double x, double& rs, double& s) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  s = fma(fma(-g, g, x), h, g);
+  rs = h + h;
+}
+
+// Factors a 16-column panel held one row per lane (the diagonal block's rows
+// in lanes 0 .. 15), by the square-root-free elimination
+//   a_{r,c2} -= (a_rc / d_c) a_{c2,c},  d_c = a_cc,
+// whose columns are scaled by 1/sqrt(d_c) off the dependent chain (a
+// reciprocal per column on it, instead of a reciprocal square root and a
+// product).  Rows below the diagonal block come out as rows of L, rows of an
+// identity as rows of L^-T.  Returns the mask of columns whose pivot is not
+// positive; those and all later columns are NaN then.
+__device__ __forceinline__ unsigned panel16(double (&a)[16], int lane) {
+  unsigned bad = 0;
+  double root[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    const double piv = lane_value(a[c], c);
+    bad |= (piv > 0.0) ? 0u : (1u << c);
+    const double b = a[c] * recip(piv);
+#pragma unroll
+    for (int c2 = c + 1; c2 < 16; ++c2) a[c2] = fma(-b, lane_value(a[c], c2), a[c2]);
+    double rs;
+    rsqrt_pair(piv, rs, root[c]);
+    a[c] *= rs;
+  }
+#pragma unroll
+  for (int c = 0; c < 16; ++c)
+    if (lane == c) a[c] = root[c];
+  if (bad) {
+    const int first = __builtin_ctz(bad);
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+      if (c >= first) a[c] = __builtin_nan("");
+  }
+  return bad;
+}
+
+// 16 x 16 block (bi, bj), bi >= bj, of a 64 x 64 lower matrix kept as ten
+// blocks, each column-major: the fragment of four columns that a wave feeds
+// to one MFMA is 64 consecutive doubles.
+__device__ __forceinline__ constexpr int blk16(int bi, int bj) { return (bi * (bi + 1) / 2 + bj) * 256; }
+
+// The diagonal fragments (bi, bj) of the 64 x 64 lower triangle by wave:
+// at most three each.
+__device__ __forceinline__ int diag_count(int w) { return (w == 1 || w == 2) ? 3 : 2; }
+__device__ __forceinline__ void diag_frag(int w, int t, int& bi, int& bj) {
+  // w0: (0,0) (3,0); w1: (1,0) (1,1) (3,1); w2: (2,0) (2,1) (2,2); w3: (3,2) (3,3)
+  if (w == 0) {
+    bi = t ? 3 : 0;
+    bj = 0;
+  } else if (w == 1) {
+    bi = t == 2 ? 3 : 1;
+    bj = t == 0 ? 0 : 1;
+  } else if (w == 2) {
+    bi = 2;
+    bj = t;
+  } else {
+    bi = 3;
+    bj = 2 + t;
+  }
+}
+
+}  // namespace
+
+struct FlowArgs {
+  TileView v;
+  double* pool;   // all tiles FP64 and contiguous: the whole matrix is in range; null: one tile column only
+  int k;          // that tile column
+  int q;          // 64-blocks per tile side
+  int j0, j1;     // block columns factored; updates from columns < j0 are already in the matrix
+  int i_end;      // one past the last block row
+  int j_pad;      // block columns [j1, j_pad) are padding: their inverses are the identity
+  double* dinv;   // inverse of diagonal block j at dinv + 4096 j
+  int* info;
+  int* flags;
+};
+
+namespace {
+
+// Block row i of the matrix: its tile row and the row offset inside a tile.
+struct Row {
+  int m, rb;
+};
+__device__ __forceinline__ Row row_of(const FlowArgs& a, int i) {
+  const int m = i / a.q;
+  return Row{m, (i - m * a.q) * kNB};
+}
+
+// Address of the first element of block column l of a block row (tile column
+// l / q, or column l - k q of tile column k).
+__device__ __forceinline__ char* block_ptr(const FlowArgs& a, Row r, int l, int esize) {
+  const int n = l / a.q;
+  const int lc = l - n * a.q;
+  const long ts = a.v.ts;
+  char* tile;
+  if (a.pool) tile = reinterpret_cast<char*>(a.pool) + tile_index(a.v, r.m, n) * ts * ts * 8;
+  else tile = static_cast<char*>(a.v.ptr[tile_index(a.v, r.m, n)]);
+  return tile + ((long)lc * kNB * ts + r.rb) * esize;
+}
+
+// Waits until the (relative) counters of four rows all exceed l and returns
+// the smallest; lane t of wave 0 polls row t % 4.
+__device__ __forceinline__ int wait_rows(const FlowArgs& a, const int (&rows)[4], int l, int* sh) {
+  if (threadIdx.x < 64) {
+    const int t = threadIdx.x;
+    const int u = t & 3;
+    const int* f = a.flags + kRows + 16 * ((u < 2 ? (u ? rows[1] : rows[0]) : (u == 2 ? rows[2] : rows[3])) - a.j0);
+    int got;
+    for (;;) {
+      got = flag_get(f);
+#pragma unroll
+      for (int off = 1; off < 4; off <<= 1) {
+        const int o = __shfl_xor(got, off, 64);
+        got = o < got ? o : got;
+      }
+      got = __builtin_amdgcn_readfirstlane(got);
+      if (got > l) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (t == 0) *sh = got;
+  }
+  __syncthreads();
+  const int got = *sh;
+  __syncthreads();
+  return got;
+}
+
+__device__ __forceinline__ void wait_diag(const FlowArgs& a, int need) {
+  if (threadIdx.x == 0) {
+    while (flag_get(a.flags + kDiag) < need) __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+}
+
+// Lower blocks of the 64 x 64 inverse at src into LDS (blk16 layout).
+__device__ __forceinline__ void load_inverse(const double* src, double* lds, int wave, int lane) {
+#pragma unroll
+  for (int t = 0; t < 5; ++t) {
+    const int c = wave + 4 * t;  // 20 half blocks
+    const int b = c >> 1;
+    const int bi = b < 1 ? 0 : (b < 3 ? 1 : (b < 6 ? 2 : 3));
+    const int bj = b - bi * (bi + 1) / 2;
+    const int kk = (c & 1) * 8 + (lane >> 3);
+    const int r = 2 * (lane & 7);
+    const double* s = src + 16 * bi + r + (16 * bj + kk) * 64;
+    __builtin_amdgcn_global_load_lds((glb_void_t*)(uintptr_t)s, (lds_void_t*)(lds + c * 128), 16, 0, 0);
+  }
+}
+
+// x = t inv^T for the wave's 16 rows: t and x are 16 x 64, four fragments of
+// lane l, element v at row l%16, column 16 f + l/16 + 4 v.  That is also the
+// layout in which the MFMA takes its left operand, so t feeds it as is.
+__device__ __forceinline__ void times_inverse(const dx4 (&t)[4], dx4 (&x)[4], const double* inv, int lane) {
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    x[f] = dx4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int g = 0; g <= f; ++g)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[f] = mfma_f64(inv[blk16(f, g) + e * 64 + lane], t[g][e], x[f]);
+  }
+}
+
+// A stage of the operand ring: NP panels of 64 rows x 16 columns.
+constexpr int kPanel = 1024;
+
+// acc[p][f] += A_p B^T over block columns [l, l_end): A_p the block rows
+// `ra` (R of them; FP32 tiles when TA is float), B the block row rb.
+// DIAG: instead, panel 0 is block row ra[0] = j-1 and panel B is j, and
+// acc[0][f] += B A^T, dacc += the wave's fragments of B B^T.
+template <int R, class TA, bool DIAG>
+__device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], dx4 (&dacc)[3], const Row (&ra)[R],
+                                          Row rb, int l, int l_end, double* lds) {
+  constexpr bool kF = sizeof(TA) == 4;
+  constexpr int A_PAN = kF ? kPanel / 2 : kPanel;  // doubles
+  constexpr int STAGE = R * A_PAN + kPanel;
+  constexpr int PER_WAVE = R * (kF ? 1 : 2) + 2;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ts = a.v.ts;
+  const int nk = (l_end - l) * 4;
+  if (nk <= 0) return;
+  const char* pa[R];
+  const char* pb = block_ptr(a, rb, l, 8);
+#pragma unroll
+  for (int p = 0; p < R; ++p) pa[p] = block_ptr(a, ra[p], l, (int)sizeof(TA));
+  int n = l / a.q;
+  int left = (a.q - (l - n * a.q)) * 4;  // slices left in the current tile column
+  // byte offsets of this lane's elements in a slice
+  uint32_t o8[2], o4;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int kk = 4 * wave + 2 * e + (lane >> 5);
+    o8[e] = (uint32_t)((((2 * (lane & 31)) ^ ((kk & 1) * 16)) + kk * ts) * 8);
+  }
+  {
+    const int kk = 4 * wave + (lane >> 4);
+    o4 = (uint32_t)((((4 * (lane & 15)) ^ ((kk & 3) * 16)) + kk * ts) * 4);
+  }
+  auto issue = [&](int buf) {
+    if (left == 0) {
+      ++n;
+      pb = block_ptr(a, rb, n * a.q, 8);
+#pragma unroll
+      for (int p = 0; p < R; ++p) pa[p] = block_ptr(a, ra[p], n * a.q, (int)sizeof(TA));
+      left = a.q * 4;
+    }
+    double* st = lds + buf * STAGE;
+#pragma unroll
+    for (int p = 0; p < R; ++p) {
+      if constexpr (kF) {
+        __builtin_amdgcn_global_load_lds((glb_void_t*)(uintptr_t)(pa[p] + o4),
+                                         (lds_void_t*)(st + p * A_PAN + wave * 128), 16, 0, 0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          __builtin_amdgcn_global_load_lds((glb_void_t*)(uintptr_t)(pa[p] + o8[e]),
+                                           (lds_void_t*)(st + p * A_PAN + (2 * wave + e) * 128), 16, 0, 0);
+      }
+      pa[p] += (long)16 * ts * sizeof(TA);
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(uintptr_t)(pb + o8[e]),
+                                       (lds_void_t*)(st + R * A_PAN + (2 * wave + e) * 128), 16, 0, 0);
+    pb += (long)16 * ts * 8;
+    --left;
+  };
+  const int k4 = lane >> 4, r16 = lane & 15;
+  const int flip = (k4 & 1) * 16;
+  int dbi[3], dbj[3];
+#pragma unroll
+  for (int t = 0; t < 3; ++t) diag_frag(wave, t < diag_count(wave) ? t : 0, dbi[t], dbj[t]);
+  double fa[2][R], fb[2][4], fx[2][3], fy[2][3];
+  auto frag = [&](int set, int buf, int kk) {
+    const double* st = lds + buf * STAGE;
+    const int k = 4 * kk + k4;
+    const double* Bp = st + R * A_PAN + k * 64 + r16;
+    if constexpr (DIAG) {
+      const double* Ap = st + k * 64 + r16;
+      fa[set][0] = Bp[(16 * wave) ^ flip];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) fb[set][f] = Ap[(16 * f) ^ flip];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        fx[set][t] = Bp[(16 * dbi[t]) ^ flip];
+        fy[set][t] = Bp[(16 * dbj[t]) ^ flip];
+      }
+    } else {
+#pragma unroll
+      for (int p = 0; p < R; ++p) {
+        if constexpr (kF) {
+          const float* Af = reinterpret_cast<const float*>(st + p * A_PAN);
+          fa[set][p] = (double)Af[k * 64 + ((16 * wave) ^ (k4 * 16)) + r16];
+        } else {
+          fa[set][p] = st[p * A_PAN + k * 64 + ((16 * wave) ^ flip) + r16];
+        }
+      }
+#pragma unroll
+      for (int f = 0; f < 4; ++f) fb[set][f] = Bp[(16 * f) ^ flip];
+    }
+  };
+  auto step = [&](int cur) {
+#pragma unroll
+    for (int p = 0; p < R; ++p)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) acc[p][f] = mfma_f64(fb[cur][f], fa[cur][p], acc[p][f]);
+    if constexpr (DIAG) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        if (t < 2 || wave == 1 || wave == 2) dacc[t] = mfma_f64(fy[cur][t], fx[cur][t], dacc[t]);
+    }
+  };
+  __builtin_amdgcn_s_barrier();
+  issue(0);
+  issue(1);  // nk >= 4
+  wait_vmcnt<PER_WAVE>();
+  __builtin_amdgcn_s_barrier();
+  frag(0, 0, 0);
+  int buf = 0;
+#pragma unroll 1
+  for (int kc = 0; kc < nk; ++kc) {
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const int cur = kk & 1, nxt = cur ^ 1;
+      if (kk < 3) {
+        frag(nxt, buf, kk + 1);
+      } else if (kc + 1 < nk) {
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt_lgkm0<0>();
+        __builtin_amdgcn_s_barrier();
+        if (kc + 2 < nk) issue(buf);
+        frag(nxt, buf ^ 1, 0);
+      }
+      step(cur);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    buf ^= 1;
+  }
+}
+
+typedef __attribute__((address_space(1))) double gdouble;
+typedef __attribute__((address_space(1))) float gfloat;
+
+// t = C - acc for the wave's 16 rows of a 64 x 64 block.
+template <class TA>
+__device__ __forceinline__ void block_minus(const char* blk, long ts, int wave, int lane, dx4 (&acc)[4]) {
+  typedef __attribute__((address_space(1))) const TA gT;
+  gT* G = (gT*)(uintptr_t)blk + 16 * wave + (lane & 15) + (long)(lane >> 4) * ts;
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[f][v] = (double)G[(long)(16 * f + 4 * v) * ts] - acc[f][v];
+}
+
+template <class TA>
+__device__ __forceinline__ void block_store(char* blk, long ts, int wave, int lane, const dx4 (&x)[4]) {
+  TA* G = reinterpret_cast<TA*>(blk) + 16 * wave + (lane & 15) + (long)(lane >> 4) * ts;
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) store_through(G + (long)(16 * f + 4 * v) * ts, (TA)x[f][v]);
+}
+
+// T task: block rows i0 .. i0 + nr - 1 (nr <= R), block column j.
+template <int R, class TA>
+__device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int j, double* lds, int* sh) {
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long ts = a.v.ts;
+  int rows[4] = {j, i0, i0 + nr - 1, i0 + (nr > 1 ? 1 : 0)};
+  Row ra[R];
+#pragma unroll
+  for (int p = 0; p < R; ++p) ra[p] = row_of(a, i0 + (p < nr ? p : 0));
+  const Row rj = row_of(a, j);
+  dx4 acc[R][4], none[3];
+#pragma unroll
+  for (int p = 0; p < R; ++p)
+#pragma unroll
+    for (int f = 0; f < 4; ++f) acc[p][f] = dx4{0.0, 0.0, 0.0, 0.0};
+  int l = a.j0;
+  while (l < j) {
+    int upto = a.j0 + wait_rows(a, rows, l - a.j0, sh);
+    if (upto > j) upto = j;
+    flow_gemm<R, TA, false>(a, acc, none, ra, rj, l, upto, lds);
+    l = upto;
+  }
+#pragma unroll
+  for (int p = 0; p < R; ++p) block_minus<TA>(block_ptr(a, ra[p], j, (int)sizeof(TA)), ts, wave, lane, acc[p]);
+  wait_diag(a, j - a.j0 + 1);  // its barrier also ends the reads of the ring
+  load_inverse(a.dinv + (long)j * 4096, lds, wave, lane);
+  wait_vmcnt<0>();
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < R; ++p) {
+    if (p < nr) {
+      dx4 x[4];
+      times_inverse(acc[p], x, lds, lane);
+      block_store<TA>(block_ptr(a, ra[p], j, (int)sizeof(TA)), ts, wave, lane, x);
+    }
+  }
+  stores_done();
+  __syncthreads();
+  if (tid < nr) flag_set(a.flags + kRows + 16 * (i0 + tid - a.j0), j - a.j0 + 1);
+}
+
+// D task of block column j.
+__device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds, int* sh) {
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long ts = a.v.ts;
+  const Row rj = row_of(a, j);
+  const int nd = diag_count(wave);
+  __builtin_amdgcn_s_setprio(2);
+  dx4 acc[1][4], dacc[3];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) acc[0][f] = dx4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int t = 0; t < 3; ++t) dacc[t] = dx4{0.0, 0.0, 0.0, 0.0};
+  char* cjj = block_ptr(a, rj, j, 8);
+  if (j > a.j0) {
+    const Row rp[1] = {row_of(a, j - 1)};
+    int rows[4] = {j, j - 1, j, j - 1};
+    int l = a.j0;
+    while (l < j - 1) {
+      int upto = a.j0 + wait_rows(a, rows, l - a.j0, sh);
+      if (upto > j - 1) upto = j - 1;
+      flow_gemm<1, double, true>(a, acc, dacc, rp, rj, l, upto, lds);
+      l = upto;
+    }
+    char* cp = block_ptr(a, rj, j - 1, 8);
+    block_minus<double>(cp, ts, wave, lane, acc[0]);
+    // the diagonal block, ahead of the wait
+    dx4 cd[3];
+    {
+      typedef __attribute__((address_space(1))) const double gD;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        int bi, bj;
+        diag_frag(wave, t < nd ? t : 0, bi, bj);
+        gD* G = (gD*)(uintptr_t)cjj + 16 * bi + (lane & 15) + (long)(16 * bj + (lane >> 4)) * ts;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) cd[t][v] = G[(long)(4 * v) * ts];
+      }
+    }
+    wait_diag(a, j - a.j0);
+    load_inverse(a.dinv + (long)(j - 1) * 4096, lds, wave, lane);
+    wait_vmcnt<0>();
+    __syncthreads();
+    dx4 x[4];
+    times_inverse(acc[0], x, lds, lane);
+    block_store<double>(cp, ts, wave, lane, x);
+    __syncthreads();
+    // X as sixteen 16 x 16 blocks (row block w, column block f), for X X^T
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) lds[(wave * 4 + f) * 256 + v * 64 + lane] = x[f][v];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      if (t < nd) {
+        int bi, bj;
+        diag_frag(wave, t, bi, bj);
+        const double* X = lds + bi * 1024 + lane;
+        const double* Y = lds + bj * 1024 + lane;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dacc[t] = mfma_f64(Y[e * 64], X[e * 64], dacc[t]);
+      }
+    }
+    stores_done();
+    __syncthreads();
+    if (tid == 0) flag_set(a.flags + kRows + 16 * (j - a.j0), j - a.j0);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      if (t < nd) {
+        int bi, bj;
+        diag_frag(wave, t, bi, bj);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) lds[blk16(bi, bj) + v * 64 + lane] = cd[t][v] - dacc[t][v];
+      }
+    }
+  } else {
+    typedef __attribute__((address_space(1))) const double gD;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      if (t < nd) {
+        int bi, bj;
+        diag_frag(wave, t, bi, bj);
+        gD* G = (gD*)(uintptr_t)cjj + 16 * bi + (lane & 15) + (long)(16 * bj + (lane >> 4)) * ts;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) lds[blk16(bi, bj) + v * 64 + lane] = G[(long)(4 * v) * ts];
+      }
+    }
+  }
+  __syncthreads();
+  double* Ls = lds;
+  double* Xs = lds + 2560;
+  for (int p = 0; p < 4; ++p) {
+    if (wave == 0) {
+      // rows 16 p + lane
+      double c[16];
+      const int bi = p + (lane >> 4);
+      const double* src = Ls + blk16(bi < 4 ? bi : p, p) + (lane & 15);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) c[e] = src[e * 16];
+      const unsigned bad = panel16(c, lane);
+      if (bad && lane == 0) atomicCAS(a.info, 0, j * kNB + 16 * p + __builtin_ctz(bad) + 1);
+      if (bi < 4) {
+        double* dst = Ls + blk16(bi, p) + (lane & 15);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dst[e * 16] = (bi > p || lane >= e) ? c[e] : 0.0;
+      }
+    } else if (wave == 1) {
+      // the diagonal block again in lanes 0 .. 15, an identity in 16 .. 31:
+      // its rows come out as rows of the inverse transposed
+      double c[16];
+      const double* src = Ls + blk16(p, p) + (lane & 15);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) c[e] = lane < 16 ? src[e * 16] : (lane == 16 + e ? 1.0 : 0.0);
+      panel16(c, lane);
+      if (lane >= 16 && lane < 32) {
+        double* dst = Xs + blk16(p, p) + (lane - 16) * 16;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dst[e] = c[e];
+      }
+    }
+    __syncthreads();
+    // Trailing fragments (bi, bj), p < bj <= bi, and the inverse's row p:
+    // X_p,b = -X_pp sum_{b <= l < p} L_pl X_lb.
+    const int nt = (3 - p) * (4 - p) / 2;
+    for (int t = wave; t < nt + p; t += 4) {
+      if (t < nt) {
+        const int r = t < 1 ? 0 : (t < 3 ? 1 : 2);
+        const int bi = p + 1 + r, bj = p + 1 + t - r * (r + 1) / 2;
+        double* S = Ls + blk16(bi, bj) + lane;
+        const double* A = Ls + blk16(bi, p) + lane;
+        const double* B = Ls + blk16(bj, p) + lane;
+        dx4 s = {S[0], S[64], S[128], S[192]};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = mfma_f64(-B[e * 64], A[e * 64], s);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[e * 64] = s[e];
+      } else {
+        const int b = t - nt;
+        dx4 y = {0.0, 0.0, 0.0, 0.0};
+        for (int l = b; l < p; ++l) {
+          const double* A = Ls + blk16(p, l) + lane;
+          const double* B = Xs + blk16(l, b) + (lane & 15) * 16 + (lane >> 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y = mfma_f64(A[e * 64], B[e * 4], y);
+        }
+        // y: lane l, element v at row l/16 + 4 v, column l%16
+        const double* D = Xs + blk16(p, p) + lane;
+        dx4 x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x = mfma_f64(-y[e], D[e * 64], x);
+        double* dst = Xs + blk16(p, b) + lane;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[e * 64] = x[e];
+      }
+    }
+    __syncthreads();
+  }
+  // the inverse, then the counter that every T task of this column waits for
+  double* dinv = a.dinv + (long)j * 4096;
+  const int r = tid & 15, c = tid >> 4;
+#pragma unroll
+  for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+    for (int bj = 0; bj <= bi; ++bj)
+      store_through(dinv + 16 * bi + r + (16 * bj + c) * 64, Xs[blk16(bi, bj) + tid]);
+  stores_done();
+  __syncthreads();
+  if (tid == 0) flag_set(a.flags + kDiag, j - a.j0 + 1);
+  __builtin_amdgcn_s_setprio(0);
+  // off the chain: the factor block itself, the zeros above it
+  gdouble* out = (gdouble*)(uintptr_t)cjj;
+#pragma unroll
+  for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < 4; ++bj) {
+      out[16 * bi + r + (long)(16 * bj + c) * ts] = bj <= bi ? Ls[blk16(bi, bj <= bi ? bj : 0) + tid] : 0.0;
+      if (bj > bi) dinv[16 * bi + r + (16 * bj + c) * 64] = 0.0;
+    }
+  gdouble* top = out - rj.rb;
+  for (int e = tid; e < rj.rb * kNB; e += 256) {
+    const int cc = e / rj.rb;
+    top[e - cc * rj.rb + (long)cc * ts] = 0.0;
+  }
+  __syncthreads();
+}
+
+// The T tasks of one block column: groups of up to R consecutive block rows
+// of [lo, i_end).  With ALIGNED the groups end at tile boundaries (the tiles
+// of a mixed-precision factor differ in their element type).
+template <int R, bool ALIGNED>
+__host__ __device__ __forceinline__ int row_groups(int lo, int i_end, int q) {
+  if (i_end <= lo) return 0;
+  if (!ALIGNED) return (i_end - lo + R - 1) / R;
+  const int first = (lo / q + 1) * q;
+  if (i_end <= first) return (i_end - lo + R - 1) / R;
+  const int rest = i_end - first;
+  return (first - lo + R - 1) / R + rest / q * ((q + R - 1) / R) + (rest % q + R - 1) / R;
+}
+template <int R, bool ALIGNED>
+__device__ __forceinline__ void row_group(int t, int lo, int i_end, int q, int& i0, int& nr) {
+  int end = i_end;
+  i0 = lo + t * R;
+  if (ALIGNED) {
+    const int first = (lo / q + 1) * q;
+    const int g0 = (first - lo + R - 1) / R;
+    if (t < g0) {
+      end = first < i_end ? first : i_end;
+    } else {
+      const int gt = (q + R - 1) / R;
+      const int tile = (t - g0) / gt;
+      i0 = first + tile * q + (t - g0 - tile * gt) * R;
+      end = first + (tile + 1) * q < i_end ? first + (tile + 1) * q : i_end;
+    }
+  }
+  nr = end - i0 < R ? end - i0 : R;
+}
+// First block row of column j's T tasks: row j + 1 belongs to D_{j+1} unless
+// j is the last column.
+__host__ __device__ __forceinline__ int rows_from(int j, int j1) { return j + 1 < j1 ? j + 2 : j + 1; }
+
+template <int R, bool MIXED>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_chol_flow(FlowArgs a) {
+  __shared__ __attribute__((aligned(16))) double lds[R == 1 ? 5120 : 2048 * (R + 1)];
+  __shared__ int sh[2];
+  const int tid = threadIdx.x;
+  int j = a.j0;
+  long base = 0;  // first task of column j
+  for (;;) {
+    if (tid == 0) sh[0] = atomicAdd(a.flags + kClaim, 1);
+    __syncthreads();
+    const long id = sh[0];
+    __syncthreads();
+    for (; j < a.j1; ++j) {
+      const int cnt = 1 + row_groups<R, MIXED>(rows_from(j, a.j1), a.i_end, a.q);
+      if (id < base + cnt) break;
+      base += cnt;
+    }
+    if (j >= a.j1) break;
+    const int t = (int)(id - base);
+    if (t == 0) {
+      task_diag(a, j, lds, sh + 1);
+      if (j + 1 == a.j1) {
+        for (long e = tid; e < (long)(a.j_pad - a.j1) * 4096; e += 256)
+          a.dinv[(long)a.j1 * 4096 + e] = ((e & 4095) % 65 == 0) ? 1.0 : 0.0;
+      }
+    } else {
+      int i0, nr;
+      row_group<R, MIXED>(t - 1, rows_from(j, a.j1), a.i_end, a.q, i0, nr);
+      if constexpr (MIXED) {
+        if (a.v.prec[tile_index(a.v, i0 / a.q, a.k)] != kF64) task_rows<R, float>(a, i0, nr, j, lds, sh + 1);
+        else task_rows<R, double>(a, i0, nr, j, lds, sh + 1);
+      } else {
+        task_rows<R, double>(a, i0, nr, j, lds, sh + 1);
+      }
+    }
+  }
+  // The last work-group leaves the counters as it found them.
+  if (tid == 0) sh[0] = atomicAdd(a.flags + kExit, 1) == (int)gridDim.x - 1;
+  __syncthreads();
+  if (!sh[0]) return;
+  for (int e = tid; e < a.i_end - a.j0; e += 256) a.flags[kRows + 16 * e] = 0;
+  if (tid == 0) a.flags[kClaim] = a.flags[kExit] = a.flags[kDiag] = 0;
+}
+
+template <int R, bool MIXED>
+void launch_flow(const FlowArgs& a, hipStream_t s) {
+  static int slots = 0;
+  if (!slots) {
+    int dev = 0, cus = 0, occ = 1;
+    EXA_HIP(hipGetDevice(&dev));
+    EXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_chol_flow<R, MIXED>, 256, 0));
+    slots = cus * (occ > 0 ? occ : 1);
+  }
+  long tasks = 0;
+  for (int j = a.j0; j < a.j1 && tasks < slots; ++j)
+    tasks += 1 + row_groups<R, MIXED>(rows_from(j, a.j1), a.i_end, a.q);
+  long grid = tasks < slots ? tasks : slots;
+  hipLaunchKernelGGL((k_chol_flow<R, MIXED>), dim3((unsigned)grid), dim3(256), 0, s, a);
+  EXA_HIP(hipGetLastError());
+}
+
+}  // namespace
+
+long chol_flow_flags(int mt, int ts) { return kRows + 16L * mt * (ts / kNB); }
+
+void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int j1, int i_end, int j_pad,
+                      double* dinv, int* info, int* flags, hipStream_t s) {
+  FlowArgs a;
+  a.v = v;
+  a.pool = pool;
+  a.k = tile_col;
+  a.q = v.ts / kNB;
+  a.j0 = j0;
+  a.j1 = j1;
+  a.i_end = i_end;
+  a.j_pad = j_pad;
+  a.dinv = dinv;
+  a.info = info;
+  a.flags = flags;
+  const int nb = v.mt * a.q;
+  if (!v.lower || j0 < 0 || j1 <= j0 || j1 > nb || i_end < j1 || i_end > nb || j_pad > nb)
+    throw std::invalid_argument("chol_flow: block range outside the matrix");
+  if (!pool && (tile_col < 0 || j0 < tile_col * a.q || j1 > (tile_col + 1) * a.q))
+    throw std::invalid_argument("chol_flow: block columns outside the tile column");
+  if (pool) launch_flow<2, false>(a, s);
+  else if (v.prec) launch_flow<3, true>(a, s);
+  else launch_flow<3, false>(a, s);
+}
+
+}  // namespace exa

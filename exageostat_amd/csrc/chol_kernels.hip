@@ -1,5 +1,5 @@
-// FP64 tile Cholesky kernels: diagonal-tile factorisation, panel triangular
-// solve and trailing update, all on FP64 MFMA.
+// FP64 tile Cholesky kernels: trailing update and the inverses of the
+// diagonal tiles, on FP64 MFMA (the panels: chol_flow.hip).
 //
 // Replaces Chameleon's CHAMELEON_dpotrf_Tile(ChamLower, C) as called from
 // EXAGEOSTAT_dmle_Tile (exageostat_exact/src/compute/MLE_dexact.c:372);
@@ -14,185 +14,6 @@
 namespace exa {
 
 using C64 = GemmCfg<64, 64, 2, 2, 16>;
-
-// ---------------------------------------------------------------------------
-// Unblocked Cholesky of the 64x64 diagonal block j of a diagonal tile, plus
-// the explicit inverse of the resulting lower-triangular block, by one wave
-// (no multi-wave barriers on the critical path of the panel).  Lane r owns
-// row r.  Column c is finished left-looking,
-//   L(r,c) = (A(r,c) - sum_{k<c} L(r,k) L(c,k)) / L(c,c),
-// and lane r then forms column r of X = L^-1 by forward substitution,
-//   X(i,r) = (delta_ir - sum_{k<i} L(i,k) X(k,r)) / L(i,i);
-// each sum is taken as four interleaved partial sums (shorter dependent
-// chains).
-// Both matrices live in LDS column-major (element (i,k) at k*LD + i), so a
-// lane's own entries of one column are contiguous across the wave and
-// L(c,k) / L(i,k) are broadcast reads.
-__global__ void __launch_bounds__(64) k_potrf_block(double* T, int ts, int j, double* dinv, int* info,
-                                                    long col_base) {
-  constexpr int LD = 65;
-  __shared__ double Ls[64 * LD];  // L(i, k) at Ls[k * LD + i]
-  __shared__ double Xs[64 * LD];  // X(i, k) at Xs[k * LD + i] (written transposed, see below)
-  const int r = threadIdx.x;
-  double* blk = T + (long)j * kNB * (ts + 1);
-  {
-    // all 64 column loads in flight before the first LDS store
-    double col[64];
-#pragma unroll
-    for (int k = 0; k < 64; ++k) col[k] = blk[r + (long)k * ts];
-#pragma unroll
-    for (int k = 0; k < 64; ++k) Ls[k * LD + r] = col[k];
-  }
-  __syncthreads();
-  for (int c = 0; c < 64; ++c) {
-    // four partial sums over k mod 4 break the dependent FMA chain
-    double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-    int k = 0;
-#pragma unroll 4
-    for (; k + 4 <= c; k += 4) {
-      p0 += Ls[k * LD + r] * Ls[k * LD + c];
-      p1 += Ls[(k + 1) * LD + r] * Ls[(k + 1) * LD + c];
-      p2 += Ls[(k + 2) * LD + r] * Ls[(k + 2) * LD + c];
-      p3 += Ls[(k + 3) * LD + r] * Ls[(k + 3) * LD + c];
-    }
-    for (; k < c; ++k) p0 += Ls[k * LD + r] * Ls[k * LD + c];
-    const double s = Ls[c * LD + r] - ((p0 + p1) + (p2 + p3));
-    if (r == c) {
-      const bool bad = !(s > 0.0);
-      if (bad) atomicCAS(info, 0, (int)(col_base + c + 1));
-      Ls[c * LD + c] = bad ? __builtin_nan("") : sqrt(s);
-    }
-    __syncthreads();
-    if (r > c) Ls[c * LD + r] = s / Ls[c * LD + c];
-    __syncthreads();
-  }
-  for (int k = 0; k < 64; ++k) blk[r + (long)k * ts] = (r >= k) ? Ls[k * LD + r] : 0.0;
-  // Lane r keeps X(i, r) at Xs[i * LD + r] (its own column, contiguous across
-  // lanes for each i).
-  for (int i = 0; i < 64; ++i) {
-    double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-    int k = 0;
-#pragma unroll 4
-    for (; k + 4 <= i; k += 4) {
-      p0 += Ls[k * LD + i] * Xs[k * LD + r];
-      p1 += Ls[(k + 1) * LD + i] * Xs[(k + 1) * LD + r];
-      p2 += Ls[(k + 2) * LD + i] * Xs[(k + 2) * LD + r];
-      p3 += Ls[(k + 3) * LD + i] * Xs[(k + 3) * LD + r];
-    }
-    for (; k < i; ++k) p0 += Ls[k * LD + i] * Xs[k * LD + r];
-    Xs[i * LD + r] = (((i == r) ? 1.0 : 0.0) - ((p0 + p1) + (p2 + p3))) / Ls[i * LD + i];
-  }
-  __syncthreads();
-  // dinv column-major: dinv[i + c*64] = X(i, c) = Xs[i * LD + c].
-  for (int c = 0; c < 64; ++c) dinv[r + c * 64] = Xs[r * LD + c];
-}
-
-// ---------------------------------------------------------------------------
-// X L^T = B for one 64-row slab X (in place of B), L lower with nL diagonal
-// 64-blocks whose inverses are in dinv.  Column sweep: for block jb,
-// X_jb = (B_jb - X_<jb L_jb,<jb^T) inv(L_jb,jb)^T.
-template <class TX>
-__device__ void trsm_slab(TX* X, long ldx, const double* L, long ldl, int nL, const double* dinv,
-                          double* lds) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave / C64::WGN;
-  const int wn = wave - wm * C64::WGN;
-  constexpr int LDT = 68;
-  for (int jb = 0; jb < nL; ++jb) {
-    dx4 acc[C64::FM][C64::FN];
-    TX* Xj = X + (long)jb * kNB * ldx;
-    acc_load<C64, TX>(acc, Xj, ldx);
-    gemm_nt_acc<C64, false, TX, double>(acc, X, ldx, L + jb * kNB, ldl, jb * kNB, lds, -1.0);
-    double* Ts = lds;
-    double* Is = lds + 64 * LDT;
-#pragma unroll
-    for (int i = 0; i < C64::FM; ++i)
-#pragma unroll
-      for (int jj = 0; jj < C64::FN; ++jj) {
-        const int c = wn * C64::WN + jj * 16 + frag_col(lane);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = wm * C64::WM + i * 16 + frag_row(lane, v);
-          Ts[c * LDT + r] = acc[i][jj][v];
-        }
-      }
-    const double* inv = dinv + (long)jb * 4096;
-    for (int e = tid; e < 64 * 32; e += 256) {
-      const int kk = e >> 5;
-      const int c2 = e & 31;
-      *reinterpret_cast<double2*>(Is + kk * LDT + 2 * c2) =
-          *reinterpret_cast<const double2*>(inv + 2 * c2 + kk * 64);
-    }
-    __syncthreads();
-    dx4 x[C64::FM][C64::FN];
-    zero_acc<C64>(x);
-#pragma unroll 4
-    for (int kk = 0; kk < 64; kk += 4) {
-      const int krow = kk + (lane >> 4);
-      double a[C64::FM], b[C64::FN];
-#pragma unroll
-      for (int i = 0; i < C64::FM; ++i) a[i] = Ts[krow * LDT + wm * C64::WM + i * 16 + (lane & 15)];
-#pragma unroll
-      for (int jj = 0; jj < C64::FN; ++jj) b[jj] = Is[krow * LDT + wn * C64::WN + jj * 16 + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < C64::FM; ++i)
-#pragma unroll
-        for (int jj = 0; jj < C64::FN; ++jj) x[i][jj] = mfma_f64(a[i], b[jj], x[i][jj]);
-    }
-    acc_update<C64, TX>(x, Xj, ldx, 0.0);
-    // X_jb is read back from global memory by the next column block of this
-    // same work-group: the barrier's workgroup-scope release/acquire makes
-    // the stores visible inside the CU (no device-scope fence, which would
-    // write back the XCD's L2).
-    __syncthreads();
-  }
-}
-
-// Panel: slabs over tiles m in (k, mt) and their 64-row blocks.
-__global__ void __launch_bounds__(256) k_trsm_panel(TileView v, int k, const double* dinv) {
-  __shared__ __attribute__((aligned(16))) double lds[2 * 64 * 68];
-  const int q = v.ts / kNB;
-  const int s = blockIdx.x;
-  const int m = k + 1 + s / q;
-  const int rb = s - (s / q) * q;
-  const double* L = tile_f64(v, k, k);
-  const long t = tile_index(v, m, k);
-  // Mixed-precision factors store off-diagonal tiles in FP32; the solve
-  // itself runs in FP64 either way.
-  if (v.prec && v.prec[t] != kF64) {
-    float* X = static_cast<float*>(v.ptr[t]) + rb * kNB;
-    trsm_slab<float>(X, v.ts, L, v.ts, q, dinv, lds);
-  } else {
-    double* X = static_cast<double*>(v.ptr[t]) + rb * kNB;
-    trsm_slab<double>(X, v.ts, L, v.ts, q, dinv, lds);
-  }
-}
-
-// Inside a diagonal tile after block j is factored: blocks (i, j), i > j.
-__global__ void __launch_bounds__(256) k_trsm_intra(double* T, int ts, int j, const double* dinv_j) {
-  __shared__ __attribute__((aligned(16))) double lds[2 * 64 * 68];
-  const int i = j + 1 + blockIdx.x;
-  double* X = T + (long)i * kNB + (long)j * kNB * ts;
-  trsm_slab<double>(X, ts, nullptr, ts, 1, dinv_j, lds);
-}
-
-// Inside a diagonal tile: blocks (i, l), j < l <= i: B_il -= B_ij B_lj^T.
-__global__ void __launch_bounds__(256) k_syrk_intra(double* T, int ts, int j) {
-  __shared__ __attribute__((aligned(16))) double lds[C64::LDS_DOUBLES];
-  int r, c;
-  tri_decode(blockIdx.x, r, c);
-  const int i = j + 1 + r;
-  const int l = j + 1 + c;
-  const double* A = T + (long)i * kNB + (long)j * kNB * ts;
-  const double* B = T + (long)l * kNB + (long)j * kNB * ts;
-  double* Cp = T + (long)i * kNB + (long)l * kNB * ts;
-  dx4 acc[C64::FM][C64::FN];
-  zero_acc<C64>(acc);
-  gemm_nt_acc<C64>(acc, A, ts, B, ts, kNB, lds, -1.0);
-  acc_update<C64>(acc, Cp, ts, 1.0);
-}
 
 // ---------------------------------------------------------------------------
 // Explicit inverse X = L_kk^-1 of every diagonal tile (for the triangular
@@ -388,30 +209,6 @@ void launch_tile_update(const TileView& v, int k, int np, int col_lo, int col_hi
   } else {
     launch_update_cfg<C64>(v, k, np, col_lo, col_hi, s);
   }
-}
-
-// ---------------------------------------------------------------------------
-void launch_potrf_tile(double* T, int ts, double* dinv_k, int* info, long col_base, hipStream_t s) {
-  const int q = ts / kNB;
-  for (int j = 0; j < q; ++j) {
-    hipLaunchKernelGGL(k_potrf_block, dim3(1), dim3(64), 0, s, T, ts, j, dinv_k + (long)j * 4096, info,
-                       col_base + (long)j * kNB);
-    if (j + 1 < q) {
-      const int nb = q - j - 1;
-      hipLaunchKernelGGL(k_trsm_intra, dim3(nb), dim3(256), 0, s, T, ts, j, dinv_k + (long)j * 4096);
-      hipLaunchKernelGGL(k_syrk_intra, dim3(nb * (nb + 1) / 2), dim3(256), 0, s, T, ts, j);
-    }
-  }
-  EXA_HIP(hipGetLastError());
-}
-
-void launch_trsm_panel(const TileView& v, int k, const double* dinv_k, hipStream_t s, int m_end) {
-  const int q = v.ts / kNB;
-  if (m_end < 0 || m_end > v.mt) m_end = v.mt;
-  const long slabs = (long)(m_end - k - 1) * q;
-  if (slabs <= 0) return;
-  hipLaunchKernelGGL(k_trsm_panel, dim3((unsigned)slabs), dim3(256), 0, s, v, k, dinv_k);
-  EXA_HIP(hipGetLastError());
 }
 
 }  // namespace exa

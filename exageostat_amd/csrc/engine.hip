@@ -145,6 +145,12 @@ uint8_t TileMatrix::prec(int mm, int nn) const {
   return h_prec_[tile_index(v, mm, nn)];
 }
 
+double* TileMatrix::pool_f64() const {
+  for (size_t t = 0; t < h_ptr_.size(); ++t)
+    if (h_prec_[t] != kF64 || h_slot_[t] != 8) return nullptr;
+  return static_cast<double*>(pool_);
+}
+
 void TileMatrix::to_host(double* A, long ld, hipStream_t s) const {
   std::vector<double> buf((size_t)ts * ts);
   std::vector<float> fbuf((size_t)ts * ts);
@@ -353,6 +359,7 @@ CholWorkspace::~CholWorkspace() {
   if (yvec_) (void)hipFree(yvec_);
   if (tpart_) (void)hipFree(tpart_);
   if (ticket_) (void)hipFree(ticket_);
+  if (flags_) (void)hipFree(flags_);
   if (info_) (void)hipFree(info_);
   if (h_info_) (void)hipHostFree(h_info_);
   for (auto e : ev_) (void)hipEventDestroy(e);
@@ -364,20 +371,24 @@ void CholWorkspace::ensure(int mt, int ts) {
   if (xinv_) (void)hipFree(xinv_);
   if (yvec_) (void)hipFree(yvec_);
   if (tpart_) (void)hipFree(tpart_);
+  if (flags_) (void)hipFree(flags_);
   dinv_ = xinv_ = yvec_ = tpart_ = nullptr;
+  flags_ = nullptr;
   mt_ = mt;
   ts_ = ts;
   EXA_HIP(hipMalloc(&dinv_, sizeof(double) * (size_t)mt * (ts / kNB) * 4096));
   EXA_HIP(hipMalloc(&xinv_, sizeof(double) * (size_t)mt * ts * ts));
   EXA_HIP(hipMalloc(&yvec_, sizeof(double) * (size_t)mt * ts));
   EXA_HIP(hipMalloc(&tpart_, sizeof(double) * (size_t)(ts / kNB) * ts));
+  EXA_HIP(hipMalloc(&flags_, sizeof(int) * chol_flow_flags(mt, ts)));
+  EXA_HIP(hipMemset(flags_, 0, sizeof(int) * chol_flow_flags(mt, ts)));
   if (!ticket_) {
     EXA_HIP(hipMalloc(&ticket_, sizeof(unsigned)));
-    // synchronous on the null stream, which does not order with the
-    // non-blocking streams the kernels run on: wait for it here
     EXA_HIP(hipMemset(ticket_, 0, sizeof(unsigned)));
-    EXA_HIP(hipDeviceSynchronize());
   }
+  // hipMemset runs on the null stream, which does not order with the
+  // non-blocking streams the kernels run on: wait for it here
+  EXA_HIP(hipDeviceSynchronize());
   if (!info_) EXA_HIP(hipMalloc(&info_, sizeof(int)));
   if (!h_info_) EXA_HIP(hipHostMalloc(&h_info_, sizeof(int), hipHostMallocDefault));
 }
@@ -458,6 +469,8 @@ void ClassLists::build(const TileMatrix& A, int band) {
   built_band = band;
 }
 
+static constexpr int kFlowBlocks = 200;
+
 int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2, bool sync,
                const ClassLists* lists, int band) {
   const int mt = A.mt;
@@ -473,14 +486,24 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
   EXA_HIP(hipMemsetAsync(d_info, 0, sizeof(int), s1));
   TileView v = A.view();
   auto rows = [&](int t) { return (double)std::min<long>(ts, (long)A.m - (long)t * ts); };
+  const int q = ts / kNB;
+  const int nb = (A.m + kNB - 1) / kNB;  // block rows that hold logical rows; the others stay the identity
+  // Tile columns >= k0 in one dataflow launch.
+  auto factor_rest = [&](int k0) {
+    const double n0 = (double)A.m - (double)k0 * ts;
+    profiled("potrf_diag", potrf_flops(n0), 0.0, s1, [&] {
+      launch_chol_flow(v, A.pool_f64(), 0, k0 * q, nb, nb, mt * q, ws.dinv_base(), d_info, ws.flags(), s1);
+    });
+  };
   auto factor_panel = [&](int k) {
     const double rk = rows(k);
-    profiled("potrf_diag", potrf_flops(rk), 0.0, s1,
-             [&] { launch_potrf_tile(A.tile(k, k), ts, ws.dinv(k), d_info, (long)k * ts, s1); });
     const double below = std::min((double)A.m, (double)row_end(k) * ts) - (double)(k + 1) * ts;
-    if (k + 1 < row_end(k))
-      profiled("trsm_panel", below * rk * rk, 0.0, s1,
-               [&] { launch_trsm_panel(v, k, ws.dinv(k), s1, row_end(k)); });
+    profiled("potrf_diag", potrf_flops(rk) + std::max(0.0, below) * rk * rk, 0.0, s1, [&] {
+      TileView pv = v;
+      if (!lists) pv.prec = nullptr;
+      launch_chol_flow(pv, nullptr, k, k * q, std::min((k + 1) * q, nb), std::min(row_end(k) * q, nb),
+                       k + 1 == mt ? mt * q : (k + 1) * q, ws.dinv_base(), d_info, ws.flags(), s1);
+    });
     // The BF16 update classes read the panel in split BF16 form.  The buffer
     // of step k is reused at step k + 2, whose panel (on s1) waits for the
     // column update of step k + 1, queued on s2 after the rest of step k.
@@ -525,14 +548,28 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
     EXA_HIP(hipEventRecord(e, st));
     return e;
   };
-  // s1 carries the panel factorisations (small kernels on the CUs the
-  // persistent update leaves free); s2 carries the trailing updates: first
+  // s1 carries the panel factorisations (one launch per tile column, on the
+  // CUs the persistent update leaves free); s2 carries the trailing updates: first
   // the column that unblocks the next panel, then the rest, which overlaps
   // with that panel on s1.
-  EXA_HIP(hipStreamWaitEvent(s2, record(s1), 0));
-  factor_panel(0);
-  hipEvent_t ev_panel = record(s1);
-  if (lists) {
+  // The FP64 factor's last kFlowBlocks block columns go into one dataflow
+  // launch: its left-looking tasks reach 46-54 TFLOP/s against 60-70 of the
+  // trailing update, but its chain costs 20 us per 64 columns where the tile
+  // steps wait for a panel and two partial update rounds (n = 12,000: 11.8
+  // against 16.1 ms; the whole of n = 20,000: 50 ms, with 100 blocks left to
+  // it 50.6, 200: 48.7, 320: 51.3; n = 40,000: 352, 350 and 354 ms).
+  const bool flow = !lists && A.pool_f64();
+  auto few = [&](int k) { return flow && nb - k * q <= kFlowBlocks; };
+  const bool whole = few(0);
+  hipEvent_t ev_panel = nullptr;
+  if (!whole) {
+    EXA_HIP(hipStreamWaitEvent(s2, record(s1), 0));
+    factor_panel(0);
+    ev_panel = record(s1);
+  }
+  if (whole) {
+    factor_rest(0);
+  } else if (lists) {
     for (int k = 0; k + 1 < mt; ++k) {
       EXA_HIP(hipStreamWaitEvent(s2, ev_panel, 0));
       if (k + 1 <= col_end(k)) update(k, k + 1, k + 1, s2);
@@ -581,6 +618,14 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
     int k = 0;
     while (k + 1 < mt) {
       EXA_HIP(hipStreamWaitEvent(s2, ev_panel, 0));
+      if (few(k + 1)) {
+        // every update of the remaining columns, then the rest at once
+        run_pending();
+        update(k, k + 1, mt - 1, s2);
+        EXA_HIP(hipStreamWaitEvent(s1, record(s2), 0));
+        factor_rest(k + 1);
+        break;
+      }
       update(k, k + 1, k + 1, s2);
       EXA_HIP(hipStreamWaitEvent(s1, record(s2), 0));
       factor_panel(k + 1);
@@ -606,9 +651,10 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
     run_pending();
   }
   // Join: s1 waits for the last updates on s2, s2 for the last panel on s1.
-  EXA_HIP(hipStreamWaitEvent(s1, record(s2), 0));
-  EXA_HIP(hipStreamWaitEvent(s2, record(s1), 0));
-  launch_zero_upper_diag(v, s1);
+  if (!whole) {
+    EXA_HIP(hipStreamWaitEvent(s1, record(s2), 0));
+    EXA_HIP(hipStreamWaitEvent(s2, record(s1), 0));
+  }
   profiled("trtri_diag", (double)mt * ts * (double)ts * ts / 3.0, 0.0, s1,
            [&] { launch_trtri_tiles(v, ws.dinv_base(), ws.xinv_base(), s1); });
   EXA_HIP(hipMemcpyAsync(ws.host_info(), d_info, sizeof(int), hipMemcpyDeviceToHost, s1));

@@ -56,6 +56,8 @@ class TileMatrix {
   void* tile_raw(int m, int n) const;
   uint8_t prec(int m, int n) const;
   size_t bytes() const { return bytes_; }
+  // Base of the tiles when all of them are FP64 and contiguous, else null.
+  double* pool_f64() const;
   // Host <-> device copies of the logical m x n matrix (column-major, ld).
   void to_host(double* A, long ld, hipStream_t s) const;
   void from_host(const double* A, long ld, hipStream_t s);
@@ -130,6 +132,8 @@ class CholWorkspace {
   double* tpart() const { return tpart_; }
   unsigned* ticket() const { return ticket_; }
   int* info() const { return info_; }      // device
+  // Zeroed progress counters of the dataflow factorisation.
+  int* flags() const { return flags_; }
   int* host_info() const { return h_info_; }  // pinned host mirror
   hipEvent_t ev(int i);
   int mt_ = 0, ts_ = 0;
@@ -143,6 +147,7 @@ class CholWorkspace {
   double* tpart_ = nullptr;
   unsigned* ticket_ = nullptr;
   int* info_ = nullptr;
+  int* flags_ = nullptr;
   int* h_info_ = nullptr;
   std::vector<hipEvent_t> ev_;
 };

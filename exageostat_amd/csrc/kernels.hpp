@@ -66,13 +66,17 @@ void launch_gen_bivariate(const TileView& v, const BivariateParams& P, long p_of
 void launch_gen_spacetime(const TileView& v, const SpaceTimeParams& P, long p_off, long ntiles, hipStream_t s);
 
 // ---- tile Cholesky building blocks (FP64) -------------------------------
-// Factor the diagonal tile (k,k) of a lower-packed matrix in place with
-// 64-wide sub-blocks; writes the inverses of the 64x64 diagonal blocks of
-// L_kk to dinv_k (q blocks of 64x64, column-major) and the first failing
-// global column + 1 to *info (left untouched on success).
-void launch_potrf_tile(double* T, int ts, double* dinv_k, int* info, long col_base, hipStream_t s);
-// A(m,k) <- A(m,k) L_kk^-T for all m in (k, m_end) (m_end < 0: mt).
-void launch_trsm_panel(const TileView& v, int k, const double* dinv_k, hipStream_t s, int m_end = -1);
+// Dataflow Cholesky (chol_flow.hip) of the 64-column blocks [j0, j1) of a
+// lower matrix, block rows [.., i_end), in one launch; updates from columns
+// < j0 are already applied.  pool: the tiles' common base when all of them
+// are FP64 and contiguous (the range may then span tile columns), else null
+// and the columns lie in tile column tile_col.  dinv: 64 x 64 inverses of
+// the diagonal blocks (block j at dinv + 4096 j; identities for the padding
+// blocks [j1, j_pad)).  flags: chol_flow_flags() ints, zero before the first
+// launch and left zero by each.
+long chol_flow_flags(int mt, int ts);
+void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int j1, int i_end, int j_pad,
+                      double* dinv, int* info, int* flags, hipStream_t s);
 // A(m,n) -= sum_{p < np} A(m,k+p) A(n,k+p)^T for n in [col_lo, col_hi],
 // m in [n, mt); np = 1 or 2 (col_lo >= k + np).
 void launch_tile_update(const TileView& v, int k, int np, int col_lo, int col_hi, hipStream_t s);
@@ -102,8 +106,6 @@ void launch_gemv_full(const TileView& v, const double* x, double* y, double* par
 void launch_gemv_full_partial(const TileView& v, const double* x, double* part, hipStream_t s);
 // y[i] = sum_{c < ncols} part[c*len + i], i < m.
 void launch_sum_columns(const double* part, int ncols, long len, double* y, long m, hipStream_t s);
-// Zero the strictly upper part of every diagonal tile of a lower matrix.
-void launch_zero_upper_diag(const TileView& v, hipStream_t s);
 
 // ---- mixed precision ---------------------------------------------------
 // dst <- src tile by tile (dst tiles FP64 or FP32 by dst.prec).

@@ -233,18 +233,6 @@ __global__ void k_sum_columns(const double* part, int ncols, long len, double* y
   y[i] = s;
 }
 
-__global__ void __launch_bounds__(256) k_zero_upper_diag(TileView v) {
-  const int k = blockIdx.y;
-  double* T = tile_f64(v, k, k);
-  const int c = blockIdx.x;
-  for (int r = threadIdx.x; r < c; r += 256) T[r + (long)c * v.ts] = 0.0;
-}
-
-void launch_zero_upper_diag(const TileView& v, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_upper_diag, dim3(v.ts, v.mt), dim3(256), 0, s, v);
-  EXA_HIP(hipGetLastError());
-}
-
 void launch_trmv_diag(const double* X, int ts, const double* t, double* y, int trans, double* part,
                       unsigned* ticket, hipStream_t s) {
   const int q = ts / kNB;

@@ -620,8 +620,8 @@ void exact_mloe_mmom(double *xobs, int *xobs_len, double *yobs, int *yobs_len, d
 
 /* ------------------------------------------------------------ measurement -- */
 /* No counterpart in the reference.  Per-kernel HIP-event timing on the
- * launching stream ("tile_update", "potrf_diag", "trsm_panel", "gen", "trsv"),
- * used by the benchmark; off by default. */
+ * launching stream ("tile_update", "potrf_diag" (diagonal blocks, panels and
+ * dataflow launches), "gen", "trsv"), used by the benchmark; off by default. */
 void exageostat_gpu_synchronize(void);
 /* No counterpart in the reference.  Tile precision classes (0 FP64, 1 FP32,
  * 3 FP32 storage with BF16 updates) of the last mixed-precision evaluation
