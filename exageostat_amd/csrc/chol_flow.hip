@@ -56,11 +56,19 @@ __device__ __forceinline__ void store_through(T* p, T v) {
   __hip_atomic_store((gT*)(uintptr_t)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ double lane_value(double x, int lane) {
-  const long u = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_readlane((int)u, lane);
-  const int hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
-  return __longlong_as_double(((long)hi << 32) | (unsigned)lo);
+// x of lane N of each row of 16 lanes, in all lanes of that row.
+template <int N>
+__device__ __forceinline__ double row_lane(double x) {
+  return __longlong_as_double(
+      __builtin_amdgcn_update_dpp(0L, (long)__double_as_longlong(x), 0x150 + N, 0xf, 0xf, true));
+}
+
+// 1/y for normal y: the hardware estimate (relative error 4.7e-8 measured)
+// with one third-order step, three dependent operations.
+__device__ __forceinline__ double recip3(double y) {
+  const double r = __builtin_amdgcn_rcp(y);
+  const double e = fma(-y, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 
 // 1/sqrt(x) and sqrt(x) for normal x > 0: the hardware estimate refined by
@@ -78,36 +86,65 @@ __device__ __forceinline__ void rsqrt_pair(double x, double& rs, double& s) {
   rs = h + h;
 }
 
-// Factors a 16-column panel held one row per lane (the diagonal block's rows
-// in lanes 0 .. 15), by the square-root-free elimination
-//   a_{r,c2} -= (a_rc / d_c) a_{c2,c},  d_c = a_cc,
-// whose columns are scaled by 1/sqrt(d_c) off the dependent chain (a
-// reciprocal per column on it, instead of a reciprocal square root and a
-// product).  Rows below the diagonal block come out as rows of L, rows of an
-// identity as rows of L^-T.  Returns the mask of columns whose pivot is not
-// positive; those and all later columns are NaN then.
-__device__ __forceinline__ unsigned panel16(double (&a)[16], int lane) {
-  unsigned bad = 0;
-  double root[16];
-#pragma unroll
-  for (int c = 0; c < 16; ++c) {
-    const double piv = lane_value(a[c], c);
-    bad |= (piv > 0.0) ? 0u : (1u << c);
-    const double b = a[c] * recip(piv);
-#pragma unroll
-    for (int c2 = c + 1; c2 < 16; ++c2) a[c2] = fma(-b, lane_value(a[c], c2), a[c2]);
-    double rs;
-    rsqrt_pair(piv, rs, root[c]);
-    a[c] *= rs;
+// One column of panel16, then the next ones.
+template <int C>
+__device__ __forceinline__ void panel_columns(double (&d)[16], double (&a)[16], double& own, int l16);
+template <int C, int C2>
+__device__ __forceinline__ void panel_update(double (&d)[16], double (&a)[16], double nd, double na) {
+  if constexpr (C2 < 16) {
+    const double s = row_lane<C2>(d[C]);
+    d[C2] = fma(s, nd, d[C2]);
+    a[C2] = fma(s, na, a[C2]);
+    panel_update<C, C2 + 1>(d, a, nd, na);
   }
+}
+template <int C>
+__device__ __forceinline__ void panel_columns(double (&d)[16], double (&a)[16], double& own, int l16) {
+  if constexpr (C < 16) {
+    const double piv = row_lane<C>(d[C]);
+    own = l16 == C ? piv : own;
+    const double r = recip3(piv);
+    panel_update<C, C + 1>(d, a, -d[C] * r, -a[C] * r);
+    panel_columns<C + 1>(d, a, own, l16);
+  }
+}
+template <int C>
+__device__ __forceinline__ void panel_scale(double (&d)[16], double (&a)[16], double rs) {
+  if constexpr (C < 16) {
+    const double r = row_lane<C>(rs);
+    d[C] *= r;
+    a[C] *= r;
+    panel_scale<C + 1>(d, a, rs);
+  }
+}
+
+// Factors a 16-column panel by one wave.  d: the 16 x 16 diagonal block, row
+// i in lane i of each row of 16 lanes (all four hold a copy, so that its
+// entries reach every lane by a DPP broadcast inside the row); a: 64 more
+// rows, one per lane.  Square-root-free elimination
+//   a_{r,c2} -= (a_rc / d_c) d_{c2,c},  d_c = d_cc,
+// the columns scaled by 1/sqrt(d_c) at the end for all sixteen pivots at
+// once: the dependent chain per column is a broadcast, a reciprocal, a
+// product and an update.  1.13 us per panel; with v_readlane broadcasts into
+// scalar registers and a square root per column 2.05 us.
+// Rows below the diagonal block come out as rows of L, rows of an identity
+// as rows of L^-T.  Returns the mask of columns whose pivot is not positive;
+// those and all later columns are NaN then.
+__device__ __forceinline__ unsigned panel16(double (&d)[16], double (&a)[16], int lane) {
+  const int l16 = lane & 15;
+  double own = 1.0, rs, root;
+  panel_columns<0>(d, a, own, l16);
+  rsqrt_pair(own, rs, root);
+  panel_scale<0>(d, a, rs);
 #pragma unroll
   for (int c = 0; c < 16; ++c)
-    if (lane == c) a[c] = root[c];
+    if (l16 == c) d[c] = root;
+  const unsigned bad = (unsigned)__ballot(!(own > 0.0)) & 0xffffu;
   if (bad) {
     const int first = __builtin_ctz(bad);
 #pragma unroll
     for (int c = 0; c < 16; ++c)
-      if (c >= first) a[c] = __builtin_nan("");
+      if (c >= first) a[c] = d[c] = __builtin_nan("");
   }
   return bad;
 }
@@ -117,24 +154,19 @@ __device__ __forceinline__ unsigned panel16(double (&a)[16], int lane) {
 // to one MFMA is 64 consecutive doubles.
 __device__ __forceinline__ constexpr int blk16(int bi, int bj) { return (bi * (bi + 1) / 2 + bj) * 256; }
 
-// The diagonal fragments (bi, bj) of the 64 x 64 lower triangle by wave:
-// at most three each.
-__device__ __forceinline__ int diag_count(int w) { return (w == 1 || w == 2) ? 3 : 2; }
+// The diagonal fragments (bi, bj) of the 64 x 64 lower triangle by wave: the
+// first block column's, which the first panel waits for, one each; the other
+// six on waves 1 .. 3.
+__device__ __forceinline__ int diag_count(int w) { return w == 0 ? 1 : 3; }
 __device__ __forceinline__ void diag_frag(int w, int t, int& bi, int& bj) {
-  // w0: (0,0) (3,0); w1: (1,0) (1,1) (3,1); w2: (2,0) (2,1) (2,2); w3: (3,2) (3,3)
-  if (w == 0) {
-    bi = t ? 3 : 0;
-    bj = 0;
-  } else if (w == 1) {
-    bi = t == 2 ? 3 : 1;
-    bj = t == 0 ? 0 : 1;
-  } else if (w == 2) {
-    bi = 2;
-    bj = t;
-  } else {
+  // w0: (0,0); w1: (1,0) (1,1) (3,1); w2: (2,0) (2,1) (2,2); w3: (3,0) (3,2) (3,3)
+  bi = w;
+  bj = t;
+  if (w == 1 && t == 2) {
     bi = 3;
-    bj = 2 + t;
+    bj = 1;
   }
+  if (w == 3 && t > 0) bj = t + 1;
 }
 
 }  // namespace
@@ -177,11 +209,11 @@ __device__ __forceinline__ char* block_ptr(const FlowArgs& a, Row r, int l, int 
 
 // Waits until the (relative) counters of four rows all exceed l and returns
 // the smallest; lane t of wave 0 polls row t % 4.
-__device__ __forceinline__ int wait_rows(const FlowArgs& a, const int (&rows)[4], int l, int* sh) {
+__device__ __forceinline__ int wait_rows(const FlowArgs& a, int r0, int r1, int r2, int r3, int l, int* sh) {
   if (threadIdx.x < 64) {
     const int t = threadIdx.x;
     const int u = t & 3;
-    const int* f = a.flags + kRows + 16 * ((u < 2 ? (u ? rows[1] : rows[0]) : (u == 2 ? rows[2] : rows[3])) - a.j0);
+    const int* f = a.flags + kRows + 16 * ((u < 2 ? (u ? r1 : r0) : (u == 2 ? r2 : r3)) - a.j0);
     int got;
     for (;;) {
       got = flag_get(f);
@@ -348,7 +380,7 @@ __device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], d
     if constexpr (DIAG) {
 #pragma unroll
       for (int t = 0; t < 3; ++t)
-        if (t < 2 || wave == 1 || wave == 2) dacc[t] = mfma_f64(fy[cur][t], fx[cur][t], dacc[t]);
+        if (t == 0 || wave != 0) dacc[t] = mfma_f64(fy[cur][t], fx[cur][t], dacc[t]);
     }
   };
   __builtin_amdgcn_s_barrier();
@@ -409,7 +441,6 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long ts = a.v.ts;
-  int rows[4] = {j, i0, i0 + nr - 1, i0 + (nr > 1 ? 1 : 0)};
   Row ra[R];
 #pragma unroll
   for (int p = 0; p < R; ++p) ra[p] = row_of(a, i0 + (p < nr ? p : 0));
@@ -421,7 +452,7 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
     for (int f = 0; f < 4; ++f) acc[p][f] = dx4{0.0, 0.0, 0.0, 0.0};
   int l = a.j0;
   while (l < j) {
-    int upto = a.j0 + wait_rows(a, rows, l - a.j0, sh);
+    int upto = a.j0 + wait_rows(a, j, i0, i0 + nr - 1, i0 + (nr > 1 ? 1 : 0), l - a.j0, sh);
     if (upto > j) upto = j;
     flow_gemm<R, TA, false>(a, acc, none, ra, rj, l, upto, lds);
     l = upto;
@@ -445,7 +476,77 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
   if (tid < nr) flag_set(a.flags + kRows + 16 * (i0 + tid - a.j0), j - a.j0 + 1);
 }
 
-// D task of block column j.
+// LDS of a D task (doubles): the operand ring, then X = L_{j,j-1}; the
+// factor's and the inverse's 16 x 16 blocks.
+constexpr int kLs = 4096, kXs = kLs + 2560, kDiagLds = kXs + 2560;
+
+// S(bi, bj) -= L(bi, p) L(bj, p)^T
+__device__ __forceinline__ void diag_update(double* Ls, int bi, int bj, int p, int lane) {
+  double* S = Ls + blk16(bi, bj) + lane;
+  const double* A = Ls + blk16(bi, p) + lane;
+  const double* B = Ls + blk16(bj, p) + lane;
+  dx4 s = {S[0], S[64], S[128], S[192]};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) s = mfma_f64(-B[e * 64], A[e * 64], s);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) S[e * 64] = s[e];
+}
+// y += L(p, l) X(l, b); y: lane l, element v at row l/16 + 4 v, column l%16.
+__device__ __forceinline__ void inverse_sum(const double* Ls, const double* Xs, dx4& y, int p, int l, int b,
+                                            int lane) {
+  const double* A = Ls + blk16(p, l) + lane;
+  const double* B = Xs + blk16(l, b) + (lane & 15) * 16 + (lane >> 4);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y = mfma_f64(A[e * 64], B[e * 4], y);
+}
+// X(p, b) = -X(p, p) y
+__device__ __forceinline__ void inverse_put(double* Xs, const dx4& y, int p, int b, int lane) {
+  const double* D = Xs + blk16(p, p) + lane;
+  dx4 x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x = mfma_f64(-y[e], D[e * 64], x);
+  double* dst = Xs + blk16(p, b) + lane;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) dst[e * 64] = x[e];
+}
+
+// Panel p of the diagonal block, by one wave.
+__device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, double* Ls, double* Xs, int lane) {
+  // lanes 0 .. 15 of c: an identity (its rows become the inverse's columns);
+  // 16 .. 63: block rows p + 1 ..
+  double d[16], c[16];
+  const int l16 = lane & 15, bi = p + (lane >> 4);
+  const double* dd = Ls + blk16(p, p) + l16;
+  const double* cc = Ls + blk16(bi < 4 ? bi : p, p) + l16;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    d[e] = dd[e * 16];
+    c[e] = cc[e * 16];
+  }
+#pragma unroll
+  for (int e = 0; e < 16; ++e) c[e] = lane < 16 ? (lane == e ? 1.0 : 0.0) : c[e];
+  const unsigned bad = panel16(d, c, lane);
+  if (bad && lane == 0) atomicCAS(a.info, 0, j * kNB + 16 * p + __builtin_ctz(bad) + 1);
+  if (lane < 16) {
+    double* dst = Xs + blk16(p, p) + lane * 16;
+    double* ldst = Ls + blk16(p, p) + lane;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      dst[e] = c[e];
+      ldst[e * 16] = lane >= e ? d[e] : 0.0;
+    }
+  } else if (bi < 4) {
+    double* dst = Ls + blk16(bi, p) + l16;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) dst[e * 16] = c[e];
+  }
+}
+
+// D task of block column j.  After the hand-over from D_{j-1}: X = L_{j,j-1},
+// S = A_jj - sum L L^T, then four 16-column panels of S by wave 0, while
+// waves 1 .. 3 bring the blocks that the next panels need up to date and
+// build the inverse; block row bi of S and of the inverse's sums stays with
+// wave bi.
 __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds, int* sh) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -454,153 +555,106 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
   const Row rj = row_of(a, j);
   const int nd = diag_count(wave);
   __builtin_amdgcn_s_setprio(2);
-  dx4 acc[1][4], dacc[3];
+  double* Ls = lds + kLs;
+  double* Xs = lds + kXs;
+  dx4 acc[1][4], dacc[3], cd[3];
 #pragma unroll
   for (int f = 0; f < 4; ++f) acc[0][f] = dx4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int t = 0; t < 3; ++t) dacc[t] = dx4{0.0, 0.0, 0.0, 0.0};
   char* cjj = block_ptr(a, rj, j, 8);
-  if (j > a.j0) {
+  const bool chained = j > a.j0;
+  char* cp = nullptr;
+  if (chained) {
     const Row rp[1] = {row_of(a, j - 1)};
-    int rows[4] = {j, j - 1, j, j - 1};
     int l = a.j0;
     while (l < j - 1) {
-      int upto = a.j0 + wait_rows(a, rows, l - a.j0, sh);
+      int upto = a.j0 + wait_rows(a, j, j - 1, j, j - 1, l - a.j0, sh);
       if (upto > j - 1) upto = j - 1;
       flow_gemm<1, double, true>(a, acc, dacc, rp, rj, l, upto, lds);
       l = upto;
     }
-    char* cp = block_ptr(a, rj, j - 1, 8);
+    cp = block_ptr(a, rj, j - 1, 8);
     block_minus<double>(cp, ts, wave, lane, acc[0]);
-    // the diagonal block, ahead of the wait
-    dx4 cd[3];
-    {
-      typedef __attribute__((address_space(1))) const double gD;
+  }
+  // the diagonal block, ahead of the wait
 #pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        int bi, bj;
-        diag_frag(wave, t < nd ? t : 0, bi, bj);
-        gD* G = (gD*)(uintptr_t)cjj + 16 * bi + (lane & 15) + (long)(16 * bj + (lane >> 4)) * ts;
+  for (int t = 0; t < 3; ++t) {
+    int bi, bj;
+    diag_frag(wave, t < nd ? t : 0, bi, bj);
+    gdouble* G = (gdouble*)(uintptr_t)cjj + 16 * bi + (lane & 15) + (long)(16 * bj + (lane >> 4)) * ts;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) cd[t][v] = G[(long)(4 * v) * ts];
-      }
+    for (int v = 0; v < 4; ++v) cd[t][v] = G[(long)(4 * v) * ts];
+  }
+  // S's fragment t: minus X X^T when there is one, into LDS
+  auto s_frag = [&](int t) {
+    int bi, bj;
+    diag_frag(wave, t, bi, bj);
+    if (chained) {
+      const double* X = lds + bi * 1024 + lane;
+      const double* Y = lds + bj * 1024 + lane;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) dacc[t] = mfma_f64(Y[e * 64], X[e * 64], dacc[t]);
     }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) Ls[blk16(bi, bj) + v * 64 + lane] = cd[t][v] - dacc[t][v];
+  };
+  if (chained) {
     wait_diag(a, j - a.j0);
-    load_inverse(a.dinv + (long)(j - 1) * 4096, lds, wave, lane);
+    load_inverse(a.dinv + (long)(j - 1) * 4096, Xs, wave, lane);
     wait_vmcnt<0>();
     __syncthreads();
     dx4 x[4];
-    times_inverse(acc[0], x, lds, lane);
-    block_store<double>(cp, ts, wave, lane, x);
-    __syncthreads();
+    times_inverse(acc[0], x, Xs, lane);
     // X as sixteen 16 x 16 blocks (row block w, column block f), for X X^T
 #pragma unroll
     for (int f = 0; f < 4; ++f)
 #pragma unroll
       for (int v = 0; v < 4; ++v) lds[(wave * 4 + f) * 256 + v * 64 + lane] = x[f][v];
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      if (t < nd) {
-        int bi, bj;
-        diag_frag(wave, t, bi, bj);
-        const double* X = lds + bi * 1024 + lane;
-        const double* Y = lds + bj * 1024 + lane;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) dacc[t] = mfma_f64(Y[e * 64], X[e * 64], dacc[t]);
-      }
-    }
-    stores_done();
-    __syncthreads();
-    if (tid == 0) flag_set(a.flags + kRows + 16 * (j - a.j0), j - a.j0);
-#pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      if (t < nd) {
-        int bi, bj;
-        diag_frag(wave, t, bi, bj);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) lds[blk16(bi, bj) + v * 64 + lane] = cd[t][v] - dacc[t][v];
-      }
-    }
-  } else {
-    typedef __attribute__((address_space(1))) const double gD;
-#pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      if (t < nd) {
-        int bi, bj;
-        diag_frag(wave, t, bi, bj);
-        gD* G = (gD*)(uintptr_t)cjj + 16 * bi + (lane & 15) + (long)(16 * bj + (lane >> 4)) * ts;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) lds[blk16(bi, bj) + v * 64 + lane] = G[(long)(4 * v) * ts];
-      }
-    }
+    block_store<double>(cp, ts, wave, lane, x);
   }
   __syncthreads();
-  double* Ls = lds;
-  double* Xs = lds + 2560;
-  for (int p = 0; p < 4; ++p) {
+  s_frag(0);
+  __syncthreads();
+  if (wave == 0) {
+    diag_panel(a, j, 0, Ls, Xs, lane);
+  } else {
+    s_frag(1);
+    s_frag(2);
+  }
+  stores_done();
+  __syncthreads();
+  if (chained && tid == 64) flag_set(a.flags + kRows + 16 * (j - a.j0), j - a.j0);
+  if (wave > 0) diag_update(Ls, wave, 1, 0, lane);
+  __syncthreads();
+  dx4 y = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+  for (int p = 1; p < 4; ++p) {
     if (wave == 0) {
-      // rows 16 p + lane
-      double c[16];
-      const int bi = p + (lane >> 4);
-      const double* src = Ls + blk16(bi < 4 ? bi : p, p) + (lane & 15);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) c[e] = src[e * 16];
-      const unsigned bad = panel16(c, lane);
-      if (bad && lane == 0) atomicCAS(a.info, 0, j * kNB + 16 * p + __builtin_ctz(bad) + 1);
-      if (bi < 4) {
-        double* dst = Ls + blk16(bi, p) + (lane & 15);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) dst[e * 16] = (bi > p || lane >= e) ? c[e] : 0.0;
+      diag_panel(a, j, p, Ls, Xs, lane);
+    } else {
+      // what panel p - 1 leaves for the panels after p, and the inverse
+      for (int bj = p + 1; bj <= wave; ++bj) diag_update(Ls, wave, bj, p - 1, lane);
+      if (p == 2 && wave == 1) {
+        dx4 z = {0.0, 0.0, 0.0, 0.0};
+        inverse_sum(Ls, Xs, z, 1, 0, 0, lane);
+        inverse_put(Xs, z, 1, 0, lane);
       }
-    } else if (wave == 1) {
-      // the diagonal block again in lanes 0 .. 15, an identity in 16 .. 31:
-      // its rows come out as rows of the inverse transposed
-      double c[16];
-      const double* src = Ls + blk16(p, p) + (lane & 15);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) c[e] = lane < 16 ? src[e * 16] : (lane == 16 + e ? 1.0 : 0.0);
-      panel16(c, lane);
-      if (lane >= 16 && lane < 32) {
-        double* dst = Xs + blk16(p, p) + (lane - 16) * 16;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) dst[e] = c[e];
+      if (p == 3 && wave < 3) {
+        const int b = wave - 1;
+        dx4 z = {0.0, 0.0, 0.0, 0.0};
+        for (int l = b; l < 2; ++l) {
+          inverse_sum(Ls, Xs, z, 2, l, b, lane);
+          inverse_sum(Ls, Xs, y, 3, l, b, lane);
+        }
+        inverse_put(Xs, z, 2, b, lane);
       }
     }
     __syncthreads();
-    // Trailing fragments (bi, bj), p < bj <= bi, and the inverse's row p:
-    // X_p,b = -X_pp sum_{b <= l < p} L_pl X_lb.
-    const int nt = (3 - p) * (4 - p) / 2;
-    for (int t = wave; t < nt + p; t += 4) {
-      if (t < nt) {
-        const int r = t < 1 ? 0 : (t < 3 ? 1 : 2);
-        const int bi = p + 1 + r, bj = p + 1 + t - r * (r + 1) / 2;
-        double* S = Ls + blk16(bi, bj) + lane;
-        const double* A = Ls + blk16(bi, p) + lane;
-        const double* B = Ls + blk16(bj, p) + lane;
-        dx4 s = {S[0], S[64], S[128], S[192]};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s = mfma_f64(-B[e * 64], A[e * 64], s);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S[e * 64] = s[e];
-      } else {
-        const int b = t - nt;
-        dx4 y = {0.0, 0.0, 0.0, 0.0};
-        for (int l = b; l < p; ++l) {
-          const double* A = Ls + blk16(p, l) + lane;
-          const double* B = Xs + blk16(l, b) + (lane & 15) * 16 + (lane >> 4);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) y = mfma_f64(A[e * 64], B[e * 4], y);
-        }
-        // y: lane l, element v at row l/16 + 4 v, column l%16
-        const double* D = Xs + blk16(p, p) + lane;
-        dx4 x = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x = mfma_f64(-y[e], D[e * 64], x);
-        double* dst = Xs + blk16(p, b) + lane;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) dst[e * 64] = x[e];
-      }
+    if (wave > p) diag_update(Ls, wave, p + 1, p, lane);
+    if (p == 3 && wave > 0) {
+      inverse_sum(Ls, Xs, y, 3, 2, wave - 1, lane);
+      inverse_put(Xs, y, 3, wave - 1, lane);
     }
     __syncthreads();
   }
@@ -669,7 +723,8 @@ __host__ __device__ __forceinline__ int rows_from(int j, int j1) { return j + 1 
 
 template <int R, bool MIXED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_chol_flow(FlowArgs a) {
-  __shared__ __attribute__((aligned(16))) double lds[R == 1 ? 5120 : 2048 * (R + 1)];
+  __shared__ __attribute__((aligned(16))) double lds[kDiagLds];
+  static_assert(2 * (R + 1) * kPanel <= kDiagLds, "the T tasks' ring");
   __shared__ int sh[2];
   const int tid = threadIdx.x;
   int j = a.j0;

@@ -554,7 +554,7 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
   // with that panel on s1.
   // The FP64 factor's last kFlowBlocks block columns go into one dataflow
   // launch: its left-looking tasks reach 46-54 TFLOP/s against 60-70 of the
-  // trailing update, but its chain costs 20 us per 64 columns where the tile
+  // trailing update, but its chain costs 17 us per 64 columns where the tile
   // steps wait for a panel and two partial update rounds (n = 12,000: 11.8
   // against 16.1 ms; the whole of n = 20,000: 50 ms, with 100 blocks left to
   // it 50.6, 200: 48.7, 320: 51.3; n = 40,000: 352, 350 and 354 ms).
