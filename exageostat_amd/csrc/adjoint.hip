@@ -130,6 +130,9 @@ static MaternGradParams matern_grad_params(const Context& ctx, KernelId kid, con
   G.beta = theta[1];
   G.con = host_matern_con(theta[2]);
   knu_prepare(theta[2], G.ko);
+  // after the covariance that read the tables on this stream
+  G.tab = ctx.l1.tables();
+  launch_knu_table_grad(G.ko, G.con, ctx.l1.tables(), ctx.s1);
   return G;
 }
 

@@ -348,6 +348,18 @@ __global__ void __launch_bounds__(256) k_grad_matern(TileView v, MaternGradParam
         continue;
       }
       const double xx = d / P.beta;
+      if (P.tab && xx >= kTabLo && xx < kTabHi) {
+        double u;
+        const int row = table_row(xx, u) * kTabFuncs;
+        const double M = table_value(P.tab, row, u), B = table_value(P.tab, row + 1, u),
+                     V = table_value(P.tab, row + 2, u);
+        if (isfinite(M) && isfinite(B) && isfinite(V)) {
+          acc[0] += w * M;
+          acc[1] += w * P.sigma2 * B / P.beta;
+          acc[2] += w * P.sigma2 * V;
+          continue;
+        }
+      }
       Dual kn, kn1;
       knu_pair(P.ko, xx, kn, kn1);
       const Dual xnu = exp(P.ko.nu * ::log(xx));  // x^nu with d/dnu = x^nu ln x

@@ -263,7 +263,14 @@ void DeviceLocations::upload(const double* x, const double* y, long n_, hipStrea
   EXA_HIP(hipStreamSynchronize(s));
 }
 
+double* DeviceLocations::tables() const {
+  if (!tab) EXA_HIP(hipMalloc(&tab, sizeof(double) * kTabDoubles));
+  return tab;
+}
+
 void DeviceLocations::release() {
+  if (tab) (void)hipFree(tab);
+  tab = nullptr;
   if (dx) (void)hipFree(dx);
   if (dy) (void)hipFree(dy);
   if (dz) (void)hipFree(dz);
@@ -278,6 +285,13 @@ void generate_covariance(TileMatrix& A, KernelId kid, const double* theta, const
                          const DeviceLocations& cols, int metric, hipStream_t s) {
   if (!A.allocated()) throw std::invalid_argument("covariance generation into an unallocated tile matrix");
   generate_covariance_tiles(A.view(), kid, theta, rows, cols, metric, 0, A.num_tiles(), s);
+}
+
+// The correlation's table for one order, or null where it has a closed form.
+static const double* corr_table(const KnuOrder<double>& ko, double con, double* tab, hipStream_t s) {
+  if (ko.closed_form) return nullptr;
+  launch_knu_table(ko, con, tab, s);
+  return tab;
 }
 
 void generate_covariance_tiles(const TileView& v, KernelId kid, const double* theta, const DeviceLocations& rows,
@@ -299,6 +313,7 @@ void generate_covariance_tiles(const TileView& v, KernelId kid, const double* th
     P.nugget = (kid == kNugget) ? theta[3] : 0.0;
     P.con = 1.0 / (std::pow(2.0, theta[2] - 1.0) * std::tgamma(theta[2]));
     knu_prepare(theta[2], P.ko);
+    P.tab = corr_table(P.ko, P.con, rows.tables(), s);
     launch_gen_matern(v, P, p0, ntiles, s);
   } else if (kid == kBivariate || kid == kBivariateBlock) {
     if (kid == kBivariate && v.ts % 2 != 0) throw std::invalid_argument("bivariate kernel needs an even tile size");
@@ -327,6 +342,10 @@ void generate_covariance_tiles(const TileView& v, KernelId kid, const double* th
     knu_prepare(nu1, P.ko11);
     knu_prepare(nu2, P.ko22);
     knu_prepare(nu12, P.ko12);
+    constexpr long one = (long)kTabRows * kTabRow;
+    P.tab11 = corr_table(P.ko11, P.con11, rows.tables(), s);
+    P.tab22 = corr_table(P.ko22, P.con22, rows.tables() + one, s);
+    P.tab12 = corr_table(P.ko12, P.con12, rows.tables() + 2 * one, s);
     launch_gen_bivariate(v, P, p0, ntiles, kid == kBivariateBlock, s);
   } else if (kid == kSpaceTime) {
     if (!rows.dz || !cols.dz) throw std::invalid_argument("space-time kernel: locations need z (time)");
@@ -346,6 +365,7 @@ void generate_covariance_tiles(const TileView& v, KernelId kid, const double* th
     P.delta = theta[6];
     P.con = 1.0 / (std::pow(2.0, theta[2] - 1.0) * std::tgamma(theta[2]));
     knu_prepare(theta[2], P.ko);
+    P.tab = corr_table(P.ko, P.con, rows.tables(), s);
     launch_gen_spacetime(v, P, p0, ntiles, s);
   } else {
     throw std::invalid_argument("unsupported kernel");

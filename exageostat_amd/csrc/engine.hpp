@@ -102,6 +102,10 @@ struct DeviceLocations {
   double* dx = nullptr;
   double* dy = nullptr;
   double* dz = nullptr;  // third coordinate (3-D locations, or time), or null
+  // Scratch for the correlation tables of covariances with these locations
+  // as rows, filled and read in the order of the stream that generates them.
+  mutable double* tab = nullptr;
+  double* tables() const;
   void upload(const double* x, const double* y, long n_, hipStream_t s, const double* z = nullptr);
   void release();
   ~DeviceLocations() { release(); }

@@ -13,6 +13,8 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
+#include <cstring>
+
 namespace exa {
 
 __device__ inline uint16_t f32_to_bf16_rne(float f) {
@@ -74,6 +76,134 @@ __device__ inline bool decode_gen_block(const TileView& v, long p_off, int& m, i
   return true;
 }
 
+// ------------------------------------------------------ table of M_nu(x) --
+// Nodes (in 1/1024) and the least-squares matrix from the node values to the
+// Chebyshev coefficients of degree <= 8.
+struct TableFit {
+  short node[kTabNodes];
+  double fit[kTabDeg + 1][kTabNodes];
+};
+
+static TableFit make_table_fit() {
+  TableFit t;
+  constexpr int D = kTabDeg + 1;
+  long double T[kTabNodes][D], A[D][D + kTabNodes];
+  for (int i = 0; i < kTabNodes; ++i) {
+    t.node[i] = (short)std::lrint(1024.0 * std::cos((2 * i + 1) * M_PI / (2 * kTabNodes)));
+    const long double u = (long double)t.node[i] / 1024;
+    T[i][0] = 1;
+    T[i][1] = u;
+    for (int k = 2; k < D; ++k) T[i][k] = 2 * u * T[i][k - 1] - T[i][k - 2];
+  }
+  for (int r = 0; r < D; ++r) {
+    for (int c = 0; c < D; ++c) {
+      A[r][c] = 0;
+      for (int i = 0; i < kTabNodes; ++i) A[r][c] += T[i][r] * T[i][c];
+    }
+    for (int i = 0; i < kTabNodes; ++i) A[r][D + i] = T[i][r];
+  }
+  for (int r = 0; r < D; ++r) {  // the Gram matrix is nearly diagonal
+    const long double p = 1 / A[r][r];
+    for (int c = 0; c < D + kTabNodes; ++c) A[r][c] *= p;
+    for (int q = 0; q < D; ++q)
+      if (q != r) {
+        const long double f = A[q][r];
+        for (int c = 0; c < D + kTabNodes; ++c) A[q][c] -= f * A[r][c];
+      }
+  }
+  for (int k = 0; k < D; ++k)
+    for (int i = 0; i < kTabNodes; ++i) t.fit[k][i] = (double)A[k][D + i];
+  return t;
+}
+
+// A general order costs some 3,000 multiply-adds per entry (series or
+// continued fraction, two exponentials, two logarithms): generation was bound
+// by them, 12.8e9 entries/s.  With a table per evaluation (13 us, 19 us with
+// the gradient's functions) an entry is a distance, a gather of nine
+// coefficients and eight multiply-adds, 170e9 entries/s: n = 5,003 1,089 ->
+// 79 us, n = 40,000 42.8 -> 3.8 ms, the gradient's reduction at n = 12,000
+// 7.43 -> 1.00 ms.  Closed forms (nu = 1/2, 3/2, 5/2) stay direct.
+//
+// Half a wave per interval, a lane per node.  The values are fitted relative
+// to the middle one, so that the small high coefficients do not carry its
+// rounding; the change from the Chebyshev to the power basis has integer
+// coefficients.
+template <int NF, class T>
+__global__ void __launch_bounds__(256) k_knu_table(KnuOrder<T> ko, T con, TableFit fit, double* tab) {
+  const int lane = threadIdx.x & 31;
+  const int row = blockIdx.x * 8 + (threadIdx.x >> 5);
+  if (row >= kTabRows) return;
+  double mid, half;
+  if (row < kTabLow) {
+    half = ldexp(1.0, kTabLoExp + (row >> 4) - 5);
+    mid = half * (33 + 2 * (row & 15));
+  } else {
+    half = 1.0 / 32;
+    mid = 2.0 + half * (2 * (row - kTabLow) + 1);
+  }
+  const double x = fma(half, fit.node[lane] * (1.0 / 1024), mid);  // exact
+  double f[NF];
+  if constexpr (NF == 1) {
+    f[0] = matern_corr(ko, con, x);
+  } else {
+    Dual kn, kn1;
+    knu_pair(ko, x, kn, kn1);
+    const Dual xnu = exp(ko.nu * ::log(x));
+    const Dual corr = con * xnu * kn;
+    f[0] = corr.v;
+    f[1] = con.v * (xnu.v * x * kn1.v - 2.0 * ko.nu.v * xnu.v * kn.v);
+    f[2] = corr.d;
+  }
+#pragma unroll
+  for (int q = 0; q < NF; ++q) {
+    const double fc = __shfl(f[q], kTabNodes / 2, 32);
+    const double g = f[q] - fc;
+    double c[kTabDeg + 1];
+#pragma unroll
+    for (int k = 0; k <= kTabDeg; ++k) {
+      double v = fit.fit[k][lane] * g;
+#pragma unroll
+      for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 32);
+      c[k] = v;
+    }
+    if (lane <= kTabDeg) {
+      // coefficient `lane` of sum_k c_k T_k(u)
+      double prev[kTabDeg + 1] = {1.0}, cur[kTabDeg + 1] = {0.0, 1.0};
+      double out = lane == 0 ? c[0] : (lane == 1 ? c[1] : 0.0);
+#pragma unroll
+      for (int k = 2; k <= kTabDeg; ++k) {
+        double next[kTabDeg + 1];
+#pragma unroll
+        for (int m = 0; m <= kTabDeg; ++m) next[m] = (m > 0 ? 2.0 * cur[m - 1] : 0.0) - prev[m];
+        double tm = 0.0;
+#pragma unroll
+        for (int m = 0; m <= kTabDeg; ++m) {
+          if (m == lane) tm = next[m];
+          prev[m] = cur[m];
+          cur[m] = next[m];
+        }
+        out = fma(tm, c[k], out);
+      }
+      if (lane == 0) out += fc;
+      tab[((long)row * NF + q) * kTabRow + lane] = out;
+    }
+  }
+}
+
+template <int NF, class T>
+static void table_launch(const KnuOrder<T>& ko, T con, double* tab, hipStream_t s) {
+  static const TableFit fit = make_table_fit();
+  hipLaunchKernelGGL((k_knu_table<NF, T>), dim3((kTabRows + 7) / 8), dim3(256), 0, s, ko, con, fit, tab);
+  EXA_HIP(hipGetLastError());
+}
+
+void launch_knu_table(const KnuOrder<double>& ko, double con, double* tab, hipStream_t s) {
+  table_launch<1, double>(ko, con, tab, s);
+}
+void launch_knu_table_grad(const KnuOrder<Dual>& ko, Dual con, double* tab, hipStream_t s) {
+  table_launch<kTabFuncs, Dual>(ko, con, tab, s);
+}
+
 __global__ void __launch_bounds__(256) k_gen_matern(TileView v, MaternParams P, long p_off) {
   int m, n, bi, bj;
   decode_gen_block(v, p_off, m, n, bi, bj);
@@ -102,7 +232,7 @@ __global__ void __launch_bounds__(256) k_gen_matern(TileView v, MaternParams P, 
       if (x == 0.0) {
         val = P.sigma2 + P.nugget;
       } else {
-        val = P.sigma2 * matern_corr(P.ko, P.con, x);
+        val = P.sigma2 * matern_corr_tab(P.tab, P.ko, P.con, x);
       }
     }
     store_prec(base, (long)i + (long)j * ts, val, prec);
@@ -150,9 +280,9 @@ __global__ void __launch_bounds__(256) k_gen_bivariate(TileView v, BivariatePara
         a11 = P.sigma22;
         a10 = a01 = P.sigma12;
       } else {
-        a00 = P.sigma11 * matern_corr(P.ko11, P.con11, x);
-        a11 = P.sigma22 * matern_corr(P.ko22, P.con22, x);
-        a10 = a01 = P.sigma12 * matern_corr(P.ko12, P.con12, x);
+        a00 = P.sigma11 * matern_corr_tab(P.tab11, P.ko11, P.con11, x);
+        a11 = P.sigma22 * matern_corr_tab(P.tab22, P.ko22, P.con22, x);
+        a10 = a01 = P.sigma12 * matern_corr_tab(P.tab12, P.ko12, P.con12, x);
       }
     }
     store_prec(base, (long)i + (long)j * ts, a00, prec);
@@ -202,11 +332,11 @@ __global__ void __launch_bounds__(256) k_gen_bivariate_block(TileView v, Bivaria
       if (x == 0.0) {
         val = sg;
       } else if (c == 0) {
-        val = sg * matern_corr(P.ko11, P.con11, x);
+        val = sg * matern_corr_tab(P.tab11, P.ko11, P.con11, x);
       } else if (c == 1) {
-        val = sg * matern_corr(P.ko12, P.con12, x);
+        val = sg * matern_corr_tab(P.tab12, P.ko12, P.con12, x);
       } else {
-        val = sg * matern_corr(P.ko22, P.con22, x);
+        val = sg * matern_corr_tab(P.tab22, P.ko22, P.con22, x);
       }
     }
     store_prec(base, (long)i + (long)j * ts, val, prec);
@@ -247,7 +377,7 @@ __global__ void __launch_bounds__(256) k_gen_spacetime(TileView v, SpaceTimePara
         val = P.sigma2 / den;
       } else {
         const double x = xs / pow(psi, 0.5 * P.beta);
-        val = P.sigma2 * matern_corr(P.ko, P.con, x) / den;
+        val = P.sigma2 * matern_corr_tab(P.tab, P.ko, P.con, x) / den;
       }
     }
     store_prec(base, (long)i + (long)j * ts, val, prec);

@@ -20,6 +20,7 @@ struct MaternParams {
   double sigma2;  // variance
   double nugget;  // added where the distance is exactly 0
   double con;     // 1/(2^(nu-1) Gamma(nu))
+  const double* tab;  // table of the correlation (launch_knu_table), or null
   KnuOrder<double> ko;
 };
 
@@ -35,6 +36,7 @@ struct BivariateParams {
   double beta;
   double sigma11, sigma22, sigma12;  // variances and rho~ sqrt(s1 s2)
   double con11, con22, con12;
+  const double *tab11, *tab22, *tab12;  // tables of the correlations, or null
   KnuOrder<double> ko11, ko22, ko12;
 };
 
@@ -52,8 +54,14 @@ struct SpaceTimeParams {
   int metric;
   double sigma2, beta_s, a, alpha, beta, delta;
   double con;  // 1/(2^(nu-1) Gamma(nu))
+  const double* tab;
   KnuOrder<double> ko;
 };
+
+// Table of M_nu (kTabRows * kTabRow doubles at tab), or, in rows of
+// kTabFuncs times that, of M_nu and its two derivative functions.
+void launch_knu_table(const KnuOrder<double>& ko, double con, double* tab, hipStream_t s);
+void launch_knu_table_grad(const KnuOrder<Dual>& ko, Dual con, double* tab, hipStream_t s);
 
 // Generation of ntiles tiles starting at tile p_off of the matrix's
 // enumeration (lower matrices: p = m (m + 1) / 2 + n, row by row; full
@@ -153,6 +161,7 @@ struct MaternGradParams {
   double sigma2;
   double beta;
   Dual con;               // 1/(2^(nu-1) Gamma(nu)) and its nu-derivative
+  const double* tab;      // launch_knu_table_grad's table, or null
   KnuOrder<Dual> ko;      // K_nu constants with nu-derivatives
 };
 // One stage of tile column k of the Takahashi sweep Z = Sigma^-1 over the
