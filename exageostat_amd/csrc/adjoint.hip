@@ -220,7 +220,9 @@ double adjoint_loglik_grad(Context& ctx, KernelId kid, const double* theta, int 
     for (int p = 0; p < np; ++p) grad[p] = std::nan("");
     return ll;
   }
-  gradient_from_factor(ctx, kid, theta, metric, ctx.fp64("the gradient and the Fisher information"), false, grad);
+  TileMatrix& A = ctx.fp64("the gradient and the Fisher information");
+  if (one_launch(A)) tile_inverses(A, ctx.ws, ctx.s1);
+  gradient_from_factor(ctx, kid, theta, metric, A, false, grad);
   const double t1 = wall_seconds();
   ctx.last = lt;
   ctx.last.grad = t1 - t0 - lt.total;
@@ -297,6 +299,7 @@ int fisher_information(Context& ctx, KernelId kid, const double* theta, int metr
   AdjointState& st = adjoint_buffers(ctx);
   TileMatrix& A = ctx.fp64("the gradient and the Fisher information");
   hipStream_t s = ctx.s1;
+  if (one_launch(A)) tile_inverses(A, ctx.ws, s);
   if (!st.D.allocated() || st.D.mt != A.mt || st.D.ts != A.ts) {
     st.D.release();
     st.M.release();

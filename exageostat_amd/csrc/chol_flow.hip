@@ -12,8 +12,10 @@
 //   D_j  (one task per block column j): block (j, j-1) and the diagonal:
 //        L_{j,j-1} = (A_{j,j-1} - sum_l L_jl L_{j-1,l}^T) inv(L_{j-1,j-1})^T,
 //        L_jj = chol(A_jj - sum_l L_jl L_jl^T), and inv(L_jj);
-//   T_ij (block rows i > j+1, one or two of them per task):
+//   T_ij (block rows i > j+1, two or three of them per task):
 //        L_ij = (A_ij - sum_l L_il L_jl^T) inv(L_jj)^T.
+// A right-hand side z is one more block row (z^T above zeros): its T tasks
+// turn it into (L^-1 z)^T beside the factorisation.
 // The sums run as far as their operands are final and then wait for the
 // next ones, so the serial chain is, per 64 columns: one 64^3 product, one
 // symmetric 64^2 x 64 product, the factorisation and inverse of one 64 x 64
@@ -182,6 +184,8 @@ struct FlowArgs {
   double* dinv;   // inverse of diagonal block j at dinv + 4096 j
   int* info;
   int* flags;
+  double* rhs;    // one more block row, i_end: 64 x 64 blocks in sequence, its rows solved with the factor
+  long long* clock;  // receives the first and the last work-group's wall clock
 };
 
 namespace {
@@ -276,10 +280,11 @@ __device__ __forceinline__ void times_inverse(const dx4 (&t)[4], dx4 (&x)[4], co
 constexpr int kPanel = 1024;
 
 // acc[p][f] += A_p B^T over block columns [l, l_end): A_p the block rows
-// `ra` (R of them; FP32 tiles when TA is float), B the block row rb.
+// `ra` (R of them; FP32 tiles when TA is float; with RHS the right-hand
+// sides' row instead), B the block row rb.
 // DIAG: instead, panel 0 is block row ra[0] = j-1 and panel B is j, and
 // acc[0][f] += B A^T, dacc += the wave's fragments of B B^T.
-template <int R, class TA, bool DIAG>
+template <int R, class TA, bool DIAG, bool RHS = false>
 __device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], dx4 (&dacc)[3], const Row (&ra)[R],
                                           Row rb, int l, int l_end, double* lds) {
   constexpr bool kF = sizeof(TA) == 4;
@@ -295,15 +300,17 @@ __device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], d
   const char* pa[R];
   const char* pb = block_ptr(a, rb, l, 8);
 #pragma unroll
-  for (int p = 0; p < R; ++p) pa[p] = block_ptr(a, ra[p], l, (int)sizeof(TA));
+  for (int p = 0; p < R; ++p)
+    pa[p] = RHS ? reinterpret_cast<char*>(a.rhs + (long)l * 4096) : block_ptr(a, ra[p], l, (int)sizeof(TA));
   int n = l / a.q;
   int left = (a.q - (l - n * a.q)) * 4;  // slices left in the current tile column
   // byte offsets of this lane's elements in a slice
-  uint32_t o8[2], o4;
+  uint32_t o8[2], o4, oz[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int kk = 4 * wave + 2 * e + (lane >> 5);
     o8[e] = (uint32_t)((((2 * (lane & 31)) ^ ((kk & 1) * 16)) + kk * ts) * 8);
+    if (RHS) oz[e] = (uint32_t)((((2 * (lane & 31)) ^ ((kk & 1) * 16)) + kk * kNB) * 8);
   }
   {
     const int kk = 4 * wave + (lane >> 4);
@@ -314,7 +321,8 @@ __device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], d
       ++n;
       pb = block_ptr(a, rb, n * a.q, 8);
 #pragma unroll
-      for (int p = 0; p < R; ++p) pa[p] = block_ptr(a, ra[p], n * a.q, (int)sizeof(TA));
+      for (int p = 0; p < R; ++p)
+        if (!RHS) pa[p] = block_ptr(a, ra[p], n * a.q, (int)sizeof(TA));
       left = a.q * 4;
     }
     double* st = lds + buf * STAGE;
@@ -326,10 +334,10 @@ __device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], d
       } else {
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-          __builtin_amdgcn_global_load_lds((glb_void_t*)(uintptr_t)(pa[p] + o8[e]),
+          __builtin_amdgcn_global_load_lds((glb_void_t*)(uintptr_t)(pa[p] + (RHS ? oz[e] : o8[e])),
                                            (lds_void_t*)(st + p * A_PAN + (2 * wave + e) * 128), 16, 0, 0);
       }
-      pa[p] += (long)16 * ts * sizeof(TA);
+      pa[p] += (long)16 * (RHS ? kNB : ts) * sizeof(TA);
     }
 #pragma unroll
     for (int e = 0; e < 2; ++e)
@@ -474,6 +482,37 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
   stores_done();
   __syncthreads();
   if (tid < nr) flag_set(a.flags + kRows + 16 * (i0 + tid - a.j0), j - a.j0 + 1);
+}
+
+// The T task of the right-hand sides' row.
+__device__ __forceinline__ void task_rhs(const FlowArgs& a, int j, double* lds, int* sh) {
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const Row rj = row_of(a, j);
+  const Row none_row[1] = {rj};
+  dx4 acc[1][4], none[3];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) acc[0][f] = dx4{0.0, 0.0, 0.0, 0.0};
+  int l = a.j0;
+  while (l < j) {
+    int upto = a.j0 + wait_rows(a, j, a.i_end, j, a.i_end, l - a.j0, sh);
+    if (upto > j) upto = j;
+    flow_gemm<1, double, false, true>(a, acc, none, none_row, rj, l, upto, lds);
+    l = upto;
+  }
+  char* blk = reinterpret_cast<char*>(a.rhs + (long)j * 4096);
+  block_minus<double>(blk, kNB, wave, lane, acc[0]);
+  wait_diag(a, j - a.j0 + 1);
+  load_inverse(a.dinv + (long)j * 4096, lds, wave, lane);
+  wait_vmcnt<0>();
+  __syncthreads();
+  dx4 x[4];
+  times_inverse(acc[0], x, lds, lane);
+  block_store<double>(blk, kNB, wave, lane, x);
+  stores_done();
+  __syncthreads();
+  if (tid == 0) flag_set(a.flags + kRows + 16 * (a.i_end - a.j0), j - a.j0 + 1);
 }
 
 // LDS of a D task (doubles): the operand ring, then X = L_{j,j-1}; the
@@ -721,7 +760,7 @@ __device__ __forceinline__ void row_group(int t, int lo, int i_end, int q, int& 
 // j is the last column.
 __host__ __device__ __forceinline__ int rows_from(int j, int j1) { return j + 1 < j1 ? j + 2 : j + 1; }
 
-template <int R, bool MIXED>
+template <int R, bool MIXED, bool RHS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_chol_flow(FlowArgs a) {
   __shared__ __attribute__((aligned(16))) double lds[kDiagLds];
   static_assert(2 * (R + 1) * kPanel <= kDiagLds, "the T tasks' ring");
@@ -729,13 +768,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   const int tid = threadIdx.x;
   int j = a.j0;
   long base = 0;  // first task of column j
+  if (RHS && blockIdx.x == 0 && tid == 0) a.clock[0] = wall_clock64();
   for (;;) {
     if (tid == 0) sh[0] = atomicAdd(a.flags + kClaim, 1);
     __syncthreads();
     const long id = sh[0];
     __syncthreads();
     for (; j < a.j1; ++j) {
-      const int cnt = 1 + row_groups<R, MIXED>(rows_from(j, a.j1), a.i_end, a.q);
+      const int cnt = 1 + RHS + row_groups<R, MIXED>(rows_from(j, a.j1), a.i_end, a.q);
       if (id < base + cnt) break;
       base += cnt;
     }
@@ -747,9 +787,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         for (long e = tid; e < (long)(a.j_pad - a.j1) * 4096; e += 256)
           a.dinv[(long)a.j1 * 4096 + e] = ((e & 4095) % 65 == 0) ? 1.0 : 0.0;
       }
+    } else if (RHS && t == 1) {
+      task_rhs(a, j, lds, sh + 1);
     } else {
       int i0, nr;
-      row_group<R, MIXED>(t - 1, rows_from(j, a.j1), a.i_end, a.q, i0, nr);
+      row_group<R, MIXED>(t - 1 - RHS, rows_from(j, a.j1), a.i_end, a.q, i0, nr);
       if constexpr (MIXED) {
         if (a.v.prec[tile_index(a.v, i0 / a.q, a.k)] != kF64) task_rows<R, float>(a, i0, nr, j, lds, sh + 1);
         else task_rows<R, double>(a, i0, nr, j, lds, sh + 1);
@@ -762,34 +804,77 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   if (tid == 0) sh[0] = atomicAdd(a.flags + kExit, 1) == (int)gridDim.x - 1;
   __syncthreads();
   if (!sh[0]) return;
-  for (int e = tid; e < a.i_end - a.j0; e += 256) a.flags[kRows + 16 * e] = 0;
+  for (int e = tid; e < a.i_end - a.j0 + RHS; e += 256) a.flags[kRows + 16 * e] = 0;
+  if (RHS && tid == 0) a.clock[1] = wall_clock64();
   if (tid == 0) a.flags[kClaim] = a.flags[kExit] = a.flags[kDiag] = 0;
 }
 
-template <int R, bool MIXED>
+template <int R, bool MIXED, bool RHS = false>
 void launch_flow(const FlowArgs& a, hipStream_t s) {
   static int slots = 0;
   if (!slots) {
     int dev = 0, cus = 0, occ = 1;
     EXA_HIP(hipGetDevice(&dev));
     EXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_chol_flow<R, MIXED>, 256, 0));
+    EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_chol_flow<R, MIXED, RHS>, 256, 0));
     slots = cus * (occ > 0 ? occ : 1);
   }
   long tasks = 0;
   for (int j = a.j0; j < a.j1 && tasks < slots; ++j)
-    tasks += 1 + row_groups<R, MIXED>(rows_from(j, a.j1), a.i_end, a.q);
+    tasks += 1 + RHS + row_groups<R, MIXED>(rows_from(j, a.j1), a.i_end, a.q);
   long grid = tasks < slots ? tasks : slots;
-  hipLaunchKernelGGL((k_chol_flow<R, MIXED>), dim3((unsigned)grid), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((k_chol_flow<R, MIXED, RHS>), dim3((unsigned)grid), dim3(256), 0, s, a);
   EXA_HIP(hipGetLastError());
+}
+
+// Before a factorisation with a right-hand side: info = 0 and z into the
+// first row of the right-hand sides' blocks (zero beyond it since their
+// allocation: the rows never mix).
+__global__ void __launch_bounds__(256) k_flow_begin(const double* z, long n, double* rhs, int* info) {
+  const long c = (long)blockIdx.x * 256 + threadIdx.x;
+  if (c == 0) *info = 0;
+  if (c < n) rhs[c * kNB] = z[c];
+}
+
+// After it: y = L^-1 z into a vector, and per work-group the sums of y^2 and
+// of log L_ii over 256 rows, written with info to host memory.
+__global__ void __launch_bounds__(256) k_flow_end(TileView v, const double* rhs, long n, double* y, const int* info,
+                                                  const long long* clock, double* host) {
+  __shared__ double red[2][4];
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  double s = 0.0, d = 0.0;
+  if (i < n) {
+    const double w = rhs[i * kNB];
+    y[i] = w;
+    s = w * w;
+    const int k = (int)(i / v.ts);
+    const long r = i - (long)k * v.ts;
+    const double l = tile_f64(v, k, k)[r + r * v.ts];
+    if (l > 0.0) d = log(l);
+  }
+  s = wave_sum(s);
+  d = wave_sum(d);
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = s;
+    red[1][threadIdx.x >> 6] = d;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const double* r = red[threadIdx.x];
+    host[4 + 2 * blockIdx.x + threadIdx.x] = (r[0] + r[1]) + (r[2] + r[3]);
+  }
+  if (i == 0) {
+    host[0] = *info;
+    host[1] = (double)(clock[1] - clock[0]);
+  }
 }
 
 }  // namespace
 
-long chol_flow_flags(int mt, int ts) { return kRows + 16L * mt * (ts / kNB); }
+long chol_flow_flags(int mt, int ts) { return kRows + 16L * (mt * (ts / kNB) + 1); }
 
 void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int j1, int i_end, int j_pad,
-                      double* dinv, int* info, int* flags, hipStream_t s) {
+                      double* dinv, int* info, int* flags, hipStream_t s, double* rhs, long long* clock) {
   FlowArgs a;
   a.v = v;
   a.pool = pool;
@@ -802,14 +887,29 @@ void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int
   a.dinv = dinv;
   a.info = info;
   a.flags = flags;
+  a.rhs = rhs;
+  a.clock = clock;
   const int nb = v.mt * a.q;
   if (!v.lower || j0 < 0 || j1 <= j0 || j1 > nb || i_end < j1 || i_end > nb || j_pad > nb)
     throw std::invalid_argument("chol_flow: block range outside the matrix");
+  if (rhs && (!pool || !clock)) throw std::invalid_argument("chol_flow: right-hand sides go with the whole matrix and a clock");
   if (!pool && (tile_col < 0 || j0 < tile_col * a.q || j1 > (tile_col + 1) * a.q))
     throw std::invalid_argument("chol_flow: block columns outside the tile column");
-  if (pool) launch_flow<2, false>(a, s);
+  if (rhs) launch_flow<2, false, true>(a, s);
+  else if (pool) launch_flow<2, false>(a, s);
   else if (v.prec) launch_flow<3, true>(a, s);
   else launch_flow<3, false>(a, s);
+}
+
+void launch_flow_begin(const double* z, long n, double* rhs, int* info, hipStream_t s) {
+  hipLaunchKernelGGL(k_flow_begin, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, z, n, rhs, info);
+  EXA_HIP(hipGetLastError());
+}
+long flow_end_doubles(long n) { return 4 + 2 * ((n + 255) / 256); }
+void launch_flow_end(const TileView& v, const double* rhs, long n, double* y, const int* info, const long long* clock,
+                     double* host, hipStream_t s) {
+  hipLaunchKernelGGL(k_flow_end, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, v, rhs, n, y, info, clock, host);
+  EXA_HIP(hipGetLastError());
 }
 
 }  // namespace exa

@@ -190,6 +190,11 @@ struct ClassLists {
 // outside the band keep the covariance.
 int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s_main, hipStream_t s_aux, bool sync = true,
                const ClassLists* lists = nullptr, int band = 0);
+// Whether the matrix is factored by one dataflow launch.
+bool one_launch(const TileMatrix& A);
+// The inverses of the diagonal tiles, which the triangular solves and the
+// gradient read; tile_potrf forms them, the one-launch evaluation does not.
+void tile_inverses(const TileMatrix& A, CholWorkspace& ws, hipStream_t s);
 // z <- L^-1 z (trans=0) or L^-T z (trans=1) with the factor from tile_potrf.
 void tile_trsv(const TileMatrix& L, const CholWorkspace& ws, double* z, int trans, hipStream_t s);
 // The same with caller-provided scratch: y (mt*ts doubles), tpart
@@ -246,6 +251,12 @@ class Context {
   double loglik(KernelId kid, const double* theta, int metric, double* logdet_out, double* dotp_out, int* info,
                 int band = 0);
   void ensure_partial(long n);
+  // Right-hand side row, clock and result mirror of the one-launch
+  // evaluation, allocated on first use.
+  double* flow_rhs = nullptr;
+  long long* flow_clock = nullptr;
+  double* flow_host = nullptr;  // pinned
+  double wall_rate = 1e8;       // ticks per second of flow_clock
   // C, or std::invalid_argument naming `what` when the context is lean.
   TileMatrix& fp64(const char* what);
 };

@@ -81,10 +81,21 @@ void launch_gen_spacetime(const TileView& v, const SpaceTimeParams& P, long p_of
 // and the columns lie in tile column tile_col.  dinv: 64 x 64 inverses of
 // the diagonal blocks (block j at dinv + 4096 j; identities for the padding
 // blocks [j1, j_pad)).  flags: chol_flow_flags() ints, zero before the first
-// launch and left zero by each.
+// launch and left zero by each.  rhs (whole matrix only): one more block row
+// of 64 x 64 blocks in sequence, solved with the factor (rows r <- r L^-T).
+// clock: receives the wall clock at the start and the end.
 long chol_flow_flags(int mt, int ts);
 void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int j1, int i_end, int j_pad,
-                      double* dinv, int* info, int* flags, hipStream_t s);
+                      double* dinv, int* info, int* flags, hipStream_t s, double* rhs = nullptr,
+                      long long* clock = nullptr);
+// info <- 0, z into the first row of rhs.
+void launch_flow_begin(const double* z, long n, double* rhs, int* info, hipStream_t s);
+// y <- the first row of rhs; host[0] <- info, host[1] <- clock[1] - clock[0],
+// host[4 + 2 b], host[5 + 2 b] <- sums of y^2 and log L_ii over rows
+// [256 b, 256 (b + 1)); flow_end_doubles(n) doubles of pinned host memory.
+long flow_end_doubles(long n);
+void launch_flow_end(const TileView& v, const double* rhs, long n, double* y, const int* info, const long long* clock,
+                     double* host, hipStream_t s);
 // A(m,n) -= sum_{p < np} A(m,k+p) A(n,k+p)^T for n in [col_lo, col_hi],
 // m in [n, mt); np = 1 or 2 (col_lo >= k + np).
 void launch_tile_update(const TileView& v, int k, int np, int col_lo, int col_hi, hipStream_t s);
