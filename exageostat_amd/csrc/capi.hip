@@ -169,16 +169,17 @@ hipStream_t seq_stream(RUNTIME_sequence_t* seq) {
 
 // Scratch of EXAGEOSTAT_dtrsv_Tile_noalloc, the entry point that allocates
 // nothing: the padded right-hand side (kNoAllocRows doubles), the solve's
-// assembly vector (kNoAllocRows), the partial sums of the diagonal-tile
-// products ((kNoAllocTs / 64) * kNoAllocTs) and the completion ticket.
-// 1.13 MB per GPU, held until the process ends.  Host code never passes
+// partial results (trsv_part_doubles(): at most 8 per row, for tiles of 16
+// blocks) and its flags (trsv_flags(): most for tiles of 64).
+// 5.2 MB per GPU, held until the process ends.  Host code never passes
 // `scratch` itself (its host-side name is not a device address): it uses
 // the device address that hipGetSymbolAddress returns for the current
 // device.
 constexpr long kNoAllocRows = 65536;  // mt * ts at most
 constexpr long kNoAllocTs = 1024;
-constexpr long kNoAllocPart = (kNoAllocTs / kNB) * kNoAllocTs;
-constexpr long kNoAllocDoubles = 2 * kNoAllocRows + kNoAllocPart + 32;
+constexpr long kNoAllocPart = 8 * kNoAllocRows;
+constexpr long kNoAllocFlags = 128 * (kNoAllocRows / kNB) + 64;
+constexpr long kNoAllocDoubles = kNoAllocRows + kNoAllocPart + kNoAllocFlags / 2;
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 
 // Device address of `scratch` on the current device, looked up once per
@@ -824,15 +825,16 @@ int EXAGEOSTAT_dtrsv_Tile_noalloc(CHAM_enum trans, CHAM_desc_t* L, double* b) {
                                   "EXAGEOSTAT_dpotrf_Tile");
     double* base = scratch_ptr();
     double* v = base;
-    double* y = base + kNoAllocRows;
-    double* tpart = y + kNoAllocRows;
-    unsigned* ticket = reinterpret_cast<unsigned*>(tpart + kNoAllocPart);
+    double* part = base + kNoAllocRows;
+    int* flags = reinterpret_cast<int*>(part + kNoAllocPart);
+    if (trsv_part_doubles(tm.mt, tm.ts) > kNoAllocPart || trsv_flags(tm.mt) > kNoAllocFlags)
+      throw std::invalid_argument("EXAGEOSTAT_dtrsv_Tile_noalloc: scratch");
     hipStream_t s = rt().s1;
-    // the padding rows of v must be zero; the ticket starts at zero
+    // the padding rows of v must be zero; the flags start at zero
     EXA_HIP(hipMemsetAsync(v, 0, sizeof(double) * padded, s));
-    EXA_HIP(hipMemsetAsync(ticket, 0, sizeof(unsigned), s));
+    EXA_HIP(hipMemsetAsync(flags, 0, sizeof(int) * trsv_flags(tm.mt), s));
     EXA_HIP(hipMemcpyAsync(v, b, sizeof(double) * tm.m, hipMemcpyHostToDevice, s));
-    tile_trsv_scratch(tm, rt().ws, v, trans == ChamTrans ? 1 : 0, s, y, tpart, ticket);
+    tile_trsv_scratch(tm, rt().ws, v, trans == ChamTrans ? 1 : 0, s, part, flags);
     EXA_HIP(hipMemcpyAsync(b, v, sizeof(double) * tm.m, hipMemcpyDeviceToHost, s));
     EXA_HIP(hipStreamSynchronize(s));
     return 0;

@@ -33,6 +33,7 @@
 // scope; a waiting work-group acquires at agent scope before it reads.
 #include "common.hpp"
 #include "besselk.hpp"
+#include "flow.hpp"
 #include "kernels.hpp"
 #include "mfma.hpp"
 
@@ -42,21 +43,6 @@ namespace {
 
 // Counters, one per 64 bytes.
 constexpr int kClaim = 0, kExit = 16, kDiag = 32, kRows = 48;
-
-__device__ __forceinline__ int flag_get(const int* f) {
-  return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Every wave's stores have left the wave; to be called before the barrier
-// that precedes flag_set.
-__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ void flag_set(int* f, int v) {
-  __hip_atomic_store(f, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class T>
-__device__ __forceinline__ void store_through(T* p, T v) {
-  typedef __attribute__((address_space(1))) T gT;
-  __hip_atomic_store((gT*)(uintptr_t)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // x of lane N of each row of 16 lanes, in all lanes of that row.
 template <int N>

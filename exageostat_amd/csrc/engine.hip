@@ -374,43 +374,36 @@ void generate_covariance_tiles(const TileView& v, KernelId kid, const double* th
 
 // --------------------------------------------------------------- Cholesky --
 CholWorkspace::~CholWorkspace() {
-  if (dinv_) (void)hipFree(dinv_);
-  if (xinv_) (void)hipFree(xinv_);
-  if (yvec_) (void)hipFree(yvec_);
-  if (tpart_) (void)hipFree(tpart_);
-  if (ticket_) (void)hipFree(ticket_);
-  if (flags_) (void)hipFree(flags_);
-  if (info_) (void)hipFree(info_);
+  if (base_) (void)hipFree(base_);
   if (h_info_) (void)hipHostFree(h_info_);
   for (auto e : ev_) (void)hipEventDestroy(e);
 }
 
 void CholWorkspace::ensure(int mt, int ts) {
-  if (dinv_ && mt <= mt_ && ts == ts_) return;
-  if (dinv_) (void)hipFree(dinv_);
-  if (xinv_) (void)hipFree(xinv_);
-  if (yvec_) (void)hipFree(yvec_);
-  if (tpart_) (void)hipFree(tpart_);
-  if (flags_) (void)hipFree(flags_);
-  dinv_ = xinv_ = yvec_ = tpart_ = nullptr;
-  flags_ = nullptr;
-  mt_ = mt;
-  ts_ = ts;
-  EXA_HIP(hipMalloc(&dinv_, sizeof(double) * (size_t)mt * (ts / kNB) * 4096));
-  EXA_HIP(hipMalloc(&xinv_, sizeof(double) * (size_t)mt * ts * ts));
-  EXA_HIP(hipMalloc(&yvec_, sizeof(double) * (size_t)mt * ts));
-  EXA_HIP(hipMalloc(&tpart_, sizeof(double) * (size_t)(ts / kNB) * ts));
-  EXA_HIP(hipMalloc(&flags_, sizeof(int) * chol_flow_flags(mt, ts)));
-  EXA_HIP(hipMemset(flags_, 0, sizeof(int) * chol_flow_flags(mt, ts)));
-  if (!ticket_) {
-    EXA_HIP(hipMalloc(&ticket_, sizeof(unsigned)));
-    EXA_HIP(hipMemset(ticket_, 0, sizeof(unsigned)));
-  }
+  if (base_ && mt <= mt_ && ts == ts_) return;
+  if (base_) (void)hipFree(base_);
+  base_ = nullptr;
+  mt_ = ts_ = 0;
+  // One allocation: the inverses, the solves' partials, and the counters and
+  // flags, which start at zero.
+  const size_t n_dinv = (size_t)mt * (ts / kNB) * 4096, n_xinv = (size_t)mt * ts * ts;
+  const size_t n_part = trsv_part_doubles(mt, ts);
+  const size_t n_flags = (chol_flow_flags(mt, ts) + 15) / 16 * 16, n_tflags = trsv_flags(mt) + 16;
+  const size_t zeros = sizeof(int) * (n_flags + n_tflags);
+  EXA_HIP(hipMalloc(&base_, sizeof(double) * (n_dinv + n_xinv + n_part) + zeros));
+  dinv_ = base_;
+  xinv_ = dinv_ + n_dinv;
+  tpart_ = xinv_ + n_xinv;
+  flags_ = reinterpret_cast<int*>(tpart_ + n_part);
+  tflags_ = flags_ + n_flags;
+  info_ = tflags_ + n_tflags - 16;
+  EXA_HIP(hipMemset(flags_, 0, zeros));
   // hipMemset runs on the null stream, which does not order with the
   // non-blocking streams the kernels run on: wait for it here
   EXA_HIP(hipDeviceSynchronize());
-  if (!info_) EXA_HIP(hipMalloc(&info_, sizeof(int)));
   if (!h_info_) EXA_HIP(hipHostMalloc(&h_info_, sizeof(int), hipHostMallocDefault));
+  mt_ = mt;
+  ts_ = ts;
 }
 
 hipEvent_t CholWorkspace::ev(int i) {
@@ -691,28 +684,13 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
 }
 
 void tile_trsv(const TileMatrix& L, const CholWorkspace& ws, double* z, int trans, hipStream_t s) {
-  tile_trsv_scratch(L, ws, z, trans, s, ws.yvec(), ws.tpart(), ws.ticket());
+  tile_trsv_scratch(L, ws, z, trans, s, ws.tpart(), ws.tflags());
 }
 
-void tile_trsv_scratch(const TileMatrix& L, const CholWorkspace& ws, double* z, int trans, hipStream_t s, double* y,
-                       double* tpart, unsigned* ticket) {
-  // Blocked substitution with the inverted diagonal tiles: y_k = X_k z_k
-  // (resp. X_k^T z_k), then the off-diagonal tiles update the remaining
-  // right-hand side; y is assembled in a scratch vector and copied back.
-  TileView v = L.view();
-  const int ts = L.ts;
-  if (!trans) {
-    for (int k = 0; k < L.mt; ++k) {
-      launch_trmv_diag(ws.xinv(k), ts, z + (long)k * ts, y + (long)k * ts, 0, tpart, ticket, s);
-      launch_gemv_panel(v, k, y + (long)k * ts, z, s);
-    }
-  } else {
-    for (int k = L.mt - 1; k >= 0; --k) {
-      launch_trmv_diag(ws.xinv(k), ts, z + (long)k * ts, y + (long)k * ts, 1, tpart, ticket, s);
-      launch_gemv_t_row(v, k, y + (long)k * ts, z, s);
-    }
-  }
-  EXA_HIP(hipMemcpyAsync(z, y, sizeof(double) * (size_t)L.mt * ts, hipMemcpyDeviceToDevice, s));
+void tile_trsv_scratch(const TileMatrix& L, const CholWorkspace& ws, double* z, int trans, hipStream_t s,
+                       double* part, int* flags) {
+  if (L.mt > ws.mt_ || L.ts != ws.ts_) throw std::invalid_argument("the matrix has not been factored");
+  launch_trsv(L.view(), ws.xinv_base(), z, trans, part, flags, s);
 }
 
 double tile_logdet(const TileMatrix& L, double* d_partial, hipStream_t s) {

@@ -129,12 +129,9 @@ class CholWorkspace {
   // Inverse of diagonal tile k (ts x ts, lower), filled by tile_potrf.
   double* xinv(int k) const { return xinv_ + (long)k * ts_ * ts_; }
   double* xinv_base() const { return xinv_; }
-  // Scratch vector of mt*ts doubles for the triangular solves.
-  double* yvec() const { return yvec_; }
-  // Partial sums ((ts/64) * ts doubles) and the zeroed completion ticket of
-  // the diagonal-tile products in the solves.
+  // Partial results and zeroed flags of the triangular solves.
   double* tpart() const { return tpart_; }
-  unsigned* ticket() const { return ticket_; }
+  int* tflags() const { return tflags_; }
   int* info() const { return info_; }      // device
   // Zeroed progress counters of the dataflow factorisation.
   int* flags() const { return flags_; }
@@ -145,11 +142,11 @@ class CholWorkspace {
   const void* factored = nullptr;
 
  private:
+  double* base_ = nullptr;  // the allocation that the following point into
   double* dinv_ = nullptr;
   double* xinv_ = nullptr;
-  double* yvec_ = nullptr;
   double* tpart_ = nullptr;
-  unsigned* ticket_ = nullptr;
+  int* tflags_ = nullptr;
   int* info_ = nullptr;
   int* flags_ = nullptr;
   int* h_info_ = nullptr;
@@ -197,10 +194,10 @@ bool one_launch(const TileMatrix& A);
 void tile_inverses(const TileMatrix& A, CholWorkspace& ws, hipStream_t s);
 // z <- L^-1 z (trans=0) or L^-T z (trans=1) with the factor from tile_potrf.
 void tile_trsv(const TileMatrix& L, const CholWorkspace& ws, double* z, int trans, hipStream_t s);
-// The same with caller-provided scratch: y (mt*ts doubles), tpart
-// ((ts/64)*ts doubles) and ticket (zero on entry; left zero).
-void tile_trsv_scratch(const TileMatrix& L, const CholWorkspace& ws, double* z, int trans, hipStream_t s, double* y,
-                       double* tpart, unsigned* ticket);
+// The same with caller-provided scratch: part (trsv_part_doubles() doubles)
+// and flags (trsv_flags() ints, zero on entry; left zero).
+void tile_trsv_scratch(const TileMatrix& L, const CholWorkspace& ws, double* z, int trans, hipStream_t s,
+                       double* part, int* flags);
 // sum_i log L_ii (deterministic order).
 double tile_logdet(const TileMatrix& L, double* d_partial, hipStream_t s);
 double device_dot(const double* a, const double* b, long n, double* d_partial, hipStream_t s);

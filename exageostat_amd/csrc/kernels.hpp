@@ -104,15 +104,14 @@ void launch_tile_update(const TileView& v, int k, int np, int col_lo, int col_hi
 void launch_trtri_tiles(const TileView& v, const double* dinv, double* xinv, hipStream_t s);
 
 // ---- vectors --------------------------------------------------------------
-// y = X t (trans = 0) or X^T t (trans = 1) for one lower ts x ts tile X;
-// part: (ts/64) * ts doubles of scratch, ticket: a zeroed device counter
-// (left zeroed), both private to the stream.
-void launch_trmv_diag(const double* X, int ts, const double* t, double* y, int trans, double* part,
-                      unsigned* ticket, hipStream_t s);
-// z_m -= L(m,k) y_k for m in (k, mt).
-void launch_gemv_panel(const TileView& v, int k, const double* yk, double* z, hipStream_t s);
-// z_m -= L(k,m)^T y_k for m in [0, k).
-void launch_gemv_t_row(const TileView& v, int k, const double* yk, double* z, hipStream_t s);
+// z <- L^-1 z (trans = 0) or L^-T z (trans = 1) for a tile factor with the
+// inverses xinv of its diagonal tiles; part: trsv_part_doubles() doubles and
+// flags: trsv_flags() zeroed ints (left zeroed) of scratch, both private to
+// the stream.
+long trsv_part_doubles(int mt, int ts);
+long trsv_flags(int mt);
+void launch_trsv(const TileView& v, const double* xinv, double* z, int trans, double* part, int* flags,
+                 hipStream_t s);
 // partial[k] = sum_i log(L_kk[i,i]) over positive pivots of each diagonal tile.
 void launch_logdet(const TileView& v, double* partial, hipStream_t s);
 // partial[b] = sum of z[i]*w[i] over 4096-element blocks.
