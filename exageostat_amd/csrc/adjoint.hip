@@ -72,17 +72,18 @@ void tile_potri_inplace(TileMatrix& A, CholWorkspace& ws, double* P, double* Q, 
   const TileView v = A.view();
   const int mt = A.mt;
   auto rows = [&](int t) { return (double)std::min<long>(A.ts, (long)A.m - (long)t * A.ts); };
+  launch_takahashi_begin(v, ws.xinv_base(), P, s);
   for (int k = mt - 1; k >= 0; --k) {
     const double below = (double)A.m - (double)(k + 1) * A.ts;
     const double rk = rows(k);
     if (k + 1 < mt) {
       profiled("potri_trmm", below * rk * rk, 0.0, s,
-               [&] { launch_takahashi_stage(v, k, ws.xinv(k), P, Q, A.tile(k, k), 0, s); });
+               [&] { launch_takahashi_stage(v, k, P, Q, A.tile(k, k), 0, s); });
       profiled("potri_col", 2.0 * below * below * rk, 0.0, s,
-               [&] { launch_takahashi_stage(v, k, ws.xinv(k), P, Q, A.tile(k, k), 1, s, W, max_split, up, f32); });
+               [&] { launch_takahashi_stage(v, k, P, Q, A.tile(k, k), 1, s, W, max_split, up, f32); });
     }
     profiled("potri_diag", 2.0 * below * rk * rk + rk * rk * rk / 3.0, 0.0, s,
-             [&] { launch_takahashi_stage(v, k, ws.xinv(k), P, Q, A.tile(k, k), 2, s, nullptr, 1, up); });
+             [&] { launch_takahashi_stage(v, k, P, Q, A.tile(k, k), 2, s, nullptr, 1, up); });
   }
   ws.factored = nullptr;
 }

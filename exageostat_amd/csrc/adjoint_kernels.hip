@@ -26,26 +26,63 @@ using C128 = GemmCfg<128, 128, 2, 2, 16>;
 using CT64 = GemmCfg<64, 64, 2, 2, 16>;
 // The FP64 column stage's blocks (gemm_nt_pipe, two work-groups per CU).
 using CP192 = GemmCfg<96, 192, 2, 2, 16>;
+// The trmm and diagonal stages' blocks.
+using CP96 = GemmCfg<96, 96, 2, 2, 16>;
+
+// P_k <- X_kk^T for every tile k: the trmm and diagonal stages of column k
+// read the transpose in their plain operand layout, and P_k is not written
+// before those stages have passed (stage k writes P_j, j > k).
+__global__ void __launch_bounds__(256) k_transpose_tiles(const double* X, double* P, int ts) {
+  __shared__ double blk[64][65];
+  const int q = ts / 64;
+  const long b = blockIdx.x;
+  const long t = b / (q * q);
+  const int rem = (int)(b - t * q * q);
+  const int r0 = (rem % q) * 64, c0 = (rem / q) * 64;
+  const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+  const double* A = X + t * ts * ts + r0 + (long)c0 * ts;
+  double* B = P + t * ts * ts + c0 + (long)r0 * ts;
+  double a[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) a[c] = A[lane + (long)(grp * 16 + c) * ts];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) blk[lane][grp * 16 + c] = a[c];
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) B[lane + (long)(grp * 16 + r) * ts] = blk[grp * 16 + r][lane];
+}
 
 // P_j = L_jk X_kk for j in (k, mt), stored transposed (tile j of P holds
-// P_j^T, column-major), so the two consumers read it row-major.
+// P_j^T, column-major), so the two consumers read it row-major: P_j^T =
+// X_kk^T L_jk^T in plain operands, with X_kk^T in tile k of P.  X_kk^T is
+// upper triangular: a block of its rows starts at its own columns, and the
+// blocks with the longest sums come first in the grid.
+// Few tiles are left in most columns, and one block's chain of ts columns
+// sets the time of a round: 96 x 96 blocks (two work-groups per CU) finish
+// in a quarter of the 242 us that a CU needs for one of 192 x 192 over 960
+// columns (n = 12,000, tiles of 960: 134 us a
+// column against 286).
 template <class C>
-__global__ void __launch_bounds__(C::NT) k_trmm_panel(TileView v, int k, const double* X, double* P) {
-  __shared__ __attribute__((aligned(16))) double lds[C::LDS_DOUBLES];
-  const int qm = v.ts / C::BM, qn = v.ts / C::BN;
-  const long b = blockIdx.x;
-  const int j = k + 1 + (int)(b / (qm * qn));
-  const int rem = (int)(b % (qm * qn));
-  const int bi = rem % qm, bj = rem / qm;
+__global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2))) k_trmm_panel(TileView v, int k, double* P) {
+  __shared__ __attribute__((aligned(16))) double lds[PipeLds<C, 2>::DOUBLES];
+  static_assert(C::BM == C::BN, "square blocks");
+  const int qb = v.ts / C::BM;
+  const long per = (long)(v.mt - k - 1) * qb;
+  const int bi = (int)(blockIdx.x / per);
+  const int rem = (int)(blockIdx.x - bi * per);
+  const int j = k + 1 + rem / qb, bj = rem % qb;
   const long ts = v.ts;
-  // X_kk is lower triangular: rows below bj*BN only.
-  const int k0 = bj * C::BN;
-  const double* A = tile_f64(v, j, k) + bi * C::BM + (long)k0 * ts;
-  const double* B = X + k0 + (long)bj * C::BN * ts;  // B(c, kk) = X[k0 + kk, bj*BN + c]
+  const long k0 = (long)bi * C::BM;
   dx4 acc[C::FM][C::FN];
   zero_acc<C>(acc);
-  gemm_nt_acc<C, true>(acc, A, ts, B, ts, (int)(ts - k0), lds, 1.0);
-  acc_store_t<C>(acc, P + (long)j * ts * ts + bj * C::BN + (long)bi * C::BM * ts, ts);
+  gemm_nt_pipe<C, 2>(
+      acc, 1,
+      [&](int, const double*& A, const double*& B) {
+        A = P + (long)k * ts * ts + bi * C::BM + k0 * ts;
+        B = tile_f64(v, j, k) + bj * C::BN + k0 * ts;
+      },
+      ts, (int)(ts - k0), lds);
+  pipe_put<C>(acc, P + (long)j * ts * ts + bi * C::BM + (long)bj * C::BN * ts, ts);
 }
 
 // Z_mk = - sum_{j>k} Z(m,j) P_j for m in (k, mt).  With nsplit > 1 the
@@ -158,12 +195,22 @@ __global__ void __launch_bounds__(256) k_sum_slabs(TileView v, int k, const doub
   const int r0 = (rem % q) * 64, c0 = (rem / q) * 64;
   const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
   double* Z = tile_f64(v, k + 1 + (int)t, k);
-  for (int c = grp; c < 64; c += 4) {
-    const long e = (long)(r0 + lane) + (long)(c0 + c) * ts;
-    double acc = 0.0;
-    for (int sp = 0; sp < nsplit; ++sp) acc += W[((long)sp * below + t) * len + e];
-    Z[e] = acc;
-    blk[lane][c] = acc;
+  // all loads of a slab in flight at once: the launch is as long as one
+  // work-group's latency where few tiles are left (64-row tiles, four slabs:
+  // 5.9 us against 18.3 with the loads one after another; n = 12,000: 42
+  // against 66)
+  double acc[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) acc[c] = 0.0;
+  for (int sp = 0; sp < nsplit; ++sp) {
+    const double* w = W + ((long)sp * below + t) * len + r0 + lane + (long)(c0 + grp * 16) * ts;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) acc[c] += w[(long)c * ts];
+  }
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    Z[r0 + lane + (long)(c0 + grp * 16 + c) * ts] = acc[c];
+    blk[lane][grp * 16 + c] = acc[c];
   }
   if (!U.ptr) return;
   __syncthreads();
@@ -171,43 +218,77 @@ __global__ void __launch_bounds__(256) k_sum_slabs(TileView v, int k, const doub
   for (int r = grp; r < 64; r += 4) Ut[(long)(c0 + lane) + (long)(r0 + r) * ts] = blk[r][lane];
 }
 
-// Split-k terms of Z_kk: Q_0 = X_kk^T X_kk, Q_i = -Z_{k+i,k}^T P_{k+i}.
-template <class C>
-__global__ void __launch_bounds__(C::NT) k_takahashi_diag(TileView v, int k, const double* X, const double* P,
-                                                          double* Q, TileView U) {
-  __shared__ __attribute__((aligned(16))) double lds[C::LDS_DOUBLES];
-  const int qm = v.ts / C::BM, qn = v.ts / C::BN;
-  const long b = blockIdx.x;
-  const int i = (int)(b / (qm * qn));
-  const int rem = (int)(b % (qm * qn));
-  const int bi = rem % qm, bj = rem / qm;
+// Split-k terms of Z_kk: Q_0 = X_kk^T X_kk, Q_i = -Z_{k+i,k}^T P_{k+i}, the
+// blocks of the lower triangle only.  X_kk^T is tile k of P and X_kk^T(r, kk)
+// = 0 for kk < r, so that sum starts at the block's rows.  Blocks as in
+// k_trmm_panel for the same reason (n = 12,000: 143 us a column
+// against 360 for all blocks of 192 x 192); without U
+// (Z_{k+i,k} read transposed) the register-staged core and its blocks.
+template <class C, bool HAS_U>
+__global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(HAS_U ? 2 : 1)))
+    k_takahashi_diag(TileView v, int k, const double* P, double* Q, TileView U) {
+  __shared__ __attribute__((aligned(16))) double lds[HAS_U ? PipeLds<C, 2>::DOUBLES : C::LDS_DOUBLES];
+  static_assert(C::BM == C::BN, "square blocks");
+  const int qb = v.ts / C::BM;
+  const int per = qb * (qb + 1) / 2;
+  const int i = (int)(blockIdx.x / per);
+  int bi, bj;
+  tri_decode(blockIdx.x - (long)i * per, bi, bj);
   const long ts = v.ts;
+  const int j = k + i;
+  const long k0 = i == 0 ? (long)bi * C::BM : 0;
+  const double* Pb = P + (long)j * ts * ts + bj * C::BN + k0 * ts;
+  double* out = Q + (long)i * ts * ts + bi * C::BM + (long)bj * C::BN * ts;
   dx4 acc[C::FM][C::FN];
   zero_acc<C>(acc);
-  if (i == 0) {
-    // X^T X: X(kk, r) = 0 for kk < r, so the sum starts at the larger block.
-    const int k0 = (bi * C::BM > bj * C::BN ? bi * C::BM : bj * C::BN);
-    gemm_nt_acc<C, true, double, double, true>(acc, X + k0 + (long)bi * C::BM * ts, ts,
-                                               X + k0 + (long)bj * C::BN * ts, ts, (int)(ts - k0), lds, 1.0);
-  } else if (U.ptr) {
-    const int j = k + i;
-    gemm_nt_acc<C>(acc, tile_f64(U, j, k) + bi * C::BM, ts, P + (long)j * ts * ts + bj * C::BN, ts, (int)ts, lds,
-                   -1.0);
+  if constexpr (HAS_U) {
+    const double* Ab = (i == 0 ? P + (long)k * ts * ts : tile_f64(U, j, k)) + bi * C::BM + k0 * ts;
+    gemm_nt_pipe<C, 2>(
+        acc, 1,
+        [&](int, const double*& A, const double*& B) {
+          A = Ab;
+          B = Pb;
+        },
+        ts, (int)(ts - k0), lds);
+    if (i == 0) pipe_put<C>(acc, out, ts);
+    else pipe_put_neg<C>(acc, out, ts);
   } else {
-    const int j = k + i;
-    gemm_nt_acc<C, false, double, double, true>(acc, tile_f64(v, j, k) + (long)bi * C::BM * ts, ts,
-                                                P + (long)j * ts * ts + bj * C::BN, ts, (int)ts, lds, -1.0);
+    if (i == 0)
+      gemm_nt_acc<C>(acc, P + (long)k * ts * ts + bi * C::BM + k0 * ts, ts, Pb, ts, (int)(ts - k0), lds, 1.0);
+    else
+      gemm_nt_acc<C, false, double, double, true>(acc, tile_f64(v, j, k) + (long)bi * C::BM * ts, ts, Pb, ts, (int)ts,
+                                                  lds, -1.0);
+    acc_update<C>(acc, out, ts, 0.0);
   }
-  acc_update<C>(acc, Q + (long)i * ts * ts + bi * C::BM + (long)bj * C::BN * ts, ts, 0.0);
 }
 
-// out[e] = sum_{i < cnt} Q[i*len + e] (fixed order), e < len.
-__global__ void k_sum_tiles(const double* Q, int cnt, long len, double* out) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= len) return;
-  double s = 0.0;
-  for (int i = 0; i < cnt; ++i) s += Q[(long)i * len + e];
-  out[e] = s;
+// Z_kk = sum_{i < cnt} Q_i (fixed order) from the sums' lower triangles, in
+// both triangles of out; one work-group per 64 x 64 block of the lower one.
+__global__ void __launch_bounds__(256) k_sum_diag(const double* Q, int cnt, int ts, double* out) {
+  __shared__ double blk[64][65];
+  int rb, cb;
+  tri_decode(blockIdx.x, rb, cb);
+  const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+  const long len = (long)ts * ts;
+  const double* q = Q + rb * 64 + lane + (long)(cb * 64 + grp * 16) * ts;
+  double acc[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) acc[c] = 0.0;
+#pragma unroll 2
+  for (int i = 0; i < cnt; ++i, q += len) {
+#pragma unroll
+    for (int c = 0; c < 16; ++c) acc[c] += q[(long)c * ts];
+  }
+#pragma unroll
+  for (int c = 0; c < 16; ++c) blk[lane][grp * 16 + c] = acc[c];
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    const int col = grp * 16 + c;
+    const double t = blk[col][lane];  // the entry across the diagonal
+    out[rb * 64 + lane + (long)(cb * 64 + col) * ts] = rb == cb && lane < col ? t : acc[c];
+    if (rb > cb) out[cb * 64 + lane + (long)(rb * 64 + col) * ts] = t;
+  }
 }
 
 // Number of j ranges of the column stage: the split (at most 4, and at most
@@ -243,13 +324,16 @@ static int takahashi_splits(const TileView& v, int k, int max_split, int* slots_
   return best;
 }
 
-template <class C, class CP>
-static void takahashi_cfg(const TileView& v, int k, const double* X, double* P, double* Q, double* W, int max_split,
+// C: blocks of the FP32 column stage and of the stages without U; CP: of the
+// FP64 column stage; CD: of the trmm and diagonal stages.
+template <class C, class CP, class CD>
+static void takahashi_cfg(const TileView& v, int k, double* P, double* Q, double* W, int max_split,
                           const TileView& U, int stage, hipStream_t s, bool f32) {
   const long per = (long)(v.ts / C::BM) * (v.ts / C::BN);
   const long below = v.mt - k - 1;
+  const int qd = v.ts / CD::BM, qc = v.ts / C::BM;
   if (stage == 0 && below > 0)
-    hipLaunchKernelGGL(k_trmm_panel<C>, dim3((unsigned)(below * per)), dim3(C::NT), 0, s, v, k, X, P);
+    hipLaunchKernelGGL(k_trmm_panel<CD>, dim3((unsigned)(below * qd * qd)), dim3(CD::NT), 0, s, v, k, P);
   if (stage == 1 && below > 0) {
     int slots = 0;
     const bool f32u = f32 && U.ptr;
@@ -281,23 +365,34 @@ static void takahashi_cfg(const TileView& v, int k, const double* X, double* P, 
                          U);
     }
   }
-  if (stage == 2)
-    hipLaunchKernelGGL(k_takahashi_diag<C>, dim3((unsigned)((below + 1) * per)), dim3(C::NT), 0, s, v, k, X,
-                       (const double*)P, Q, U);
+  if (stage == 2) {
+    if (U.ptr)
+      hipLaunchKernelGGL((k_takahashi_diag<CD, true>), dim3((unsigned)((below + 1) * (qd * (qd + 1) / 2))), dim3(CD::NT), 0, s,
+                         v, k, (const double*)P, Q, U);
+    else
+      hipLaunchKernelGGL((k_takahashi_diag<C, false>), dim3((unsigned)((below + 1) * (qc * (qc + 1) / 2))), dim3(C::NT), 0, s,
+                         v, k, (const double*)P, Q, U);
+  }
   EXA_HIP(hipGetLastError());
 }
 
-void launch_takahashi_stage(const TileView& v, int k, const double* X, double* P, double* Q, double* Zkk,
-                            int stage, hipStream_t s, double* W, int max_split, const TileView* U, bool f32) {
+void launch_takahashi_begin(const TileView& v, const double* xinv, double* P, hipStream_t s) {
+  const long q = v.ts / 64;
+  hipLaunchKernelGGL(k_transpose_tiles, dim3((unsigned)(v.mt * q * q)), dim3(256), 0, s, xinv, P, v.ts);
+  EXA_HIP(hipGetLastError());
+}
+
+void launch_takahashi_stage(const TileView& v, int k, double* P, double* Q, double* Zkk, int stage, hipStream_t s,
+                            double* W, int max_split, const TileView* U, bool f32) {
   TileView u{};
   if (U) u = *U;
-  if (v.ts % 192 == 0) takahashi_cfg<C192, CP192>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
-  else if (v.ts % 128 == 0) takahashi_cfg<C128, C128>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
-  else takahashi_cfg<CT64, CT64>(v, k, X, P, Q, W, max_split, u, stage, s, f32);
+  if (v.ts % 192 == 0) takahashi_cfg<C192, CP192, CP96>(v, k, P, Q, W, max_split, u, stage, s, f32);
+  else if (v.ts % 128 == 0) takahashi_cfg<C128, C128, CT64>(v, k, P, Q, W, max_split, u, stage, s, f32);
+  else takahashi_cfg<CT64, CT64, CT64>(v, k, P, Q, W, max_split, u, stage, s, f32);
   if (stage == 2) {
-    const long len = (long)v.ts * v.ts;
-    hipLaunchKernelGGL(k_sum_tiles, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, s, (const double*)Q,
-                       v.mt - k, len, Zkk);
+    const int q = v.ts / 64;
+    hipLaunchKernelGGL(k_sum_diag, dim3((unsigned)(q * (q + 1) / 2)), dim3(256), 0, s, (const double*)Q, v.mt - k, v.ts,
+                       Zkk);
     EXA_HIP(hipGetLastError());
   }
 }

@@ -176,16 +176,16 @@ struct MaternGradParams {
 };
 // One stage of tile column k of the Takahashi sweep Z = Sigma^-1 over the
 // factor in v (0: P_j = L_jk X_kk; 1: Z_mk for m > k; 2: Z_kk into Zkk,
-// with Q as split-k scratch of mt tiles).  X = L_kk^-1, P: mt tiles.
+// with Q as split-k scratch of mt tiles).  P: mt tiles, first filled by
+// launch_takahashi_begin with the transposed inverses of the diagonal tiles.
 // W (may be null): slabs for splitting stage 1's sum over j into up to
 // max_split ranges, max_split * (mt - 1) tiles.  U (may be null): a lower
 // tile matrix of v's geometry that receives Z_mk^T in tile (m, k), so that
 // the later stages read no transposed operands.  f32 (with U): stage 1 on
 // the FP32 matrix cores (operands rounded to FP32, FP32 sums).
-void launch_takahashi_stage(const TileView& v, int k, const double* X, double* P, double* Q, double* Zkk,
-                            int stage, hipStream_t s, double* W = nullptr, int max_split = 1,
-                            const TileView* U = nullptr,
-                            bool f32 = false);
+void launch_takahashi_begin(const TileView& v, const double* xinv, double* P, hipStream_t s);
+void launch_takahashi_stage(const TileView& v, int k, double* P, double* Q, double* Zkk, int stage, hipStream_t s,
+                            double* W = nullptr, int max_split = 1, const TileView* U = nullptr, bool f32 = false);
 struct BivariateGradParams {
   const double* x;
   const double* y;

@@ -394,6 +394,18 @@ __device__ __forceinline__ void pipe_sub(const dx4 (&acc)[C::FM][C::FN], double*
   }
 }
 
+// C = acc.
+template <class C>
+__device__ __forceinline__ void pipe_put(const dx4 (&acc)[C::FM][C::FN], double* Cp, long ldc) {
+  auto* G = pipe_base<C>(Cp, ldc);
+#pragma unroll
+  for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int i = 0; i < C::FM; ++i) G[i * 16 + (long)(j * 16 + 4 * v) * ldc] = acc[i][j][v];
+}
+
 // C = -acc.
 template <class C>
 __device__ __forceinline__ void pipe_put_neg(const dx4 (&acc)[C::FM][C::FN], double* Cp, long ldc) {
