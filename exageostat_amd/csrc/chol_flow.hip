@@ -43,12 +43,25 @@ namespace {
 
 // Counters, one per 64 bytes.
 constexpr int kClaim = 0, kExit = 16, kDiag = 32, kRows = 48;
+// What a diagonal block's inverse holds before it is written: a signalling
+// NaN, which no arithmetic result is.
+constexpr long long kUnset = 0x7ff4dead00000001;
 
 // x of lane N of each row of 16 lanes, in all lanes of that row.
 template <int N>
 __device__ __forceinline__ double row_lane(double x) {
   return __longlong_as_double(
       __builtin_amdgcn_update_dpp(0L, (long)__double_as_longlong(x), 0x150 + N, 0xf, 0xf, true));
+}
+
+// y += (x of lane N of each row of 16 lanes) * z, the broadcast inside the
+// multiply-add (the compiler makes a move of its own of it: three
+// instructions per pair of updates instead of two).  x must not come from
+// one of the two preceding vector instructions: panel_columns waits before
+// it reads the pivot, on which z depends.
+template <int N>
+__device__ __forceinline__ void fma_row_lane(double& y, double x, double z) {
+  asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(y) : "v"(x), "v"(z), "n"(N));
 }
 
 // 1/y for normal y: the hardware estimate (relative error 4.7e-8 measured)
@@ -80,15 +93,17 @@ __device__ __forceinline__ void panel_columns(double (&d)[16], double (&a)[16], 
 template <int C, int C2>
 __device__ __forceinline__ void panel_update(double (&d)[16], double (&a)[16], double nd, double na) {
   if constexpr (C2 < 16) {
-    const double s = row_lane<C2>(d[C]);
-    d[C2] = fma(s, nd, d[C2]);
-    a[C2] = fma(s, na, a[C2]);
+    fma_row_lane<C2>(d[C2], d[C], nd);
+    fma_row_lane<C2>(a[C2], d[C], na);
     panel_update<C, C2 + 1>(d, a, nd, na);
   }
 }
 template <int C>
 __device__ __forceinline__ void panel_columns(double (&d)[16], double (&a)[16], double& own, int l16) {
   if constexpr (C < 16) {
+    // a DPP operand needs two wait states after its write, which the
+    // compiler does not see inside the assembly of fma_row_lane
+    asm("s_nop 1" : "+v"(d[C]));
     const double piv = row_lane<C>(d[C]);
     own = l16 == C ? piv : own;
     const double r = recip3(piv);
@@ -225,9 +240,16 @@ __device__ __forceinline__ int wait_rows(const FlowArgs& a, int r0, int r1, int 
   return got;
 }
 
+// T tasks that are not next poll less often: all of them poll one counter
+// (n = 1,600: 437 -> 407 us).
 __device__ __forceinline__ void wait_diag(const FlowArgs& a, int need) {
   if (threadIdx.x == 0) {
-    while (flag_get(a.flags + kDiag) < need) __builtin_amdgcn_s_sleep(1);
+    for (;;) {
+      const int got = flag_get(a.flags + kDiag);
+      if (got >= need) break;
+      if (got + 1 < need) __builtin_amdgcn_s_sleep(64);
+      else __builtin_amdgcn_s_sleep(1);
+    }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
@@ -248,7 +270,33 @@ __device__ __forceinline__ void load_inverse(const double* src, double* lds, int
   }
 }
 
-// x = t inv^T for the wave's 16 rows: t and x are 16 x 64, four fragments of
+// The same from an inverse that is being written: read until no element is
+// the unset value, then into LDS: one way through memory where the counter
+// takes three (data written, counter set, data read).  Only the next D task
+// reads like this; the counter is looked at beside it, so the loop ends in
+// any case.
+__device__ __forceinline__ void fetch_inverse(const FlowArgs& a, int j, double* lds, int tid) {
+  const double* src = a.dinv + (long)j * 4096 + (tid & 15) + (tid >> 4) * 64;
+  double v[10];
+  for (int last = 0;;) {
+#pragma unroll
+    for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+      for (int bj = 0; bj <= bi; ++bj) v[bi * (bi + 1) / 2 + bj] = load_through(src + 16 * bi + 16 * bj * 64);
+    bool unset = false;
+#pragma unroll
+    for (int t = 0; t < 10; ++t) unset |= __double_as_longlong(v[t]) == kUnset;
+    if (!unset || last) break;
+    last = flag_get(a.flags + kDiag) > j - a.j0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  }
+  __syncthreads();  // the LDS may still be read
+#pragma unroll
+  for (int t = 0; t < 10; ++t) lds[t * 256 + tid] = v[t];
+  __syncthreads();
+}
+
+// x = -t inv^T for the wave's 16 rows: t and x are 16 x 64, four fragments of
 // lane l, element v at row l%16, column 16 f + l/16 + 4 v.  That is also the
 // layout in which the MFMA takes its left operand, so t feeds it as is.
 __device__ __forceinline__ void times_inverse(const dx4 (&t)[4], dx4 (&x)[4], const double* inv, int lane) {
@@ -258,7 +306,7 @@ __device__ __forceinline__ void times_inverse(const dx4 (&t)[4], dx4 (&x)[4], co
 #pragma unroll
     for (int g = 0; g <= f; ++g)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[f] = mfma_f64(inv[blk16(f, g) + e * 64 + lane], t[g][e], x[f]);
+      for (int e = 0; e < 4; ++e) x[f] = mfma_f64(inv[blk16(f, g) + e * 64 + lane], -t[g][e], x[f]);
   }
 }
 
@@ -408,15 +456,16 @@ __device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], d
 typedef __attribute__((address_space(1))) double gdouble;
 typedef __attribute__((address_space(1))) float gfloat;
 
-// t = C - acc for the wave's 16 rows of a 64 x 64 block.
+// acc = -C for the wave's 16 rows of a 64 x 64 block: the products are added
+// to it, so that nothing is left to read when the last of them is done.
 template <class TA>
-__device__ __forceinline__ void block_minus(const char* blk, long ts, int wave, int lane, dx4 (&acc)[4]) {
+__device__ __forceinline__ void block_neg(const char* blk, long ts, int wave, int lane, dx4 (&acc)[4]) {
   typedef __attribute__((address_space(1))) const TA gT;
   gT* G = (gT*)(uintptr_t)blk + 16 * wave + (lane & 15) + (long)(lane >> 4) * ts;
 #pragma unroll
   for (int f = 0; f < 4; ++f)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) acc[f][v] = (double)G[(long)(16 * f + 4 * v) * ts] - acc[f][v];
+    for (int v = 0; v < 4; ++v) acc[f][v] = -(double)G[(long)(16 * f + 4 * v) * ts];
 }
 
 template <class TA>
@@ -439,11 +488,12 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
 #pragma unroll
   for (int p = 0; p < R; ++p) ra[p] = row_of(a, i0 + (p < nr ? p : 0));
   const Row rj = row_of(a, j);
+  // The row that D_{j+2} waits for goes ahead of the group's others.  Its
+  // counter is then D_{j+2}'s: it is not stored again with theirs.
+  const bool early = i0 == j + 2 && nr > 1;
   dx4 acc[R][4], none[3];
 #pragma unroll
-  for (int p = 0; p < R; ++p)
-#pragma unroll
-    for (int f = 0; f < 4; ++f) acc[p][f] = dx4{0.0, 0.0, 0.0, 0.0};
+  for (int p = 0; p < R; ++p) block_neg<TA>(block_ptr(a, ra[p], j, (int)sizeof(TA)), ts, wave, lane, acc[p]);
   int l = a.j0;
   while (l < j) {
     int upto = a.j0 + wait_rows(a, j, i0, i0 + nr - 1, i0 + (nr > 1 ? 1 : 0), l - a.j0, sh);
@@ -451,8 +501,6 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
     flow_gemm<R, TA, false>(a, acc, none, ra, rj, l, upto, lds);
     l = upto;
   }
-#pragma unroll
-  for (int p = 0; p < R; ++p) block_minus<TA>(block_ptr(a, ra[p], j, (int)sizeof(TA)), ts, wave, lane, acc[p]);
   wait_diag(a, j - a.j0 + 1);  // its barrier also ends the reads of the ring
   load_inverse(a.dinv + (long)j * 4096, lds, wave, lane);
   wait_vmcnt<0>();
@@ -464,10 +512,15 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
       times_inverse(acc[p], x, lds, lane);
       block_store<TA>(block_ptr(a, ra[p], j, (int)sizeof(TA)), ts, wave, lane, x);
     }
+    if (p == 0 && early) {
+      stores_done();
+      __syncthreads();
+      if (tid == 0) flag_set(a.flags + kRows + 16 * (i0 - a.j0), j - a.j0 + 1);
+    }
   }
   stores_done();
   __syncthreads();
-  if (tid < nr) flag_set(a.flags + kRows + 16 * (i0 + tid - a.j0), j - a.j0 + 1);
+  if (tid < nr && !(early && tid == 0)) flag_set(a.flags + kRows + 16 * (i0 + tid - a.j0), j - a.j0 + 1);
 }
 
 // The T task of the right-hand sides' row.
@@ -478,8 +531,8 @@ __device__ __forceinline__ void task_rhs(const FlowArgs& a, int j, double* lds, 
   const Row rj = row_of(a, j);
   const Row none_row[1] = {rj};
   dx4 acc[1][4], none[3];
-#pragma unroll
-  for (int f = 0; f < 4; ++f) acc[0][f] = dx4{0.0, 0.0, 0.0, 0.0};
+  char* blk = reinterpret_cast<char*>(a.rhs + (long)j * 4096);
+  block_neg<double>(blk, kNB, wave, lane, acc[0]);
   int l = a.j0;
   while (l < j) {
     int upto = a.j0 + wait_rows(a, j, a.i_end, j, a.i_end, l - a.j0, sh);
@@ -487,8 +540,6 @@ __device__ __forceinline__ void task_rhs(const FlowArgs& a, int j, double* lds, 
     flow_gemm<1, double, false, true>(a, acc, none, none_row, rj, l, upto, lds);
     l = upto;
   }
-  char* blk = reinterpret_cast<char*>(a.rhs + (long)j * 4096);
-  block_minus<double>(blk, kNB, wave, lane, acc[0]);
   wait_diag(a, j - a.j0 + 1);
   load_inverse(a.dinv + (long)j * 4096, lds, wave, lane);
   wait_vmcnt<0>();
@@ -524,12 +575,17 @@ __device__ __forceinline__ void inverse_sum(const double* Ls, const double* Xs, 
 #pragma unroll
   for (int e = 0; e < 4; ++e) y = mfma_f64(A[e * 64], B[e * 4], y);
 }
-// X(p, b) = -X(p, p) y
-__device__ __forceinline__ void inverse_put(double* Xs, const dx4& y, int p, int b, int lane) {
+// X(p, b) = -X(p, p) y, in the layout of a 16 x 16 block (element e of lane
+// l at 64 e + l).
+__device__ __forceinline__ dx4 inverse_of(const double* Xs, const dx4& y, int p, int lane) {
   const double* D = Xs + blk16(p, p) + lane;
   dx4 x = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int e = 0; e < 4; ++e) x = mfma_f64(-y[e], D[e * 64], x);
+  return x;
+}
+__device__ __forceinline__ void inverse_put(double* Xs, const dx4& y, int p, int b, int lane) {
+  const dx4 x = inverse_of(Xs, y, p, lane);
   double* dst = Xs + blk16(p, b) + lane;
 #pragma unroll
   for (int e = 0; e < 4; ++e) dst[e * 64] = x[e];
@@ -572,6 +628,12 @@ __device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, doub
 // waves 1 .. 3 bring the blocks that the next panels need up to date and
 // build the inverse; block row bi of S and of the inverse's sums stays with
 // wave bi.
+// Measured per block column (n = 1,600): 14.3 us, of which 9.0 are the four
+// panels and what lies between them, 1.7 X, 1.2 the first fragments and the
+// stores of X, 0.6 the last row of the inverse, 1.7 its way into the next
+// task's LDS; 17.0 before the hand-over read the inverse itself
+// (fetch_inverse), X was published ahead of the panels, the sums began with
+// the block they are subtracted from, and the waiting T tasks polled less.
 __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds, int* sh) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -582,15 +644,21 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
   __builtin_amdgcn_s_setprio(2);
   double* Ls = lds + kLs;
   double* Xs = lds + kXs;
-  dx4 acc[1][4], dacc[3], cd[3];
-#pragma unroll
-  for (int f = 0; f < 4; ++f) acc[0][f] = dx4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int t = 0; t < 3; ++t) dacc[t] = dx4{0.0, 0.0, 0.0, 0.0};
+  dx4 acc[1][4], dacc[3];
   char* cjj = block_ptr(a, rj, j, 8);
   const bool chained = j > a.j0;
   char* cp = nullptr;
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    int bi, bj;
+    diag_frag(wave, t < nd ? t : 0, bi, bj);
+    gdouble* G = (gdouble*)(uintptr_t)cjj + 16 * bi + (lane & 15) + (long)(16 * bj + (lane >> 4)) * ts;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) dacc[t][v] = -G[(long)(4 * v) * ts];
+  }
   if (chained) {
+    cp = block_ptr(a, rj, j - 1, 8);
+    block_neg<double>(cp, ts, wave, lane, acc[0]);
     const Row rp[1] = {row_of(a, j - 1)};
     int l = a.j0;
     while (l < j - 1) {
@@ -599,17 +667,6 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
       flow_gemm<1, double, true>(a, acc, dacc, rp, rj, l, upto, lds);
       l = upto;
     }
-    cp = block_ptr(a, rj, j - 1, 8);
-    block_minus<double>(cp, ts, wave, lane, acc[0]);
-  }
-  // the diagonal block, ahead of the wait
-#pragma unroll
-  for (int t = 0; t < 3; ++t) {
-    int bi, bj;
-    diag_frag(wave, t < nd ? t : 0, bi, bj);
-    gdouble* G = (gdouble*)(uintptr_t)cjj + 16 * bi + (lane & 15) + (long)(16 * bj + (lane >> 4)) * ts;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) cd[t][v] = G[(long)(4 * v) * ts];
   }
   // S's fragment t: minus X X^T when there is one, into LDS
   auto s_frag = [&](int t) {
@@ -622,13 +679,10 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
       for (int e = 0; e < 16; ++e) dacc[t] = mfma_f64(Y[e * 64], X[e * 64], dacc[t]);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) Ls[blk16(bi, bj) + v * 64 + lane] = cd[t][v] - dacc[t][v];
+    for (int v = 0; v < 4; ++v) Ls[blk16(bi, bj) + v * 64 + lane] = -dacc[t][v];
   };
   if (chained) {
-    wait_diag(a, j - a.j0);
-    load_inverse(a.dinv + (long)(j - 1) * 4096, Xs, wave, lane);
-    wait_vmcnt<0>();
-    __syncthreads();
+    fetch_inverse(a, j - 1, Xs, tid);
     dx4 x[4];
     times_inverse(acc[0], x, Xs, lane);
     // X as sixteen 16 x 16 blocks (row block w, column block f), for X X^T
@@ -640,16 +694,17 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
   }
   __syncthreads();
   s_frag(0);
+  stores_done();
   __syncthreads();
+  // X is out: D_{j+1} and the T tasks of its column wait for it
+  if (chained && tid == 64) flag_set(a.flags + kRows + 16 * (j - a.j0), j - a.j0);
   if (wave == 0) {
     diag_panel(a, j, 0, Ls, Xs, lane);
   } else {
     s_frag(1);
     s_frag(2);
   }
-  stores_done();
   __syncthreads();
-  if (chained && tid == 64) flag_set(a.flags + kRows + 16 * (j - a.j0), j - a.j0);
   if (wave > 0) diag_update(Ls, wave, 1, 0, lane);
   __syncthreads();
   dx4 y = {0.0, 0.0, 0.0, 0.0};
@@ -676,20 +731,25 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
       }
     }
     __syncthreads();
+    if (p == 3) break;
     if (wave > p) diag_update(Ls, wave, p + 1, p, lane);
-    if (p == 3 && wave > 0) {
-      inverse_sum(Ls, Xs, y, 3, 2, wave - 1, lane);
-      inverse_put(Xs, y, 3, wave - 1, lane);
-    }
     __syncthreads();
   }
-  // the inverse, then the counter that every T task of this column waits for
+  // the inverse, then the counter that every T task of this column waits
+  // for; the last block row straight from the registers of waves 1 .. 3
   double* dinv = a.dinv + (long)j * 4096;
+  if (wave > 0) {
+    inverse_sum(Ls, Xs, y, 3, 2, wave - 1, lane);
+    const dx4 x = inverse_of(Xs, y, 3, lane);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      store_through(dinv + 48 + (lane & 15) + (16 * (wave - 1) + 4 * e + (lane >> 4)) * 64, x[e]);
+  }
   const int r = tid & 15, c = tid >> 4;
 #pragma unroll
   for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
-    for (int bj = 0; bj <= bi; ++bj)
+    for (int bj = bi == 3 ? 3 : 0; bj <= bi; ++bj)
       store_through(dinv + 16 * bi + r + (16 * bj + c) * 64, Xs[blk16(bi, bj) + tid]);
   stores_done();
   __syncthreads();
@@ -813,13 +873,20 @@ void launch_flow(const FlowArgs& a, hipStream_t s) {
   EXA_HIP(hipGetLastError());
 }
 
-// Before a factorisation with a right-hand side: info = 0 and z into the
-// first row of the right-hand sides' blocks (zero beyond it since their
+// Before a factorisation: info = 0 and the inverses unset; with a right-hand
+// side also z into the first row of its blocks (zero beyond it since their
 // allocation: the rows never mix).
-__global__ void __launch_bounds__(256) k_flow_begin(const double* z, long n, double* rhs, int* info) {
+__global__ void __launch_bounds__(256) k_flow_begin(const double* z, long n, double* rhs, double* dinv, long nd,
+                                                    int* info) {
   const long c = (long)blockIdx.x * 256 + threadIdx.x;
   if (c == 0) *info = 0;
   if (c < n) rhs[c * kNB] = z[c];
+  for (long e = c; e < nd; e += (long)gridDim.x * 256) reinterpret_cast<long long*>(dinv)[e] = kUnset;
+}
+__global__ void __launch_bounds__(256) k_flow_reset(double* dinv, long nd, int* info) {
+  const long c = (long)blockIdx.x * 256 + threadIdx.x;
+  if (c == 0) *info = 0;
+  for (long e = c; e < nd; e += (long)gridDim.x * 256) reinterpret_cast<long long*>(dinv)[e] = kUnset;
 }
 
 // After it: y = L^-1 z into a vector, and per work-group the sums of y^2 and
@@ -887,8 +954,12 @@ void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int
   else launch_flow<3, false>(a, s);
 }
 
-void launch_flow_begin(const double* z, long n, double* rhs, int* info, hipStream_t s) {
-  hipLaunchKernelGGL(k_flow_begin, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, z, n, rhs, info);
+void launch_flow_begin(const double* z, long n, double* rhs, double* dinv, long nd, int* info, hipStream_t s) {
+  hipLaunchKernelGGL(k_flow_begin, dim3((unsigned)(nd / 2048 + (n + 255) / 256)), dim3(256), 0, s, z, n, rhs, dinv, nd, info);
+  EXA_HIP(hipGetLastError());
+}
+void launch_flow_reset(double* dinv, long nd, int* info, hipStream_t s) {
+  hipLaunchKernelGGL(k_flow_reset, dim3((unsigned)(nd / 2048 + 1)), dim3(256), 0, s, dinv, nd, info);
   EXA_HIP(hipGetLastError());
 }
 long flow_end_doubles(long n) { return 4 + 2 * ((n + 255) / 256); }

@@ -503,11 +503,11 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
   auto col_end = [&](int k) { return band > 0 ? std::min(mt - 1, k + band - 1) : mt - 1; };
   ws.ensure(mt, ts);
   int* d_info = ws.info();
-  EXA_HIP(hipMemsetAsync(d_info, 0, sizeof(int), s1));
   TileView v = A.view();
   auto rows = [&](int t) { return (double)std::min<long>(ts, (long)A.m - (long)t * ts); };
   const int q = ts / kNB;
   const int nb = (A.m + kNB - 1) / kNB;  // block rows that hold logical rows; the others stay the identity
+  launch_flow_reset(ws.dinv_base(), (long)nb * 4096, d_info, s1);
   // Tile columns >= k0 in one dataflow launch.
   auto factor_rest = [&](int k0) {
     const double n0 = (double)A.m - (double)k0 * ts;
@@ -574,7 +574,7 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
   // with that panel on s1.
   // The FP64 factor's last kFlowBlocks block columns go into one dataflow
   // launch: its left-looking tasks reach 46-54 TFLOP/s against 60-70 of the
-  // trailing update, but its chain costs 17 us per 64 columns where the tile
+  // trailing update, but its chain costs 14 to 19 us per 64 columns where the tile
   // steps wait for a panel and two partial update rounds (n = 12,000: 11.8
   // against 16.1 ms; the whole of n = 20,000: 50 ms, with 100 blocks left to
   // it 50.6, 200: 48.7, 320: 51.3; n = 40,000: 352, 350 and 354 ms).
@@ -788,7 +788,7 @@ double Context::loglik(KernelId kid, const double* theta, int metric, double* lo
     const int q = ts / kNB;
     profiled("gen", 0.0, 4.0 * (double)N * (N + 1.0), s1,
              [&] { generate_covariance(C, kid, theta, l1, l1, metric, s1); });
-    launch_flow_begin(Zcpy.d, N, flow_rhs, ws.info(), s1);
+    launch_flow_begin(Zcpy.d, N, flow_rhs, ws.dinv_base(), nb * 4096, ws.info(), s1);
     profiled("potrf_diag", potrf_flops(N), 0.0, s1, [&] {
       launch_chol_flow(C.view(), C.pool_f64(), 0, 0, (int)nb, (int)nb, C.mt * q, ws.dinv_base(), ws.info(),
                        ws.flags(), s1, flow_rhs, flow_clock);

@@ -88,8 +88,11 @@ long chol_flow_flags(int mt, int ts);
 void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int j1, int i_end, int j_pad,
                       double* dinv, int* info, int* flags, hipStream_t s, double* rhs = nullptr,
                       long long* clock = nullptr);
-// info <- 0, z into the first row of rhs.
-void launch_flow_begin(const double* z, long n, double* rhs, int* info, hipStream_t s);
+// Before the first launch of a factorisation: info <- 0 and the nd doubles
+// of dinv that it will write unset.  launch_flow_begin: the same and z into
+// the first row of rhs.
+void launch_flow_reset(double* dinv, long nd, int* info, hipStream_t s);
+void launch_flow_begin(const double* z, long n, double* rhs, double* dinv, long nd, int* info, hipStream_t s);
 // y <- the first row of rhs; host[0] <- info, host[1] <- clock[1] - clock[0],
 // host[4 + 2 b], host[5 + 2 b] <- sums of y^2 and log L_ii over rows
 // [256 b, 256 (b + 1)); flow_end_doubles(n) doubles of pinned host memory.
