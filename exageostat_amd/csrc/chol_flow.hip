@@ -857,19 +857,28 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 
 template <int R, bool MIXED, bool RHS = false>
 void launch_flow(const FlowArgs& a, hipStream_t s) {
-  static int slots = 0;
+  static int cus = 0, slots = 0;
   if (!slots) {
-    int dev = 0, cus = 0, occ = 1;
+    int dev = 0, n = 0, occ = 1;
     EXA_HIP(hipGetDevice(&dev));
-    EXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    EXA_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
     EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_chol_flow<R, MIXED, RHS>, 256, 0));
-    slots = cus * (occ > 0 ? occ : 1);
+    cus = n;
+    slots = n * (occ > 0 ? occ : 1);
   }
+  // Small matrices wait for the chain, which is faster without a second
+  // work-group on its CU (more LDS than half a CU's keeps it away); larger
+  // ones for the sums.  Likelihood, one / two work-groups per CU: n = 2,000
+  // 437 / 453 us, 3,200 675 / 755, 4,400 1,134 / 1,156, 5,003 1,514 / 1,428,
+  // 6,000 2,270 / 2,000.
+  constexpr int kChainBlocks = 70, kMoreLds = 16384;
+  const bool alone = a.pool && a.i_end - a.j0 <= kChainBlocks;
+  const int most = alone ? cus : slots;
   long tasks = 0;
-  for (int j = a.j0; j < a.j1 && tasks < slots; ++j)
+  for (int j = a.j0; j < a.j1 && tasks < most; ++j)
     tasks += 1 + RHS + row_groups<R, MIXED>(rows_from(j, a.j1), a.i_end, a.q);
-  long grid = tasks < slots ? tasks : slots;
-  hipLaunchKernelGGL((k_chol_flow<R, MIXED, RHS>), dim3((unsigned)grid), dim3(256), 0, s, a);
+  const long grid = tasks < most ? tasks : most;
+  hipLaunchKernelGGL((k_chol_flow<R, MIXED, RHS>), dim3((unsigned)grid), dim3(256), alone ? kMoreLds : 0, s, a);
   EXA_HIP(hipGetLastError());
 }
 
