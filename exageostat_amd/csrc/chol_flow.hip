@@ -87,28 +87,60 @@ __device__ __forceinline__ void rsqrt_pair(double x, double& rs, double& s) {
   rs = h + h;
 }
 
-// One column of panel16, then the next ones.
-template <int C>
-__device__ __forceinline__ void panel_columns(double (&d)[16], double (&a)[16], double& own, int l16);
+// Column C's update of column C2.
 template <int C, int C2>
 __device__ __forceinline__ void panel_update(double (&d)[16], double (&a)[16], double nd, double na) {
   if constexpr (C2 < 16) {
     fma_row_lane<C2>(d[C2], d[C], nd);
     fma_row_lane<C2>(a[C2], d[C], na);
-    panel_update<C, C2 + 1>(d, a, nd, na);
   }
 }
+template <int C, int C2>
+__device__ __forceinline__ void panel_updates(double (&d)[16], double (&a)[16], double nd, double na) {
+  if constexpr (C2 < 16) {
+    panel_update<C, C2>(d, a, nd, na);
+    panel_updates<C, C2 + 1>(d, a, nd, na);
+  }
+}
+// The updates from column C, given -d[C] / d_c and -a[C] / d_c, with the
+// chain of the next pivot's reciprocal between them: in program order, since
+// the compiler does not know how long either takes.
 template <int C>
-__device__ __forceinline__ void panel_columns(double (&d)[16], double (&a)[16], double& own, int l16) {
-  if constexpr (C < 16) {
+__device__ __forceinline__ void panel_columns(double (&d)[16], double (&a)[16], double& own, int l16, double nd,
+                                              double na) {
+  if constexpr (C < 15) {
+    panel_update<C, C + 1>(d, a, nd, na);
+    panel_update<C, C + 2>(d, a, nd, na);
+    __builtin_amdgcn_sched_barrier(0);
     // a DPP operand needs two wait states after its write, which the
     // compiler does not see inside the assembly of fma_row_lane
-    asm("s_nop 1" : "+v"(d[C]));
-    const double piv = row_lane<C>(d[C]);
-    own = l16 == C ? piv : own;
-    const double r = recip3(piv);
-    panel_update<C, C + 1>(d, a, -d[C] * r, -a[C] * r);
-    panel_columns<C + 1>(d, a, own, l16);
+    asm("s_nop 1" : "+v"(d[C + 1]));
+    const double piv = row_lane<C + 1>(d[C + 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    panel_update<C, C + 3>(d, a, nd, na);
+    __builtin_amdgcn_sched_barrier(0);
+    const double r = __builtin_amdgcn_rcp(piv);
+    __builtin_amdgcn_sched_barrier(0);
+    panel_update<C, C + 4>(d, a, nd, na);
+    panel_update<C, C + 5>(d, a, nd, na);
+    own = l16 == C + 1 ? piv : own;
+    __builtin_amdgcn_sched_barrier(0);
+    const double e = fma(-piv, r, 1.0);
+    __builtin_amdgcn_sched_barrier(0);
+    panel_update<C, C + 6>(d, a, nd, na);
+    __builtin_amdgcn_sched_barrier(0);
+    const double e2 = fma(e, e, e);
+    __builtin_amdgcn_sched_barrier(0);
+    panel_update<C, C + 7>(d, a, nd, na);
+    __builtin_amdgcn_sched_barrier(0);
+    const double r3 = fma(r, e2, r);
+    __builtin_amdgcn_sched_barrier(0);
+    panel_update<C, C + 8>(d, a, nd, na);
+    __builtin_amdgcn_sched_barrier(0);
+    const double nd1 = -d[C + 1] * r3, na1 = -a[C + 1] * r3;
+    __builtin_amdgcn_sched_barrier(0);
+    panel_updates<C, C + 9>(d, a, nd, na);
+    panel_columns<C + 1>(d, a, own, l16, nd1, na1);
   }
 }
 template <int C>
@@ -134,9 +166,13 @@ __device__ __forceinline__ void panel_scale(double (&d)[16], double (&a)[16], do
 // as rows of L^-T.  Returns the mask of columns whose pivot is not positive;
 // those and all later columns are NaN then.
 __device__ __forceinline__ unsigned panel16(double (&d)[16], double (&a)[16], int lane) {
-  const int l16 = lane & 15;
-  double own = 1.0, rs, root;
-  panel_columns<0>(d, a, own, l16);
+  int l16 = lane & 15;
+  asm("" : "+v"(l16));  // comparisons with it stay here
+  double rs, root;
+  const double piv = row_lane<0>(d[0]);
+  double own = l16 == 0 ? piv : 1.0;
+  const double r = recip3(piv);
+  panel_columns<0>(d, a, own, l16, -d[0] * r, -a[0] * r);
   rsqrt_pair(own, rs, root);
   panel_scale<0>(d, a, rs);
 #pragma unroll
@@ -553,8 +589,8 @@ __device__ __forceinline__ void task_rhs(const FlowArgs& a, int j, double* lds, 
 }
 
 // LDS of a D task (doubles): the operand ring, then X = L_{j,j-1}; the
-// factor's and the inverse's 16 x 16 blocks.
-constexpr int kLs = 4096, kXs = kLs + 2560, kDiagLds = kXs + 2560;
+// factor's and the inverse's 16 x 16 blocks, and a 16 x 16 identity.
+constexpr int kLs = 4096, kXs = kLs + 2560, kId = kXs + 2560, kDiagLds = kId + 256;
 
 // S(bi, bj) -= L(bi, p) L(bj, p)^T
 __device__ __forceinline__ void diag_update(double* Ls, int bi, int bj, int p, int lane) {
@@ -592,20 +628,19 @@ __device__ __forceinline__ void inverse_put(double* Xs, const dx4& y, int p, int
 }
 
 // Panel p of the diagonal block, by one wave.
-__device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, double* Ls, double* Xs, int lane) {
+__device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, double* Ls, double* Xs, const double* id,
+                                           int lane) {
   // lanes 0 .. 15 of c: an identity (its rows become the inverse's columns);
   // 16 .. 63: block rows p + 1 ..
   double d[16], c[16];
   const int l16 = lane & 15, bi = p + (lane >> 4);
   const double* dd = Ls + blk16(p, p) + l16;
-  const double* cc = Ls + blk16(bi < 4 ? bi : p, p) + l16;
+  const double* cc = (lane < 16 ? id : Ls + blk16(bi < 4 ? bi : p, p)) + l16;
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     d[e] = dd[e * 16];
     c[e] = cc[e * 16];
   }
-#pragma unroll
-  for (int e = 0; e < 16; ++e) c[e] = lane < 16 ? (lane == e ? 1.0 : 0.0) : c[e];
   const unsigned bad = panel16(d, c, lane);
   if (bad && lane == 0) atomicCAS(a.info, 0, j * kNB + 16 * p + __builtin_ctz(bad) + 1);
   if (lane < 16) {
@@ -614,7 +649,7 @@ __device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, doub
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       dst[e] = c[e];
-      ldst[e * 16] = lane >= e ? d[e] : 0.0;
+      ldst[e * 16] = d[e];  // the zeros above the diagonal when it is written out
     }
   } else if (bi < 4) {
     double* dst = Ls + blk16(bi, p) + l16;
@@ -699,7 +734,7 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
   // X is out: D_{j+1} and the T tasks of its column wait for it
   if (chained && tid == 64) flag_set(a.flags + kRows + 16 * (j - a.j0), j - a.j0);
   if (wave == 0) {
-    diag_panel(a, j, 0, Ls, Xs, lane);
+    diag_panel(a, j, 0, Ls, Xs, lds + kId, lane);
   } else {
     s_frag(1);
     s_frag(2);
@@ -711,7 +746,7 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
 #pragma unroll 1
   for (int p = 1; p < 4; ++p) {
     if (wave == 0) {
-      diag_panel(a, j, p, Ls, Xs, lane);
+      diag_panel(a, j, p, Ls, Xs, lds + kId, lane);
     } else {
       // what panel p - 1 leaves for the panels after p, and the inverse
       for (int bj = p + 1; bj <= wave; ++bj) diag_update(Ls, wave, bj, p - 1, lane);
@@ -761,7 +796,8 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
   for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
     for (int bj = 0; bj < 4; ++bj) {
-      out[16 * bi + r + (long)(16 * bj + c) * ts] = bj <= bi ? Ls[blk16(bi, bj <= bi ? bj : 0) + tid] : 0.0;
+      out[16 * bi + r + (long)(16 * bj + c) * ts] =
+          bj < bi || (bj == bi && r >= c) ? Ls[blk16(bi, bj <= bi ? bj : 0) + tid] : 0.0;
       if (bj > bi) dinv[16 * bi + r + (16 * bj + c) * 64] = 0.0;
     }
   gdouble* top = out - rj.rb;
@@ -814,6 +850,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   const int tid = threadIdx.x;
   int j = a.j0;
   long base = 0;  // first task of column j
+  lds[kId + tid] = tid % 17 == 0 ? 1.0 : 0.0;
   if (RHS && blockIdx.x == 0 && tid == 0) a.clock[0] = wall_clock64();
   for (;;) {
     if (tid == 0) sh[0] = atomicAdd(a.flags + kClaim, 1);
