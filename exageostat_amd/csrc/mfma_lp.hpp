@@ -4,7 +4,7 @@
 //
 // It computes acc += A * B^T for a BM x BN block from panel tiles that were
 // converted once per step into BF16 parts (k_split_panel), copied into a
-// three-stage LDS ring with direct-to-LDS loads.
+// ring in LDS with direct-to-LDS loads, and read from there one step ahead.
 // Result layout (measured on gfx950 with an in-bounds single-wave probe):
 // lane l, element v holds D[4*(l/16)+v][l%16]; operand layout: lane l holds
 // A[l%16][8*(l/16)+e] and B^T[l%16][8*(l/16)+e], e = 0..7.
@@ -12,6 +12,8 @@
 
 #include "common.hpp"
 #include "mfma.hpp"
+
+#include <type_traits>
 
 namespace exa {
 
@@ -111,9 +113,9 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint3
 //
 // The product copies the operands with
 // global_load_lds_dwordx4 (each wave-wide instruction writes 64 lanes x 16
-// bytes contiguously into LDS, no registers involved) into a three-stage
-// ring.  The LDS layout of a stage is the panel's own [k-group][row][8]:
-// array a (A hi, B hi, A lo, B lo) holds G = BK/8 groups of its rows.  A
+// bytes contiguously into LDS, no registers involved) into a ring of 32-deep
+// slices.  The LDS layout of a stage is the panel's own [k-group][row][8]:
+// array a (A hi, B hi, A lo, B lo) holds 4 groups of its rows.  A
 // 16-lane quarter of a fragment read covers 16 consecutive rows of one
 // group, 256 contiguous bytes, so neither the copies nor the reads conflict
 // on LDS banks.
@@ -124,23 +126,30 @@ struct Bf16dLds {
   static constexpr int A_ARR = G * C::BM * 8;  // halves
   static constexpr int B_ARR = G * C::BN * 8;
   static constexpr int STAGE = NARR * (A_ARR + B_ARR);
-  static constexpr int NSTAGE = 3;
+  static constexpr int NSTAGE = NSPLIT >= 3 ? 3 : 6;
   static constexpr int HALVES = NSTAGE * STAGE;
   static constexpr int CHUNKS = NARR * G * (C::BM + C::BN) / 64;  // wave-wide copies per stage
   static constexpr int PER_WAVE = CHUNKS / C::NW;
+  static_assert(C::BK == 32, "one slice is one step of the matrix cores");
   static_assert(C::BM % 64 == 0 && C::BN % 64 == 0, "rows must be whole 64-row chunks");
   static_assert(CHUNKS % C::NW == 0, "copies must split evenly over the waves");
 };
 
-
-
 // acc += A * B^T (A and B rows from the split panels, so the caller
-// subtracts the result), for K a multiple of BK.  The ring holds
-// slices kc, kc+1, kc+2: at step kc each wave waits for its own copies of
-// slice kc, a barrier makes every wave's copies visible and ends every read
-// of slice kc-1, whose buffer then receives slice kc+2.  The barrier is a
-// bare s_barrier: the copies are ordered by the explicit counter waits, and
-// LDS reads complete before the MFMAs that consume them.
+// subtracts the result), for K a multiple of 64.
+//
+// What bounds it is the LDS as much as the matrix cores (192 x 192 blocks, a
+// slice of the three products: 196 KB through the LDS against 1,728 cycles of
+// MFMA per SIMD), so the two have to run at the same time.  Fragments are
+// read one column group of B ahead of their use, the rows of A for the next
+// slice beside the column groups of the current one, and copies, reads and
+// adds stand between the MFMAs, each of which leaves 12 of its 16 cycles to
+// other instructions.  One barrier per slice: there every wave's copies of
+// the next slice have landed (they are then read), and every wave is past
+// the previous slice, whose buffer receives new copies.
+// Measured on 224 CUs, 192 x 192 x 960, three products: 39.6 us a block (1.20
+// PFLOP/s; 44.7 with the reads of a slice before its MFMAs), 50.2 with the
+// update of C from HBM (61); one product 18.0 us (18.7).
 template <class C, int NSPLIT>
 __device__ __forceinline__ void gemm_nt_bf16d(fx4 (&acc)[C::FM][C::FN], const uint16_t* __restrict__ Ah,
                                                   const uint16_t* __restrict__ Bh, long lo_off, long gs, int K,
@@ -153,89 +162,146 @@ __device__ __forceinline__ void gemm_nt_bf16d(fx4 (&acc)[C::FM][C::FN], const ui
   const int wn = wave - wm * C::WGN;
   // The copy decomposition is uniform per wave: keep it in scalar registers.
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);
+  const unsigned lane16 = lane * 16;
   // copy j of this wave: chunk c = wave * PER_WAVE + j of array (hi/lo,
   // A/B), k-group g, 64-row block rc; lo parts sit lo_off halves after hi.
-  auto issue = [&](int kc, int buf) {
-#pragma unroll
-    for (int j = 0; j < L::PER_WAVE; ++j) {
-      constexpr int per_a = L::G * (C::BM / 64), per_b = L::G * (C::BN / 64);
-      int c = wave_s * L::PER_WAVE + j;
-      const int pair = c / (per_a + per_b);  // 0: hi, 1: lo
-      c -= pair * (per_a + per_b);
-      const bool is_b = c >= per_a;
-      if (is_b) c -= per_a;
-      const int rows = is_b ? C::BN : C::BM;
-      const int g = c / (rows / 64);
-      const int rc = c - g * (rows / 64);
-      const uint16_t* base = is_b ? Bh : Ah;
-      const long goff = pair * lo_off + ((long)(kc * L::G + g) * gs + rc * 64) * 8;
-      const int loff = buf * L::STAGE + pair * (L::A_ARR + L::B_ARR) + (is_b ? L::A_ARR : 0) + (g * rows + rc * 64) * 8;
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(uintptr_t)(base + goff + lane * 8), (lds_void_t*)(lds + loff), 16,
-                                       0, 0);
-    }
+  auto issue = [&](int kc, int buf, int j) {
+    constexpr int per_a = L::G * (C::BM / 64), per_b = L::G * (C::BN / 64);
+    int c = wave_s * L::PER_WAVE + j;
+    const int pair = c / (per_a + per_b);  // 0: hi, 1: lo
+    c -= pair * (per_a + per_b);
+    const bool is_b = c >= per_a;
+    if (is_b) c -= per_a;
+    const int rows = is_b ? C::BN : C::BM;
+    const int g = c / (rows / 64);
+    const int rc = c - g * (rows / 64);
+    const uint16_t* base = is_b ? Bh : Ah;
+    const long goff = pair * lo_off + ((long)(kc * L::G + g) * gs + rc * 64) * 8;
+    const int loff = buf * L::STAGE + pair * (L::A_ARR + L::B_ARR) + (is_b ? L::A_ARR : 0) + (g * rows + rc * 64) * 8;
+    typedef __attribute__((address_space(1))) const char gchar;
+    gchar* src = (gchar*)(uintptr_t)(base + goff);  // uniform: one lane offset serves all copies
+    __builtin_amdgcn_global_load_lds((glb_void_t*)(src + lane16), (lds_void_t*)(lds + loff), 16, 0, 0);
   };
-  auto compute = [&](int buf) {
-    const uint16_t* st = lds + buf * L::STAGE;
-#pragma unroll
-    for (int kk = 0; kk < C::BK; kk += 32) {
-      const int gq = kk / 8 + (lane >> 4);
-      bf16x8 ah[C::FM], bh[C::FN];
-#pragma unroll
-      for (int i = 0; i < C::FM; ++i)
-        ah[i] = *reinterpret_cast<const bf16x8*>(st + (gq * C::BM + wm * C::WM + i * 16 + (lane & 15)) * 8);
-#pragma unroll
-      for (int j = 0; j < C::FN; ++j)
-        bh[j] = *reinterpret_cast<const bf16x8*>(st + L::A_ARR + (gq * C::BN + wn * C::WN + j * 16 + (lane & 15)) * 8);
-      if (NSPLIT >= 3) {
-        bf16x8 al[C::FM], bl[C::FN];
-        const uint16_t* sl = st + L::A_ARR + L::B_ARR;
-#pragma unroll
-        for (int i = 0; i < C::FM; ++i)
-          al[i] = *reinterpret_cast<const bf16x8*>(sl + (gq * C::BM + wm * C::WM + i * 16 + (lane & 15)) * 8);
-#pragma unroll
-        for (int j = 0; j < C::FN; ++j)
-          bl[j] = *reinterpret_cast<const bf16x8*>(sl + L::A_ARR + (gq * C::BN + wn * C::WN + j * 16 + (lane & 15)) * 8);
-        // Each 32-deep chunk is summed by its own MFMA chain from zero
-        // (smallest terms first) and added to the running sum with one
-        // round-to-nearest FP32 add: the MFMA's internal accumulation is
-        // not correctly rounded (about 1 ulp of error per instruction,
-        // measured on gfx950), and chaining all 3 K / 32 instructions into
-        // one accumulator lets that error build up at the running sum's
-        // magnitude.
-#pragma unroll
-        for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-          for (int j = 0; j < C::FN; ++j) {
-            fx4 t = {0.f, 0.f, 0.f, 0.f};
-            if (NSPLIT == 4) t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bl[j], t, 0, 0, 0);
-            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], t, 0, 0, 0);
-            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], t, 0, 0, 0);
-            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], t, 0, 0, 0);
-            acc[i][j] += t;
-          }
-      } else {
-#pragma unroll
-        for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-          for (int j = 0; j < C::FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-      }
-    }
-  };
+  constexpr bool SPLIT = NSPLIT >= 3;
+  constexpr int S = L::NSTAGE;
   const int nk = K / C::BK;
+  const int row = (lane >> 4), r16 = lane & 15;
+  const int ao = (row * C::BM + wm * C::WM + r16) * 8, bo = L::A_ARR + (row * C::BN + wn * C::WN + r16) * 8;
+  constexpr int LO = L::A_ARR + L::B_ARR;
+  bf16x8 ah[2][C::FM], al[SPLIT ? C::FM : 1], bh[2], bl[2];
+  auto read_hi = [&](int set, const uint16_t* st, int i) {
+    ah[set][i] = *reinterpret_cast<const bf16x8*>(st + ao + i * 128);
+  };
+  auto read_lo = [&](const uint16_t* st, int i) {
+    if constexpr (SPLIT) al[i] = *reinterpret_cast<const bf16x8*>(st + LO + ao + i * 128);
+  };
+  auto read_b = [&](int set, const uint16_t* st, int j) {
+    bh[set] = *reinterpret_cast<const bf16x8*>(st + bo + j * 128);
+    if (SPLIT) bl[set] = *reinterpret_cast<const bf16x8*>(st + LO + bo + j * 128);
+  };
   // The ring may still be read by the previous block's last steps.
   __builtin_amdgcn_s_barrier();
-  issue(0, 0);
-  if (nk > 1) issue(1, 1);
-  int buf = 0;
-  for (int kc = 0; kc < nk; ++kc) {
-    if (kc + 1 < nk) wait_vmcnt<L::PER_WAVE>();
-    else wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-    if (kc + 2 < nk) issue(kc + 2, buf == 0 ? 2 : buf - 1);
-    compute(buf);
-    buf = buf == 2 ? 0 : buf + 1;
+#pragma unroll
+  for (int st = 0; st < S - 1; ++st)
+#pragma unroll
+    for (int j = 0; j < L::PER_WAVE; ++j) issue(st < nk ? st : nk - 1, st, j);
+  wait_vmcnt<(S - 2) * L::PER_WAVE>();
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i) {
+    read_hi(0, lds, i);
+    read_lo(lds, i);
   }
+  read_b(0, lds, 0);
+  int buf = 0;
+  constexpr int NP = NSPLIT;                   // products, smallest terms first
+  constexpr int SLOTS = NP * C::FM;            // MFMAs per column group
+  // A group's MFMAs go in two halves of its row fragments, so that one half's
+  // sums are added, one or two values per MFMA, during the other's products.
+  constexpr int H = C::FM / 2;
+  static_assert(C::FM % 2 == 0, "two halves");
+  // Each 32-deep chunk is summed by its own MFMA chain from zero (smallest
+  // terms first) and added to the running sum with one round-to-nearest FP32
+  // add: the MFMA's internal accumulation is not correctly rounded (about 1
+  // ulp of error per instruction, measured on gfx950), and chaining all
+  // 3 K / 32 instructions into one accumulator lets that error build up at
+  // the running sum's magnitude.
+  fx4 t[SPLIT ? C::FM : 1];
+#pragma unroll
+  for (int i = 0; i < (SPLIT ? C::FM : 1); ++i) t[i] = fx4{0.f, 0.f, 0.f, 0.f};
+  auto slice = [&](auto par, int kc) {
+    constexpr int P = decltype(par)::value;  // the slice's fragment set of A
+    constexpr int FN = C::FN;
+    const int nbuf = buf == S - 1 ? 0 : buf + 1;
+    const uint16_t* st = lds + buf * L::STAGE;
+    const uint16_t* sn = lds + nbuf * L::STAGE;
+    const int kn = kc + S - 1 < nk ? kc + S - 1 : nk - 1;  // (past the end: a copy that nothing reads)
+    const int bn = buf == 0 ? S - 1 : buf - 1;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int cur = (P * FN + j) & 1;  // B's sets alternate over all column groups
+      const int jp = (j + FN - 1) % FN;
+      if (j == 0) {
+        wait_vmcnt<(S - 3) * L::PER_WAVE>();
+        __builtin_amdgcn_s_barrier();
+      }
+#pragma unroll
+      for (int sl = 0; sl < SLOTS; ++sl) {
+        const int h = sl / (NP * H), r = sl % (NP * H);
+        const int p = NP - 1 - r / H, i = h * H + r % H;  // 3: lo lo, 2: lo hi, 1: hi lo, 0: hi hi
+        if constexpr (SPLIT) {
+          const bf16x8 x = p >= 2 ? al[i] : ah[P][i], y = p == 3 || p == 1 ? bl[cur] : bh[cur];
+          if (p == NP - 1) {
+            t[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, fx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          } else {
+            t[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, t[i], 0, 0, 0);
+          }
+        } else {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[P][i], bh[cur], acc[i][j], 0, 0, 0);
+        }
+        if constexpr (SPLIT) {
+#pragma unroll
+          for (int e = 4 * r / NP; e < 4 * (r + 1) / NP; ++e) {
+            const int ie = (1 - h) * H + e / 4;
+            acc[ie][h ? j : jp][e % 4] += t[ie][e % 4];
+          }
+        }
+        // B of the next group; the high parts of the next slice's A in all
+        // groups but the last; its low parts in the last one, each over the
+        // current one right after its last use (after the last slice: what is
+        // there, unused).  Not before a group's first MFMA: the wait for a
+        // fragment is a wait for all LDS reads here, since the compiler takes
+        // the direct-to-LDS copies for unordered ones.
+        if (sl == 1) read_b(cur ^ 1, j + 1 < FN ? st : sn, j + 1 < FN ? j + 1 : 0);
+        if (j < FN - 1) {
+          const int i0 = j * C::FM / (FN - 1), i1 = (j + 1) * C::FM / (FN - 1);
+#pragma unroll
+          for (int ia = i0; ia < i1; ++ia) {
+            const int at = 3 + (ia - i0) * (SLOTS - 4) / (i1 - i0);
+            if ((at < SLOTS ? at : SLOTS - 1) == sl) read_hi(P ^ 1, sn, ia);
+          }
+        }
+        if (SPLIT && j == FN - 1 && r > (NP - 3) * H && r <= (NP - 2) * H) read_lo(sn, h * H + r - (NP - 3) * H - 1);
+        if (j == 0) {
+#pragma unroll
+          for (int c = 0; c < L::PER_WAVE; ++c)
+            if (c * SLOTS / L::PER_WAVE == sl) issue(kn, bn, c);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    buf = nbuf;
+  };
+#pragma unroll 1
+  for (int kc = 0; kc < nk; kc += 2) {
+    slice(std::integral_constant<int, 0>{}, kc);
+    slice(std::integral_constant<int, 1>{}, kc + 1);
+  }
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = H; i < C::FM; ++i) acc[i][C::FN - 1] += t[i];
+  }
+  wait_vmcnt<0>();
 }
 
 }  // namespace exa

@@ -120,10 +120,13 @@ void launch_split_panel(const TileView& v, int k, uint16_t* split, hipStream_t s
 // One block of C(m,n) -= A(m,k) B(n,k)^T, C of precision class CLS.
 template <int CLS, int BS>
 struct ClassCfg;
-// FP64 class: the FP64 core.
+// FP64 class: the FP64 core.  Few FP64 tiles meet many CUs, so the blocks are
+// short ones: 192 x 192 over 960 columns kept a CU for 300 us, which was most
+// of the column update that every panel waits for (n = 30,720: 375 us on
+// average, 190 with 64 x 192).
 template <int BS>
 struct ClassCfg<kF64, BS> {
-  using C = typename std::conditional<BS == 192, GemmCfg<192, 192, 2, 4, 16>,
+  using C = typename std::conditional<BS == 192, GemmCfg<64, 192, 2, 4, 16>,
             typename std::conditional<BS == 128, GemmCfg<128, 128, 2, 2, 16>, GemmCfg<64, 64, 2, 2, 16>>::type>::type;
   static constexpr int LDS_BYTES = C::LDS_DOUBLES * 8;
 };
@@ -147,8 +150,7 @@ struct ClassCfg<kF32Q, BS> {
 // Far class: FP32 storage, single BF16 MFMA operands.
 template <int BS>
 struct ClassCfg<kF32B, BS> {
-  using C = typename std::conditional<BS == 192, LpCfg<192, 192, 2, 4, 64>,
-            typename std::conditional<BS == 128, LpCfg<128, 128, 2, 2, 64>, LpCfg<64, 64, 2, 2, 64>>::type>::type;
+  using C = typename ClassCfg<kF32, BS>::C;
   static constexpr int NSPLIT = 1;
   static constexpr int LDS_BYTES = Bf16dLds<C, NSPLIT>::HALVES * 2;
 };
@@ -194,8 +196,9 @@ __device__ __forceinline__ void class_update(const TileView& v, int k, int m, in
     const uint16_t* Bh = split + 2 * (long)n * tt + (long)bj * C::BN * 8;
     fx4 acc[C::FM][C::FN];
     zero_acc_lp<C>(acc);
+    float* Cp = static_cast<float*>(v.ptr[tc]) + co;
     gemm_nt_bf16d<C, ClassCfg<CLS, BS>::NSPLIT>(acc, Ah, Bh, tt, v.ts, v.ts, reinterpret_cast<uint16_t*>(lds));
-    acc_add_lp<C, float>(acc, static_cast<float*>(v.ptr[tc]) + co, v.ts, -1.f);
+    acc_add_lp<C, float>(acc, Cp, v.ts, -1.f);
   }
 }
 
@@ -262,24 +265,25 @@ static void launch_per_class(const TileView& v, int k, const FusedSpans& sp, con
 }
 
 // The trailing update of one step over all three precision classes in one
-// persistent launch.  XCD x takes slice x of the FP64 class's block list,
-// then slice x of the FP32 list, then of the far list (the slowest blocks
-// first; contiguous slices keep the A and B panels hot in the XCD's L2), and
-// its work-groups stride through that sequence.  One launch instead of one
-// per class removes two launch tails per update.  Blocks are q x q per tile
-// pair (packed m << 16 | n); the strictly upper blocks of diagonal tiles
-// are skipped.
+// persistent launch.  XCD x takes slice x of each class's block list in
+// turn, and its work-groups stride through that sequence: work-groups that
+// start neighbouring blocks together stay together along K, so that an
+// operand slice is read once per XCD (claiming blocks from a counter instead
+// evens the ends out but loses that: 1,194 against 928 ms per evaluation at n = 90,000).
+// One launch instead of one per class removes two launch tails per update.
+// The strictly upper blocks of diagonal tiles (tile pairs packed m << 16 |
+// n) are skipped.
 template <int BS, int F32CLS>
 __global__ void __launch_bounds__((ClassCfg<kF64, BS>::C::NT))
     k_update_fused(TileView v, int k, FusedSpans sp, int nx, const uint16_t* split) {
   static_assert(ClassCfg<kF64, BS>::C::NT == ClassCfg<F32CLS, BS>::C::NT &&
                     ClassCfg<kF64, BS>::C::NT == ClassCfg<kF32B, BS>::C::NT,
                 "the classes share one work-group shape");
+  using CF = typename ClassCfg<kF64, BS>::C;
   constexpr int LB = ClassCfg<F32CLS, BS>::LDS_BYTES > ClassCfg<kF64, BS>::LDS_BYTES
                          ? ClassCfg<F32CLS, BS>::LDS_BYTES
                          : ClassCfg<kF64, BS>::LDS_BYTES;
   __shared__ __attribute__((aligned(16))) unsigned char lds[LB];
-  const int q = v.ts / BS;
   const int w = blockIdx.x;
   const int x = w % nx;
   const int gx = gridDim.x / nx;
@@ -303,16 +307,18 @@ __global__ void __launch_bounds__((ClassCfg<kF64, BS>::C::NT))
         c = 2;
       }
     }
+    const int cl = sp.cls[c];
+    const int bm = cl == 0 ? CF::BM : BS, bn = cl == 0 ? CF::BN : BS;
+    const int qm = v.ts / bm, per = qm * (v.ts / bn);
     const long b = st[c] + j;
-    const long p = b / (q * q);
-    const int rem = (int)(b - p * (q * q));
-    const int bi = rem % q;
-    const int bj = rem / q;
+    const long p = b / per;
+    const int rem = (int)(b - p * per);
+    const int bi = rem % qm;
+    const int bj = rem / qm;
     const int pk = sp.pairs[c][p];
     const int m = pk >> 16;
     const int n = pk & 0xFFFF;
-    if (m == n && bi < bj) continue;
-    const int cl = sp.cls[c];
+    if (m == n && (bi + 1) * bm <= bj * bn) continue;
     if (cl == 0) class_update<kF64, BS>(v, k, m, n, bi, bj, split, lds);
     else if (cl == 1) class_update<F32CLS, BS>(v, k, m, n, bi, bj, split, lds);
     else class_update<kF32B, BS>(v, k, m, n, bi, bj, split, lds);
@@ -342,11 +348,13 @@ static int fused_grid_cap() {
 
 template <int BS, int F32CLS>
 static void launch_fused_bs(const TileView& v, int k, const FusedSpans& sp0, const uint16_t* split, hipStream_t s) {
+  using CF = typename ClassCfg<kF64, BS>::C;
   const long q = v.ts / BS;
   FusedSpans sp = sp0;
   long total = 0;
   for (int c = 0; c < 3; ++c) {
-    sp.nblocks[c] = sp0.nblocks[c] * q * q;  // pairs -> blocks
+    // pairs -> blocks
+    sp.nblocks[c] = sp0.nblocks[c] * (sp.cls[c] == 0 ? (long)(v.ts / CF::BM) * (v.ts / CF::BN) : q * q);
     total += sp.nblocks[c];
   }
   if (total <= 0) return;
