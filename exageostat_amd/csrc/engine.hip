@@ -77,6 +77,12 @@ void TileMatrix::allocate(int m_, int n_, int ts_, bool lower_, const std::vecto
   if (ts_ <= 0 || ts_ % kNB != 0 || ts_ > 1024)
     throw std::invalid_argument("tile size must be a multiple of 64 and at most 1024");
   if (lower_ && m_ != n_) throw std::invalid_argument("lower-packed matrices must be square");
+  // The same matrix again, all FP64 (kriging allocates per call): its memory
+  // and tables are kept.  Giving them back and asking again took 0.48 of
+  // 2.45 ms at n = 6,000.
+  if (d_prec_ && m == m_ && n == n_ && ts == ts_ && lower == lower_ && prec.empty() && pool_f64() &&
+      fp64_slots_ == fp64_slots)
+    return;
   release();
   m = m_;
   n = n_;
