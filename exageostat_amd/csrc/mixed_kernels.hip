@@ -325,9 +325,12 @@ __global__ void __launch_bounds__((ClassCfg<kF64, BS>::C::NT))
   }
 }
 
-// Work-groups of the fused update: one per CU less the CUs left to the
-// panel factorisation on the other stream (32 by default, 4 per XCD; with
-// fewer the diagonal factorisation starves), times the occupancy.
+// Work-groups of the fused update: one per CU, times the occupancy.  The
+// panel factorisation on the other stream then runs when they end: it is one
+// launch per tile column now, and leaving CUs to it costs the update more
+// than the overlap gives.  CUs left, ms per evaluation at n = 30,720 /
+// 90,000: 32 69.1 / 980, 24 69.3 / 961, 16 69.7 / 982, 8 67.5 / 928,
+// 0 65.4 / 912 (EXAGEOSTAT_RESERVE_CUS overrides).
 template <int BS, int F32CLS>
 static int fused_grid_cap() {
   static int cap = 0;
@@ -337,7 +340,7 @@ static int fused_grid_cap() {
   EXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_update_fused<BS, F32CLS>,
                                                        ClassCfg<kF64, BS>::C::NT, 0));
-  int reserve = 32;
+  int reserve = 0;
   if (const char* e = getenv("EXAGEOSTAT_RESERVE_CUS")) reserve = atoi(e);
   if (reserve < 0 || reserve >= cus) reserve = 0;
   cap = (cus - reserve) * (occ > 0 ? occ : 1);
