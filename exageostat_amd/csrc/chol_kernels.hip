@@ -160,11 +160,12 @@ __global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2)))
 
 static int g_update_wgs = 0;
 
-// Work-groups of the persistent update: CUs minus a reserve for the panel
-// factorisation (EXAGEOSTAT_RESERVE_CUS, default 8: at n = 90,000 the FP64
-// factorisation takes 4.40 s with 4 or 8 reserved CUs, 4.52 s with 16 and
-// 4.66 s with 24), times the occupancy,
-// rounded down to a multiple of 8 (XCDs).
+// Work-groups of the persistent update: one round of the whole chip, rounded
+// down to a multiple of 8 (XCDs).  CUs kept free for the panel factorisation
+// on the other stream (EXAGEOSTAT_RESERVE_CUS) cost the update more than the
+// overlap gives, since a panel is one launch: with 0 / 8 / 16 of them the
+// FP64 likelihood takes 49.7 / 51.5 / 52.1 ms at n = 20,000, 355 / 365 / 375 ms
+// at n = 40,000 and 3.72 / 3.83 s (0 / 8) at n = 90,000.
 template <class C>
 static int update_grid_cap() {
   static int cap = 0;
@@ -173,7 +174,7 @@ static int update_grid_cap() {
   EXA_HIP(hipGetDevice(&dev));
   EXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_tile_update<C>, C::NT, 0));
-  int reserve = 8;
+  int reserve = 0;
   if (const char* e = getenv("EXAGEOSTAT_RESERVE_CUS")) reserve = atoi(e);
   if (reserve < 0 || reserve >= cus) reserve = 0;
   cap = (cus - reserve) * (occ > 0 ? occ : 1);
