@@ -56,6 +56,12 @@ static constexpr int kPotriSplit = 4;
 
 void destroy_adjoint(AdjointState* a) { delete a; }
 
+// Rows up to which the sweep takes the two-launch columns.  Likelihood with
+// gradient, blocked stages / two launches: n = 900, tiles of 64 896 / 696 us, of
+// 320 572 / 485; 1,600, 320 877 / 762; 2,000, 192 1,789 / 1,193; 2,880, 320 1,726 /
+// 1,748 and 64 3,521 / 3,390.
+static constexpr long kSmallRows = 2560;
+
 // Z = Sigma^-1 in place of the factor held in A (tile_potrf output, with the
 // inverted diagonal tiles in ws).
 void tile_potri_inplace(TileMatrix& A, CholWorkspace& ws, double* P, double* Q, hipStream_t s, double* W,
@@ -73,6 +79,12 @@ void tile_potri_inplace(TileMatrix& A, CholWorkspace& ws, double* P, double* Q, 
   const int mt = A.mt;
   auto rows = [&](int t) { return (double)std::min<long>(A.ts, (long)A.m - (long)t * A.ts); };
   launch_takahashi_begin(v, ws.xinv_base(), P, s);
+  if (U && !f32 && (long)mt * A.ts <= kSmallRows) {
+    const double n = (double)A.m;
+    profiled("potri_col", 2.0 / 3.0 * n * n * n, 0.0, s, [&] { launch_sweep_small(v, P, uv, s); });
+    ws.factored = nullptr;
+    return;
+  }
   for (int k = mt - 1; k >= 0; --k) {
     const double below = (double)A.m - (double)(k + 1) * A.ts;
     const double rk = rows(k);

@@ -291,6 +291,128 @@ __global__ void __launch_bounds__(256) k_sum_diag(const double* Q, int cnt, int 
   }
 }
 
+// ---- small matrices --------------------------------------------------------
+// Up to some 2,500 rows the stages above are as long as their launches and
+// their work-groups' latency (five launches per column, 45 us with tiles of 64).
+// There every P_jk is formed in one launch, P_jk^T in tile (j, k) of U, and a
+// column takes two launches: Z_mk for m > k, and Z_kk.
+template <class C>
+__global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2)))
+    k_trmm_all(TileView v, const double* P, TileView U) {
+  __shared__ __attribute__((aligned(16))) double lds[PipeLds<C, 2>::DOUBLES];
+  const int qb = v.ts / C::BM;
+  const long pair = blockIdx.x / (qb * qb);
+  const int rem = (int)(blockIdx.x - pair * qb * qb);
+  int r, k;
+  tri_decode(pair, r, k);
+  const int j = r + 1;  // k <= r = j - 1
+  const int bi = rem / qb, bj = rem % qb;
+  const long ts = v.ts;
+  const long k0 = (long)bi * C::BM;
+  dx4 acc[C::FM][C::FN];
+  zero_acc<C>(acc);
+  gemm_nt_pipe<C, 2>(
+      acc, 1,
+      [&](int, const double*& A, const double*& B) {
+        A = P + (long)k * ts * ts + bi * C::BM + k0 * ts;
+        B = tile_f64(v, j, k) + bj * C::BN + k0 * ts;
+      },
+      ts, (int)(ts - k0), lds);
+  pipe_put<C>(acc, tile_f64(U, j, k) + bi * C::BM + (long)bj * C::BN * ts, ts);
+}
+
+// One 32 x 16 block of Z_mk = - sum_{j>k} Z(m,j) P_jk (DIAG: of the lower
+// triangle of Z_kk = X_kk^T X_kk - sum_{j>k} Z_jk^T P_jk, written to both).
+// The eight waves take every eighth 16-deep chunk of the sum, operands straight
+// from memory, and their partial sums are added in a fixed order: no sum is
+// longer than an eighth of it, and there is no second launch.
+// Z_jk^T and Z(m,j) = Z_jm^T for j > m are read along columns.
+// Bound by the latency of its loads and of the launch (n = 900, tiles of 64: 21 us
+// a column for both launches against 45 for five).
+template <bool DIAG>
+__global__ void __launch_bounds__(512) k_sweep_small(TileView v, int k, const double* P, TileView U) {
+  constexpr int BR = 32, BC = 16;
+  __shared__ double red[8][BR * BC];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long ts = v.ts;
+  const int qr = v.ts / BR, qc = v.ts / BC;
+  int m = k, bi, bj;
+  if (DIAG) {
+    bi = blockIdx.x % qr;
+    bj = blockIdx.x / qr;
+    if ((bi + 1) * BR <= bj * BC) return;
+  } else {
+    const int per = qr * qc;
+    m = k + 1 + blockIdx.x / per;
+    const int rem = blockIdx.x % per;
+    bi = rem % qr;
+    bj = rem / qr;
+  }
+  const int per_seg = v.ts / 16;
+  const int j0 = DIAG ? k : k + 1;  // DIAG: "j = k" is X^T X
+  const int chunks = (v.mt - j0) * per_seg;
+  const int r16 = lane & 15, k4 = lane >> 4;
+  typedef __attribute__((address_space(1))) const double gD;
+  double a[2][8], b[2][4];
+  auto fetch = [&](int set, int ch) {
+    const int j = j0 + ch / per_seg;
+    const long kk = (long)(ch % per_seg) * 16 + k4;
+    const bool xx = DIAG && j == k;
+    const double* Bt = (xx ? P + (long)k * ts * ts : tile_f64(U, j, k)) + bj * BC + r16;
+    const bool along = DIAG ? !xx : j > m;  // A(r, kk) at kk + r ts
+    const double* At = xx ? P + (long)k * ts * ts : (DIAG ? tile_f64(v, j, k) : tile_f64(v, j > m ? j : m, j > m ? m : j));
+    const long ar = along ? ts : 1, ak = along ? 1 : ts;
+    gD* A = (gD*)(uintptr_t)(At + (long)(bi * BR + r16) * ar + kk * ak);
+    gD* B = (gD*)(uintptr_t)(Bt + kk * ts);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      a[set][e] = A[4 * e * ak];
+      a[set][4 + e] = A[16 * ar + 4 * e * ak];
+      b[set][e] = B[4 * e * ts];
+    }
+    if (xx) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[set][e] = -a[set][e];
+    }
+  };
+  dx4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+  auto step = [&](int set) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      acc[0] = mfma_f64(a[set][e], b[set][e], acc[0]);
+      acc[1] = mfma_f64(a[set][4 + e], b[set][e], acc[1]);
+    }
+  };
+  int ch = wave;
+  if (ch < chunks) fetch(0, ch);
+  for (; ch < chunks; ch += 16) {
+    if (ch + 8 < chunks) fetch(1, ch + 8);
+    step(0);
+    if (ch + 8 >= chunks) break;
+    if (ch + 16 < chunks) fetch(0, ch + 16);
+    step(1);
+  }
+  // element e of lane l: row 16 i + l/16 + 4 e, column l%16
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[wave][16 * i + k4 + 4 * e + BR * r16] = acc[i][e];
+  __syncthreads();
+  double z = 0.0;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) z += red[w][tid];
+  const int r = bi * BR + tid % BR, c = bj * BC + tid / BR;
+  double* Z = tile_f64(v, m, k);
+  if (!DIAG) {
+    Z[r + c * ts] = -z;
+  } else if (r >= c) {
+    Z[r + c * ts] = -z;
+    if (r > c) Z[c + r * ts] = -z;
+  }
+}
+
 // Number of j ranges of the column stage: the split (at most 4, and at most
 // one tile per range, and only as many as the slab buffer holds) whose work
 // units fill whole rounds of the concurrent work-groups best; each extra
@@ -379,6 +501,28 @@ static void takahashi_cfg(const TileView& v, int k, double* P, double* Q, double
 void launch_takahashi_begin(const TileView& v, const double* xinv, double* P, hipStream_t s) {
   const long q = v.ts / 64;
   hipLaunchKernelGGL(k_transpose_tiles, dim3((unsigned)(v.mt * q * q)), dim3(256), 0, s, xinv, P, v.ts);
+  EXA_HIP(hipGetLastError());
+}
+
+void launch_sweep_small(const TileView& v, const double* P, const TileView& U, hipStream_t s) {
+  if (U.mt != v.mt || U.ts != v.ts || !U.lower || !v.lower) throw std::invalid_argument("sweep: grids differ");
+  const long pairs = (long)v.mt * (v.mt - 1) / 2;
+  if (pairs > 0) {
+    if (v.ts % 192 == 0) {
+      const long q = v.ts / CP96::BM;
+      hipLaunchKernelGGL(k_trmm_all<CP96>, dim3((unsigned)(pairs * q * q)), dim3(CP96::NT), 0, s, v, P, U);
+    } else {
+      const long q = v.ts / CT64::BM;
+      hipLaunchKernelGGL(k_trmm_all<CT64>, dim3((unsigned)(pairs * q * q)), dim3(CT64::NT), 0, s, v, P, U);
+    }
+  }
+  const long per = (long)(v.ts / 32) * (v.ts / 16);
+  for (int k = v.mt - 1; k >= 0; --k) {
+    const long below = v.mt - k - 1;
+    if (below > 0)
+      hipLaunchKernelGGL(k_sweep_small<false>, dim3((unsigned)(below * per)), dim3(512), 0, s, v, k, P, U);
+    hipLaunchKernelGGL(k_sweep_small<true>, dim3((unsigned)per), dim3(512), 0, s, v, k, P, U);
+  }
   EXA_HIP(hipGetLastError());
 }
 

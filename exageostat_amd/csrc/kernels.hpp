@@ -189,6 +189,9 @@ struct MaternGradParams {
 void launch_takahashi_begin(const TileView& v, const double* xinv, double* P, hipStream_t s);
 void launch_takahashi_stage(const TileView& v, int k, double* P, double* Q, double* Zkk, int stage, hipStream_t s,
                             double* W = nullptr, int max_split = 1, const TileView* U = nullptr, bool f32 = false);
+// The whole sweep for small matrices (after launch_takahashi_begin); U: a
+// lower tile matrix of v's geometry, scratch.
+void launch_sweep_small(const TileView& v, const double* P, const TileView& U, hipStream_t s);
 struct BivariateGradParams {
   const double* x;
   const double* y;

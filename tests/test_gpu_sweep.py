@@ -1,7 +1,8 @@
 """The inverse from the tile factor at the sizes where the sweep's blocks
-change: 96 x 96 blocks for tiles of a multiple of 192 and 64 x 64 blocks else,
-one tile, ragged last tiles, tiles whose 64-row blocks straddle the 96-row
-ones."""
+change: with the transposed copy up to 2,560 rows in two launches a column,
+beyond (and without it) in blocked stages of 96 x 96 blocks for tiles of a
+multiple of 192 and 64 x 64 blocks else; one tile, ragged last tiles, tiles
+whose 64-row blocks straddle the 96-row ones."""
 from __future__ import annotations
 
 import numpy as np
@@ -11,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 EPS = np.finfo(float).eps
 KN = "univariate_matern_nuggets_stationary"
-SIZES = [(60, 64), (321, 64), (900, 64), (700, 128), (193, 192), (900, 192), (1500, 576), (1281, 320), (2100, 960)]
+SIZES = [(60, 64), (321, 64), (900, 64), (700, 128), (193, 192), (900, 192), (1500, 576), (1281, 320), (2560, 64),
+         (2100, 128), (2200, 192), (2600, 64), (2600, 128), (2600, 192), (2100, 960)]
 
 
 @pytest.fixture(scope="module")
