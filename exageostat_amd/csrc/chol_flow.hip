@@ -163,21 +163,20 @@ __device__ __forceinline__ void panel_scale(double (&d)[16], double (&a)[16], do
 // product and an update.  1.13 us per panel; with v_readlane broadcasts into
 // scalar registers and a square root per column 2.05 us.
 // Rows below the diagonal block come out as rows of L, rows of an identity
-// as rows of L^-T.  Returns the mask of columns whose pivot is not positive;
-// those and all later columns are NaN then.
-__device__ __forceinline__ unsigned panel16(double (&d)[16], double (&a)[16], int lane) {
+// as rows of L^-T.  root: the diagonal entry of L of the lane's column (d
+// holds it as a product, one rounding further off).  Returns the mask of
+// columns whose pivot is not positive; those and all later columns are NaN
+// then.
+__device__ __forceinline__ unsigned panel16(double (&d)[16], double (&a)[16], double& root, int lane) {
   int l16 = lane & 15;
   asm("" : "+v"(l16));  // comparisons with it stay here
-  double rs, root;
+  double rs;
   const double piv = row_lane<0>(d[0]);
   double own = l16 == 0 ? piv : 1.0;
   const double r = recip3(piv);
   panel_columns<0>(d, a, own, l16, -d[0] * r, -a[0] * r);
   rsqrt_pair(own, rs, root);
   panel_scale<0>(d, a, rs);
-#pragma unroll
-  for (int c = 0; c < 16; ++c)
-    if (l16 == c) d[c] = root;
   const unsigned bad = (unsigned)__ballot(!(own > 0.0)) & 0xffffu;
   if (bad) {
     const int first = __builtin_ctz(bad);
@@ -641,7 +640,8 @@ __device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, doub
     d[e] = dd[e * 16];
     c[e] = cc[e * 16];
   }
-  const unsigned bad = panel16(d, c, lane);
+  double root;
+  const unsigned bad = panel16(d, c, root, lane);
   if (bad && lane == 0) atomicCAS(a.info, 0, j * kNB + 16 * p + __builtin_ctz(bad) + 1);
   if (lane < 16) {
     double* dst = Xs + blk16(p, p) + lane * 16;
@@ -651,6 +651,7 @@ __device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, doub
       dst[e] = c[e];
       ldst[e * 16] = d[e];  // the zeros above the diagonal when it is written out
     }
+    if (!(bad & ((2u << lane) - 1))) ldst[lane * 16] = root;  // (from the first bad column on: the NaN)
   } else if (bi < 4) {
     double* dst = Ls + blk16(bi, p) + l16;
 #pragma unroll
