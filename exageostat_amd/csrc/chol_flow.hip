@@ -927,7 +927,9 @@ __global__ void __launch_bounds__(256) k_flow_begin(const double* z, long n, dou
                                                     int* info) {
   const long c = (long)blockIdx.x * 256 + threadIdx.x;
   if (c == 0) *info = 0;
-  if (c < n) rhs[c * kNB] = z[c];
+  // The padding too (nd / 64 columns): the buffer serves matrices of several
+  // orders, and a NaN left there would spread over its block as 0 * NaN.
+  if (c < nd / kNB) rhs[c * kNB] = c < n ? z[c] : 0.0;
   for (long e = c; e < nd; e += (long)gridDim.x * 256) reinterpret_cast<long long*>(dinv)[e] = kUnset;
 }
 __global__ void __launch_bounds__(256) k_flow_reset(double* dinv, long nd, int* info) {
@@ -939,13 +941,13 @@ __global__ void __launch_bounds__(256) k_flow_reset(double* dinv, long nd, int* 
 // After it: y = L^-1 z into a vector, and per work-group the sums of y^2 and
 // of log L_ii over 256 rows, written with info to host memory.
 __global__ void __launch_bounds__(256) k_flow_end(TileView v, const double* rhs, long n, double* y, const int* info,
-                                                  const long long* clock, double* host) {
+                                                  const long long* clock, double* host, bool keep) {
   __shared__ double red[2][4];
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   double s = 0.0, d = 0.0;
   if (i < n) {
     const double w = rhs[i * kNB];
-    y[i] = w;
+    if (!keep || *info == 0) y[i] = w;
     s = w * w;
     const int k = (int)(i / v.ts);
     const long r = i - (long)k * v.ts;
@@ -1011,8 +1013,9 @@ void launch_flow_reset(double* dinv, long nd, int* info, hipStream_t s) {
 }
 long flow_end_doubles(long n) { return 4 + 2 * ((n + 255) / 256); }
 void launch_flow_end(const TileView& v, const double* rhs, long n, double* y, const int* info, const long long* clock,
-                     double* host, hipStream_t s) {
-  hipLaunchKernelGGL(k_flow_end, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, v, rhs, n, y, info, clock, host);
+                     double* host, bool keep, hipStream_t s) {
+  hipLaunchKernelGGL(k_flow_end, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, v, rhs, n, y, info, clock, host,
+                     keep);
   EXA_HIP(hipGetLastError());
 }
 

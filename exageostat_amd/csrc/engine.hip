@@ -769,6 +769,37 @@ void Context::ensure_partial(long n) {
   partial_len = n;
 }
 
+int Context::factor_solve(TileMatrix& A, const double* z, double* y) {
+  const long n = A.m, nb = (n + kNB - 1) / kNB;
+  if (!flow_clock) {
+    int wall_khz = 0;
+    EXA_HIP(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, 0));
+    wall_rate = wall_khz > 0 ? 1e3 * wall_khz : 1e8;
+    EXA_HIP(hipMalloc(&flow_clock, 2 * sizeof(long long)));
+  }
+  if (flow_blocks < nb) {
+    if (flow_rhs) (void)hipFree(flow_rhs);
+    if (flow_host) (void)hipHostFree(flow_host);
+    flow_rhs = flow_host = nullptr;
+    flow_blocks = 0;
+    EXA_HIP(hipHostMalloc(&flow_host, sizeof(double) * flow_end_doubles(nb * kNB), hipHostMallocDefault));
+    EXA_HIP(hipMalloc(&flow_rhs, sizeof(double) * nb * 4096));
+    EXA_HIP(hipMemset(flow_rhs, 0, sizeof(double) * nb * 4096));
+    EXA_HIP(hipDeviceSynchronize());
+    flow_blocks = nb;
+  }
+  ws.ensure(A.mt, A.ts);
+  launch_flow_begin(z, n, flow_rhs, ws.dinv_base(), nb * 4096, ws.info(), s1);
+  profiled("potrf_diag", potrf_flops(n), 0.0, s1, [&] {
+    launch_chol_flow(A.view(), A.pool_f64(), 0, 0, (int)nb, (int)nb, A.mt * (A.ts / kNB), ws.dinv_base(), ws.info(),
+                     ws.flags(), s1, flow_rhs, flow_clock);
+  });
+  launch_flow_end(A.view(), flow_rhs, n, y, ws.info(), flow_clock, flow_host, y == z, s1);
+  ws.factored = A.tile_raw(0, 0);
+  EXA_HIP(hipStreamSynchronize(s1));
+  return (int)flow_host[0];
+}
+
 double Context::loglik(KernelId kid, const double* theta, int metric, double* logdet_out, double* dotp_out,
                        int* info, int band) {
   if (band < 0) throw std::invalid_argument("diag_thick must be positive");
@@ -780,35 +811,15 @@ double Context::loglik(KernelId kid, const double* theta, int metric, double* lo
     // sums, without a host synchronisation between them and with the results
     // written to pinned host memory (n = 400: 281 -> 146 us, n = 1,600: 679 -> 486 us against separate
     // solve launches and five synchronisations).
-    const long nb = (N + kNB - 1) / kNB;
-    if (!flow_rhs) {
-      int wall_khz = 0;
-      EXA_HIP(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, 0));
-      wall_rate = wall_khz > 0 ? 1e3 * wall_khz : 1e8;
-      EXA_HIP(hipMalloc(&flow_clock, 2 * sizeof(long long)));
-      EXA_HIP(hipHostMalloc(&flow_host, sizeof(double) * flow_end_doubles(N), hipHostMallocDefault));
-      EXA_HIP(hipMalloc(&flow_rhs, sizeof(double) * nb * 4096));
-      EXA_HIP(hipMemset(flow_rhs, 0, sizeof(double) * nb * 4096));
-      EXA_HIP(hipDeviceSynchronize());
-    }
-    const int q = ts / kNB;
     profiled("gen", 0.0, 4.0 * (double)N * (N + 1.0), s1,
              [&] { generate_covariance(C, kid, theta, l1, l1, metric, s1); });
-    launch_flow_begin(Zcpy.d, N, flow_rhs, ws.dinv_base(), nb * 4096, ws.info(), s1);
-    profiled("potrf_diag", potrf_flops(N), 0.0, s1, [&] {
-      launch_chol_flow(C.view(), C.pool_f64(), 0, 0, (int)nb, (int)nb, C.mt * q, ws.dinv_base(), ws.info(),
-                       ws.flags(), s1, flow_rhs, flow_clock);
-    });
-    launch_flow_end(C.view(), flow_rhs, N, work.d, ws.info(), flow_clock, flow_host, s1);
-    ws.factored = C.tile_raw(0, 0);
-    EXA_HIP(hipStreamSynchronize(s1));
+    const int inf = factor_solve(C, Zcpy.d, work.d);
     double dotp = 0.0, logdet = 0.0;
     for (long b = 0; b < (N + 255) / 256; ++b) {
       dotp += flow_host[4 + 2 * b];
       logdet += flow_host[5 + 2 * b];
     }
     logdet *= 2.0;
-    const int inf = (int)flow_host[0];
     if (info) *info = inf;
     const double t4 = wall_seconds();
     if (Profiler::get().enabled()) Profiler::get().collect();

@@ -248,9 +248,14 @@ class Context {
   double loglik(KernelId kid, const double* theta, int metric, double* logdet_out, double* dotp_out, int* info,
                 int band = 0);
   void ensure_partial(long n);
-  // Right-hand side row, clock and result mirror of the one-launch
-  // evaluation, allocated on first use.
+  // A, which satisfies one_launch, factored with y = L^-1 z in the same
+  // launch; the failing column or 0.  y may be z, which a failure leaves as
+  // it was.
+  int factor_solve(TileMatrix& A, const double* z, double* y);
+  // Right-hand side row, clock and result mirror of factor_solve, allocated
+  // on first use and again for a larger matrix.
   double* flow_rhs = nullptr;
+  long flow_blocks = 0;  // capacity, 64-row blocks
   long long* flow_clock = nullptr;
   double* flow_host = nullptr;  // pinned
   double wall_rate = 1e8;       // ticks per second of flow_clock

@@ -90,15 +90,16 @@ void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int
                       long long* clock = nullptr);
 // Before the first launch of a factorisation: info <- 0 and the nd doubles
 // of dinv that it will write unset.  launch_flow_begin: the same and z into
-// the first row of rhs.
+// the first row of rhs, zeros behind it up to nd / 64 columns.
 void launch_flow_reset(double* dinv, long nd, int* info, hipStream_t s);
 void launch_flow_begin(const double* z, long n, double* rhs, double* dinv, long nd, int* info, hipStream_t s);
 // y <- the first row of rhs; host[0] <- info, host[1] <- clock[1] - clock[0],
 // host[4 + 2 b], host[5 + 2 b] <- sums of y^2 and log L_ii over rows
 // [256 b, 256 (b + 1)); flow_end_doubles(n) doubles of pinned host memory.
+// keep: y is left alone when info is not 0.
 long flow_end_doubles(long n);
 void launch_flow_end(const TileView& v, const double* rhs, long n, double* y, const int* info, const long long* clock,
-                     double* host, hipStream_t s);
+                     double* host, bool keep, hipStream_t s);
 // A(m,n) -= sum_{p < np} A(m,k+p) A(n,k+p)^T for n in [col_lo, col_hi],
 // m in [n, mt); np = 1 or 2 (col_lo >= k + np).
 void launch_tile_update(const TileView& v, int k, int np, int col_lo, int col_hi, hipStream_t s);
