@@ -31,6 +31,14 @@
 // Memory: finished blocks are written through to the device's coherence
 // point (agent-scope stores), then the row's counter is released at agent
 // scope; a waiting work-group acquires at agent scope before it reads.
+// Counters only rise.  A row's counter is stored by one task after another,
+// each of which has waited for the value before (T_ij and D_j for row i at
+// l = j - 1), so stores are enough there.  The diagonal's is not: D_{j+1}
+// reads inv(L_jj) itself (fetch_inverse) and may store its value before D_j
+// has, so both raise it (flag_raise); a plain store of D_j that arrived last
+// would leave the T tasks of column j + 1 waiting for good.  A work-group
+// claims, and waits for the claim, after its last counter store, so that all
+// of them have arrived when it counts itself out and the last one resets.
 #include "common.hpp"
 #include "besselk.hpp"
 #include "flow.hpp"
@@ -789,7 +797,7 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
       store_through(dinv + 16 * bi + r + (16 * bj + c) * 64, Xs[blk16(bi, bj) + tid]);
   stores_done();
   __syncthreads();
-  if (tid == 0) flag_set(a.flags + kDiag, j - a.j0 + 1);
+  if (tid == 0) flag_raise(a.flags + kDiag, j - a.j0 + 1);
   __builtin_amdgcn_s_setprio(0);
   // off the chain: the factor block itself, the zeros above it
   gdouble* out = (gdouble*)(uintptr_t)cjj;

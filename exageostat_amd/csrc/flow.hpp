@@ -14,8 +14,13 @@ __device__ __forceinline__ int flag_get(const int* f) {
 // Every wave's stores have left the wave; to be called before the barrier
 // that precedes flag_set.
 __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ void flag_set(int* f, int v) {
+__host__ __device__ __forceinline__ void flag_set(int* f, int v) {
   __hip_atomic_store(f, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The same for a counter whose writers have not seen each other's values: it
+// never goes back, in whatever order their stores arrive.
+__host__ __device__ __forceinline__ void flag_raise(int* f, int v) {
+  __hip_atomic_fetch_max(f, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <class T>
 __device__ __forceinline__ void store_through(T* p, T v) {
