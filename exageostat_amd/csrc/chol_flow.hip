@@ -330,8 +330,11 @@ __device__ __forceinline__ void fetch_inverse(const FlowArgs& a, int j, double* 
 #pragma unroll
     for (int t = 0; t < 10; ++t) unset |= __double_as_longlong(v[t]) == kUnset;
     if (!unset || last) break;
+    // The last look follows the counter by an acquire at agent scope, which
+    // pairs with its release: it sees the whole inverse.
     last = flag_get(a.flags + kDiag) > j - a.j0;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   }
   __syncthreads();  // the LDS may still be read
 #pragma unroll
