@@ -319,8 +319,12 @@ __global__ void __launch_bounds__((ClassCfg<kF64, BS>::C::NT))
     const int m = pk >> 16;
     const int n = pk & 0xFFFF;
     if (m == n && (bi + 1) * bm <= bj * bn) continue;
-    if (cl == 0) class_update<kF64, BS>(v, k, m, n, bi, bj, split, lds);
-    else if (cl == 1) class_update<F32CLS, BS>(v, k, m, n, bi, bj, split, lds);
+    if (cl == 0) {
+      // gemm_nt_acc stores to LDS before its first barrier; a BF16 block before
+      // it ends without one, its last reads and copies still under way.
+      __syncthreads();
+      class_update<kF64, BS>(v, k, m, n, bi, bj, split, lds);
+    } else if (cl == 1) class_update<F32CLS, BS>(v, k, m, n, bi, bj, split, lds);
     else class_update<kF32B, BS>(v, k, m, n, bi, bj, split, lds);
   }
 }
