@@ -949,8 +949,10 @@ __global__ void __launch_bounds__(256) k_flow_reset(double* dinv, long nd, int* 
   for (long e = c; e < nd; e += (long)gridDim.x * 256) reinterpret_cast<long long*>(dinv)[e] = kUnset;
 }
 
-// After it: y = L^-1 z into a vector, and per work-group the sums of y^2 and
-// of log L_ii over 256 rows, written with info to host memory.
+// After it: y = L^-1 z into a vector (zeros into its padding, which a solve on
+// the tiles may have left as NaN and the transposed solve reads), and per
+// work-group the sums of y^2 and of log L_ii over 256 rows, written with info
+// to host memory.
 __global__ void __launch_bounds__(256) k_flow_end(TileView v, const double* rhs, long n, double* y, const int* info,
                                                   const long long* clock, double* host, bool keep) {
   __shared__ double red[2][4];
@@ -964,6 +966,8 @@ __global__ void __launch_bounds__(256) k_flow_end(TileView v, const double* rhs,
     const long r = i - (long)k * v.ts;
     const double l = tile_f64(v, k, k)[r + r * v.ts];
     if (l > 0.0) d = log(l);
+  } else if (i < (long)v.mt * v.ts && !keep) {
+    y[i] = 0.0;
   }
   s = wave_sum(s);
   d = wave_sum(d);
@@ -972,7 +976,7 @@ __global__ void __launch_bounds__(256) k_flow_end(TileView v, const double* rhs,
     red[1][threadIdx.x >> 6] = d;
   }
   __syncthreads();
-  if (threadIdx.x < 2) {
+  if (threadIdx.x < 2 && (long)blockIdx.x * 256 < n) {
     const double* r = red[threadIdx.x];
     host[4 + 2 * blockIdx.x + threadIdx.x] = (r[0] + r[1]) + (r[2] + r[3]);
   }
@@ -1025,8 +1029,9 @@ void launch_flow_reset(double* dinv, long nd, int* info, hipStream_t s) {
 long flow_end_doubles(long n) { return 4 + 2 * ((n + 255) / 256); }
 void launch_flow_end(const TileView& v, const double* rhs, long n, double* y, const int* info, const long long* clock,
                      double* host, bool keep, hipStream_t s) {
-  hipLaunchKernelGGL(k_flow_end, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, v, rhs, n, y, info, clock, host,
-                     keep);
+  const long padded = (long)v.mt * v.ts;
+  hipLaunchKernelGGL(k_flow_end, dim3((unsigned)((padded + 255) / 256)), dim3(256), 0, s, v, rhs, n, y, info, clock,
+                     host, keep);
   EXA_HIP(hipGetLastError());
 }
 

@@ -93,10 +93,10 @@ void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int
 // the first row of rhs, zeros behind it up to nd / 64 columns.
 void launch_flow_reset(double* dinv, long nd, int* info, hipStream_t s);
 void launch_flow_begin(const double* z, long n, double* rhs, double* dinv, long nd, int* info, hipStream_t s);
-// y <- the first row of rhs; host[0] <- info, host[1] <- clock[1] - clock[0],
+// y (mt * ts doubles) <- the first row of rhs and zeros; host[0] <- info, host[1] <- clock[1] - clock[0],
 // host[4 + 2 b], host[5 + 2 b] <- sums of y^2 and log L_ii over rows
 // [256 b, 256 (b + 1)); flow_end_doubles(n) doubles of pinned host memory.
-// keep: y is left alone when info is not 0.
+// keep: y is left alone when info is not 0, and its padding always.
 long flow_end_doubles(long n);
 void launch_flow_end(const TileView& v, const double* rhs, long n, double* y, const int* info, const long long* clock,
                      double* host, bool keep, hipStream_t s);
