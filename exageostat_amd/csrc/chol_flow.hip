@@ -72,6 +72,11 @@ __device__ __forceinline__ void fma_row_lane(double& y, double x, double z) {
   asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(y) : "v"(x), "v"(z), "n"(N));
 }
 
+// Pivots for which recip3 and rsqrt_pair hold with a margin; a panel with a
+// positive one outside (subnormal, near overflow, infinite) is factored again
+// by divisions and roots (diag_panel_slow).
+constexpr double kPivotMin = 0x1p-1000, kPivotMax = 0x1p+1000;
+
 // 1/y for normal y: the hardware estimate (relative error 4.7e-8 measured)
 // with one third-order step, three dependent operations.
 __device__ __forceinline__ double recip3(double y) {
@@ -174,8 +179,9 @@ __device__ __forceinline__ void panel_scale(double (&d)[16], double (&a)[16], do
 // as rows of L^-T.  root: the diagonal entry of L of the lane's column (d
 // holds it as a product, one rounding further off).  Returns the mask of
 // columns whose pivot is not positive; those and all later columns are NaN
-// then.
-__device__ __forceinline__ unsigned panel16(double (&d)[16], double (&a)[16], double& root, int lane) {
+// then.  again: the first pivot outside the range that this serves is a
+// positive one; the results are not to be used then.
+__device__ __forceinline__ unsigned panel16(double (&d)[16], double (&a)[16], double& root, bool& again, int lane) {
   int l16 = lane & 15;
   asm("" : "+v"(l16));  // comparisons with it stay here
   double rs;
@@ -185,8 +191,13 @@ __device__ __forceinline__ unsigned panel16(double (&d)[16], double (&a)[16], do
   panel_columns<0>(d, a, own, l16, -d[0] * r, -a[0] * r);
   rsqrt_pair(own, rs, root);
   panel_scale<0>(d, a, rs);
+  again = false;
+  const unsigned odd = (unsigned)__ballot(!(own >= kPivotMin && own <= kPivotMax)) & 0xffffu;
+  if (!odd) return 0;
   const unsigned bad = (unsigned)__ballot(!(own > 0.0)) & 0xffffu;
-  if (bad) {
+  if (__builtin_ctz(odd) < __builtin_ctz(bad | 0x10000u)) {
+    again = true;
+  } else {
     const int first = __builtin_ctz(bad);
 #pragma unroll
     for (int c = 0; c < 16; ++c)
@@ -637,6 +648,49 @@ __device__ __forceinline__ void inverse_put(double* Xs, const dx4& y, int p, int
   for (int e = 0; e < 4; ++e) dst[e * 64] = x[e];
 }
 
+// The wave's LDS accesses before it are done, and seen by all its lanes.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// Panel p of the diagonal block, by one wave, in LDS and with a root and
+// divisions per column: for pivots at the ends of the range of doubles and
+// infinite ones (whose column becomes zero), which diag_panel's reciprocals
+// do not serve.  Rare, so its time does not matter.
+__device__ __forceinline__ void diag_panel_slow(const FlowArgs& a, int j, int p, double* Ls, double* Xs, int lane) {
+  asm("" : "+v"(lane));  // nothing of this is computed ahead of its call
+  double* D = Ls + blk16(p, p);
+  const int bi = p + (lane >> 4);
+  // the lane's row of 16, step apart: of an identity (lanes 0 .. 15, in Xs) or
+  // of a block row below
+  double* row = lane < 16 ? Xs + blk16(p, p) + 16 * lane : Ls + blk16(bi < 4 ? bi : p, p) + (lane & 15);
+  const int step = lane < 16 ? 1 : 16;
+  const bool mine = bi < 4;
+  if (lane < 16)
+    for (int e = 0; e < 16; ++e) row[e] = e == lane ? 1.0 : 0.0;
+  wave_sync();
+#pragma unroll 1
+  for (int c = 0; c < 16; ++c) {
+    const double piv = D[c * 16 + c];
+    const bool bad = !(piv > 0.0);
+    if (bad && lane == 0) atomicCAS(a.info, 0, j * kNB + 16 * p + c + 1);
+    const double s = bad ? __builtin_nan("") : sqrt(piv);
+    wave_sync();
+    if (lane < 16 && lane >= c) D[c * 16 + lane] = lane > c ? D[c * 16 + lane] / s : s;
+    if (mine) row[c * step] /= s;
+    wave_sync();
+#pragma unroll 1
+    for (int e = c + 1; e < 16; ++e) {
+      const double l = D[c * 16 + e];
+      if (lane < 16 && lane >= e) D[e * 16 + lane] -= D[c * 16 + lane] * l;
+      if (mine) row[e * step] -= row[c * step] * l;
+    }
+    wave_sync();
+  }
+}
+
 // Panel p of the diagonal block, by one wave.
 __device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, double* Ls, double* Xs, const double* id,
                                            int lane) {
@@ -652,7 +706,12 @@ __device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, doub
     c[e] = cc[e * 16];
   }
   double root;
-  const unsigned bad = panel16(d, c, root, lane);
+  bool again;
+  const unsigned bad = panel16(d, c, root, again, lane);
+  if (again) {
+    diag_panel_slow(a, j, p, Ls, Xs, lane);
+    return;
+  }
   if (bad && lane == 0) atomicCAS(a.info, 0, j * kNB + 16 * p + __builtin_ctz(bad) + 1);
   if (lane < 16) {
     double* dst = Xs + blk16(p, p) + lane * 16;
