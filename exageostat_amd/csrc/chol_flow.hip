@@ -240,7 +240,7 @@ struct FlowArgs {
   int* info;
   int* flags;
   double* rhs;    // one more block row, i_end: 64 x 64 blocks in sequence, its rows solved with the factor
-  long long* clock;  // receives the first and the last work-group's wall clock
+  long long* clock;  // receives the wall clock of the start, the end, and when the last block is factored
 };
 
 namespace {
@@ -598,6 +598,7 @@ __device__ __forceinline__ void task_rhs(const FlowArgs& a, int j, double* lds, 
     l = upto;
   }
   wait_diag(a, j - a.j0 + 1);
+  if (tid == 0 && j + 1 == a.j1) a.clock[2] = wall_clock64();
   load_inverse(a.dinv + (long)j * 4096, lds, wave, lane);
   wait_vmcnt<0>();
   __syncthreads();
@@ -1011,7 +1012,7 @@ __global__ void __launch_bounds__(256) k_flow_reset(double* dinv, long nd, int* 
 // After it: y = L^-1 z into a vector (zeros into its padding, which a solve on
 // the tiles may have left as NaN and the transposed solve reads), and per
 // work-group the sums of y^2 and of log L_ii over 256 rows, written with info
-// to host memory.
+// and the phases' ticks to host memory.
 __global__ void __launch_bounds__(256) k_flow_end(TileView v, const double* rhs, long n, double* y, const int* info,
                                                   const long long* clock, double* host, bool keep) {
   __shared__ double red[2][4];
@@ -1041,7 +1042,9 @@ __global__ void __launch_bounds__(256) k_flow_end(TileView v, const double* rhs,
   }
   if (i == 0) {
     host[0] = *info;
-    host[1] = (double)(clock[1] - clock[0]);
+    host[1] = (double)(clock[2] - clock[0]);
+    host[2] = (double)(clock[1] - clock[2]);
+    host[3] = (double)(wall_clock64() - clock[1]);
   }
 }
 

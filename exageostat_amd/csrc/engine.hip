@@ -775,7 +775,7 @@ int Context::factor_solve(TileMatrix& A, const double* z, double* y) {
     int wall_khz = 0;
     EXA_HIP(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, 0));
     wall_rate = wall_khz > 0 ? 1e3 * wall_khz : 1e8;
-    EXA_HIP(hipMalloc(&flow_clock, 2 * sizeof(long long)));
+    EXA_HIP(hipMalloc(&flow_clock, 3 * sizeof(long long)));
   }
   if (flow_blocks < nb) {
     if (flow_rhs) (void)hipFree(flow_rhs);
@@ -823,12 +823,14 @@ double Context::loglik(KernelId kid, const double* theta, int metric, double* lo
     if (info) *info = inf;
     const double t4 = wall_seconds();
     if (Profiler::get().enabled()) Profiler::get().collect();
-    // One device interval: the factorisation with the solve in it.  The rest
-    // is generation and launches; the sums take a few microseconds.
+    // Device intervals: the factorisation (with all of the solve but its last
+    // block inside), the rest of the solve, and the sums of both results.
+    // Generation has the rest, launches and the closing synchronisation too.
     last.total = t4 - t0;
     last.facto = std::min(flow_host[1] / wall_rate, last.total);
-    last.gen = last.total - last.facto;
-    last.logdet = last.solve = 0.0;
+    last.solve = std::min(flow_host[2] / wall_rate, last.total - last.facto);
+    last.logdet = std::min(flow_host[3] / wall_rate, last.total - last.facto - last.solve);
+    last.gen = last.total - last.facto - last.solve - last.logdet;
     if (logdet_out) *logdet_out = logdet;
     if (dotp_out) *dotp_out = dotp;
     return -0.5 * dotp - 0.5 * logdet - (N / 2.0) * std::log(2.0 * M_PI);

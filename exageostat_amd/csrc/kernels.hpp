@@ -83,7 +83,8 @@ void launch_gen_spacetime(const TileView& v, const SpaceTimeParams& P, long p_of
 // blocks [j1, j_pad)).  flags: chol_flow_flags() ints, zero before the first
 // launch and left zero by each.  rhs (whole matrix only): one more block row
 // of 64 x 64 blocks in sequence, solved with the factor (rows r <- r L^-T).
-// clock: receives the wall clock at the start and the end.
+// clock: receives the wall clock at the start [0], the end [1] and when the
+// last diagonal block is factored [2].
 long chol_flow_flags(int mt, int ts);
 void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int j1, int i_end, int j_pad,
                       double* dinv, int* info, int* flags, hipStream_t s, double* rhs = nullptr,
@@ -93,7 +94,8 @@ void launch_chol_flow(const TileView& v, double* pool, int tile_col, int j0, int
 // the first row of rhs, zeros behind it up to nd / 64 columns.
 void launch_flow_reset(double* dinv, long nd, int* info, hipStream_t s);
 void launch_flow_begin(const double* z, long n, double* rhs, double* dinv, long nd, int* info, hipStream_t s);
-// y (mt * ts doubles) <- the first row of rhs and zeros; host[0] <- info, host[1] <- clock[1] - clock[0],
+// y (mt * ts doubles) <- the first row of rhs and zeros; host[0] <- info, host[1 .. 3] <-
+// ticks of the factorisation, of the solve after it, and from there to here,
 // host[4 + 2 b], host[5 + 2 b] <- sums of y^2 and log L_ii over rows
 // [256 b, 256 (b + 1)); flow_end_doubles(n) doubles of pinned host memory.
 // keep: y is left alone when info is not 0, and its padding always.

@@ -284,9 +284,9 @@ typedef struct {
   int status;           /* 0 ok; >0 first non-positive pivot + 1; <0 error   */
   double logdet;        /* last log|Sigma|                                   */
   double time_gen;      /* last evaluation, seconds per phase                */
-  double time_facto;    /* up to 12,800 rows in FP64 with the forward solve   */
-  double time_logdet;   /* inside it; time_logdet and time_solve are then 0   */
-  double time_solve;
+  double time_facto;    /* Up to 12,800 rows in FP64 the forward solve runs   */
+  double time_logdet;   /* inside the factorisation: time_solve is then what  */
+  double time_solve;    /* it takes beyond it, and time_logdet both sums.     */
   double time_total;
   double mp_fp32_corr;  /* mixed: off-diagonal tiles whose largest
                            correlation is >= this stay FP32, others BF16     */
