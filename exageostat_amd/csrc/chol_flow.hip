@@ -966,15 +966,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 
 template <int R, bool MIXED, bool RHS = false>
 void launch_flow(const FlowArgs& a, hipStream_t s) {
-  static int cus = 0, slots = 0;
-  if (!slots) {
+  struct Room {
+    int cus, slots;
+  };
+  static const Room room = [] {  // by the first thread that comes here; others wait for it
     int dev = 0, n = 0, occ = 1;
     EXA_HIP(hipGetDevice(&dev));
     EXA_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
     EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_chol_flow<R, MIXED, RHS>, 256, 0));
-    cus = n;
-    slots = n * (occ > 0 ? occ : 1);
-  }
+    return Room{n, n * (occ > 0 ? occ : 1)};
+  }();
   // Small matrices wait for the chain, which is faster without a second
   // work-group on its CU (more LDS than half a CU's keeps it away); larger
   // ones for the sums.  Likelihood, one / two work-groups per CU: n = 2,000
@@ -982,7 +983,7 @@ void launch_flow(const FlowArgs& a, hipStream_t s) {
   // 6,000 2,270 / 2,000.
   constexpr int kChainBlocks = 70, kMoreLds = 16384;
   const bool alone = a.pool && a.i_end - a.j0 <= kChainBlocks;
-  const int most = alone ? cus : slots;
+  const int most = alone ? room.cus : room.slots;
   long tasks = 0;
   for (int j = a.j0; j < a.j1 && tasks < most; ++j)
     tasks += 1 + RHS + row_groups<R, MIXED>(rows_from(j, a.j1), a.i_end, a.q);

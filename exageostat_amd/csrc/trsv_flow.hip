@@ -292,14 +292,13 @@ int strip_parts(int ts) { return (ts / kNB + 3) / 4; }
 
 template <bool TRANS, bool MIXED, int PER>
 void launch(const TrsvArgs& a, hipStream_t s) {
-  static int slots = 0;
-  if (!slots) {
+  static const int slots = [] {  // by the first thread that comes here; others wait for it
     int dev = 0, cus = 0, occ = 1;
     EXA_HIP(hipGetDevice(&dev));
     EXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_trsv_flow<TRANS, MIXED, PER>, 256, 0));
-    slots = cus * (occ > 0 ? occ : 1);
-  }
+    return cus * (occ > 0 ? occ : 1);
+  }();
   const long tasks = PER == 1 ? a.v.mt : (long)a.q * a.parts * (2 * a.v.mt - 1) + a.v.mt;
   hipLaunchKernelGGL((k_trsv_flow<TRANS, MIXED, PER>), dim3((unsigned)(tasks < slots ? tasks : slots)), dim3(256), 0, s,
                      a);
