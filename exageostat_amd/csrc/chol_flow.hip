@@ -66,7 +66,8 @@ __device__ __forceinline__ double row_lane(double x) {
 // multiply-add (the compiler makes a move of its own of it: three
 // instructions per pair of updates instead of two).  x must not come from
 // one of the two preceding vector instructions: panel_columns waits before
-// it reads the pivot, on which z depends.
+// it reads the pivot, on which z depends (tests/test_flow_wait_states_cpu.py
+// looks for both in the generated code).
 template <int N>
 __device__ __forceinline__ void fma_row_lane(double& y, double x, double z) {
   asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(y) : "v"(x), "v"(z), "n"(N));
