@@ -994,8 +994,8 @@ void launch_flow(const FlowArgs& a, hipStream_t s) {
 }
 
 // Before a factorisation: info = 0 and the inverses unset; with a right-hand
-// side also z into the first row of its blocks (zero beyond it since their
-// allocation: the rows never mix).
+// side also z into the first row of its blocks.  The other rows are zero since
+// their allocation, or NaN once a factorisation has failed: the rows never mix.
 __global__ void __launch_bounds__(256) k_flow_begin(const double* z, long n, double* rhs, double* dinv, long nd,
                                                     int* info) {
   const long c = (long)blockIdx.x * 256 + threadIdx.x;
