@@ -514,16 +514,40 @@ __device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], d
 typedef __attribute__((address_space(1))) double gdouble;
 typedef __attribute__((address_space(1))) float gfloat;
 
-// acc = -C for the wave's 16 rows of a 64 x 64 block: the products are added
-// to it, so that nothing is left to read when the last of them is done.
+// The wave's 16 rows of a 64 x 64 block.
 template <class TA>
-__device__ __forceinline__ void block_neg(const char* blk, long ts, int wave, int lane, dx4 (&acc)[4]) {
+__device__ __forceinline__ void block_load(const char* blk, long ts, int wave, int lane, dx4 (&c)[4]) {
   typedef __attribute__((address_space(1))) const TA gT;
   gT* G = (gT*)(uintptr_t)blk + 16 * wave + (lane & 15) + (long)(lane >> 4) * ts;
 #pragma unroll
   for (int f = 0; f < 4; ++f)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) acc[f][v] = -(double)G[(long)(16 * f + 4 * v) * ts];
+    for (int v = 0; v < 4; ++v) c[f][v] = (double)G[(long)(16 * f + 4 * v) * ts];
+}
+
+// The sums of products run from zero over kSumBlocks block columns each and
+// are then subtracted from C.  Added to -C one after another, every product
+// would be rounded at C's magnitude, and in one long sum at that sum's: error
+// of z^T C^-1 z (rms, against 80-bit arithmetic, exponential kernel, nugget 0 /
+// 0.05) at n = 5,000 58e-16 / 28e-16 and at 9,000 68e-16 / 75e-16 from -C, 15e-16 /
+// 8e-16 and 17e-16 / 10e-16 from zero, 7e-16 / 8e-16 and 11e-16 / 7e-16 like this; the
+// time is the same.
+constexpr int kSumBlocks = 16;
+template <int N>
+__device__ __forceinline__ void sum_zero(dx4 (&acc)[N]) {
+#pragma unroll
+  for (int f = 0; f < N; ++f) acc[f] = dx4{0.0, 0.0, 0.0, 0.0};
+}
+template <int N>
+__device__ __forceinline__ void sum_flush(dx4 (&acc)[N], dx4 (&c)[N]) {
+#pragma unroll
+  for (int f = 0; f < N; ++f) c[f] -= acc[f];
+  sum_zero(acc);
+}
+// acc = -(C - acc)
+__device__ __forceinline__ void block_sub(dx4 (&acc)[4], const dx4 (&c)[4]) {
+#pragma unroll
+  for (int f = 0; f < 4; ++f) acc[f] -= c[f];
 }
 
 template <class TA>
@@ -549,16 +573,34 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
   // The row that D_{j+2} waits for goes ahead of the group's others.  Its
   // counter is then D_{j+2}'s: it is not stored again with theirs.
   const bool early = i0 == j + 2 && nr > 1;
-  dx4 acc[R][4], none[3];
+  // Two rows' C is read ahead of everything (at the end, n = 1,600 took 373 us
+  // instead of 358); for three there are no registers, and it is read row by
+  // row, the first during the wait for the inverse.
+  constexpr int AHEAD = R < 3 ? R : 1;
+  dx4 acc[R][4], c[AHEAD][4], none[3];
+  auto load_c = [&](int p) {
+    block_load<TA>(block_ptr(a, ra[p < R ? p : 0], j, (int)sizeof(TA)), ts, wave, lane, c[p % AHEAD]);
+  };
+  if constexpr (AHEAD == R) {
 #pragma unroll
-  for (int p = 0; p < R; ++p) block_neg<TA>(block_ptr(a, ra[p], j, (int)sizeof(TA)), ts, wave, lane, acc[p]);
-  int l = a.j0;
+    for (int p = 0; p < R; ++p) load_c(p);
+  }
+#pragma unroll
+  for (int p = 0; p < R; ++p) sum_zero(acc[p]);
+  int l = a.j0, have = l, flush = l + kSumBlocks;
   while (l < j) {
-    int upto = a.j0 + wait_rows(a, j, i0, i0 + nr - 1, i0 + (nr > 1 ? 1 : 0), l - a.j0, sh);
-    if (upto > j) upto = j;
+    if (have <= l) have = a.j0 + wait_rows(a, j, i0, i0 + nr - 1, i0 + (nr > 1 ? 1 : 0), l - a.j0, sh);
+    int upto = have < j ? have : j;
+    if (AHEAD == R && upto > flush) upto = flush;
     flow_gemm<R, TA, false>(a, acc, none, ra, rj, l, upto, lds);
     l = upto;
+    if (AHEAD == R && l == flush) {
+#pragma unroll
+      for (int p = 0; p < R; ++p) sum_flush(acc[p], c[p % AHEAD]);
+      flush += kSumBlocks;
+    }
   }
+  if constexpr (AHEAD < R) load_c(0);
   wait_diag(a, j - a.j0 + 1);  // its barrier also ends the reads of the ring
   load_inverse(a.dinv + (long)j * 4096, lds, wave, lane);
   wait_vmcnt<0>();
@@ -567,6 +609,8 @@ __device__ __forceinline__ void task_rows(const FlowArgs& a, int i0, int nr, int
   for (int p = 0; p < R; ++p) {
     if (p < nr) {
       dx4 x[4];
+      block_sub(acc[p], c[p % AHEAD]);
+      if (p + AHEAD < R) load_c(p + AHEAD);
       times_inverse(acc[p], x, lds, lane);
       block_store<TA>(block_ptr(a, ra[p], j, (int)sizeof(TA)), ts, wave, lane, x);
     }
@@ -588,15 +632,21 @@ __device__ __forceinline__ void task_rhs(const FlowArgs& a, int j, double* lds, 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const Row rj = row_of(a, j);
   const Row none_row[1] = {rj};
-  dx4 acc[1][4], none[3];
+  dx4 acc[1][4], c[4], none[3];
   char* blk = reinterpret_cast<char*>(a.rhs + (long)j * 4096);
-  block_neg<double>(blk, kNB, wave, lane, acc[0]);
-  int l = a.j0;
+  block_load<double>(blk, kNB, wave, lane, c);
+  sum_zero(acc[0]);
+  int l = a.j0, have = l, flush = l + kSumBlocks;
   while (l < j) {
-    int upto = a.j0 + wait_rows(a, j, a.i_end, j, a.i_end, l - a.j0, sh);
-    if (upto > j) upto = j;
+    if (have <= l) have = a.j0 + wait_rows(a, j, a.i_end, j, a.i_end, l - a.j0, sh);
+    int upto = have < j ? have : j;
+    if (upto > flush) upto = flush;
     flow_gemm<1, double, false, true>(a, acc, none, none_row, rj, l, upto, lds);
     l = upto;
+    if (l == flush) {
+      sum_flush(acc[0], c);
+      flush += kSumBlocks;
+    }
   }
   wait_diag(a, j - a.j0 + 1);
   if (tid == 0 && j + 1 == a.j1) a.clock[2] = wall_clock64();
@@ -604,6 +654,7 @@ __device__ __forceinline__ void task_rhs(const FlowArgs& a, int j, double* lds, 
   wait_vmcnt<0>();
   __syncthreads();
   dx4 x[4];
+  block_sub(acc[0], c);
   times_inverse(acc[0], x, lds, lane);
   block_store<double>(blk, kNB, wave, lane, x);
   stores_done();
@@ -615,16 +666,18 @@ __device__ __forceinline__ void task_rhs(const FlowArgs& a, int j, double* lds, 
 // factor's and the inverse's 16 x 16 blocks, and a 16 x 16 identity.
 constexpr int kLs = 4096, kXs = kLs + 2560, kId = kXs + 2560, kDiagLds = kId + 256;
 
-// S(bi, bj) -= L(bi, p) L(bj, p)^T
+// S(bi, bj) -= L(bi, p) L(bj, p)^T, the product summed by itself like the long
+// sums
 __device__ __forceinline__ void diag_update(double* Ls, int bi, int bj, int p, int lane) {
   double* S = Ls + blk16(bi, bj) + lane;
   const double* A = Ls + blk16(bi, p) + lane;
   const double* B = Ls + blk16(bj, p) + lane;
-  dx4 s = {S[0], S[64], S[128], S[192]};
+  const dx4 c = {S[0], S[64], S[128], S[192]};
+  dx4 s = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int e = 0; e < 4; ++e) s = mfma_f64(-B[e * 64], A[e * 64], s);
+  for (int e = 0; e < 4; ++e) s = mfma_f64(B[e * 64], A[e * 64], s);
 #pragma unroll
-  for (int e = 0; e < 4; ++e) S[e * 64] = s[e];
+  for (int e = 0; e < 4; ++e) S[e * 64] = c[e] - s[e];
 }
 // y += L(p, l) X(l, b); y: lane l, element v at row l/16 + 4 v, column l%16.
 __device__ __forceinline__ void inverse_sum(const double* Ls, const double* Xs, dx4& y, int p, int l, int b,
@@ -740,8 +793,8 @@ __device__ __forceinline__ void diag_panel(const FlowArgs& a, int j, int p, doub
 // panels and what lies between them, 1.7 X, 1.2 the first fragments and the
 // stores of X, 0.6 the last row of the inverse, 1.7 its way into the next
 // task's LDS; 17.0 before the hand-over read the inverse itself
-// (fetch_inverse), X was published ahead of the panels, the sums began with
-// the block they are subtracted from, and the waiting T tasks polled less.
+// (fetch_inverse), X was published ahead of the panels, the blocks that the
+// sums are subtracted from were read ahead, and the waiting T tasks polled less.
 __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds, int* sh) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -752,7 +805,7 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
   __builtin_amdgcn_s_setprio(2);
   double* Ls = lds + kLs;
   double* Xs = lds + kXs;
-  dx4 acc[1][4], dacc[3];
+  dx4 acc[1][4], dacc[3], cx[4], dc[3];
   char* cjj = block_ptr(a, rj, j, 8);
   const bool chained = j > a.j0;
   char* cp = nullptr;
@@ -762,19 +815,28 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
     diag_frag(wave, t < nd ? t : 0, bi, bj);
     gdouble* G = (gdouble*)(uintptr_t)cjj + 16 * bi + (lane & 15) + (long)(16 * bj + (lane >> 4)) * ts;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) dacc[t][v] = -G[(long)(4 * v) * ts];
+    for (int v = 0; v < 4; ++v) dc[t][v] = G[(long)(4 * v) * ts];
   }
+  sum_zero(dacc);
   if (chained) {
     cp = block_ptr(a, rj, j - 1, 8);
-    block_neg<double>(cp, ts, wave, lane, acc[0]);
+    block_load<double>(cp, ts, wave, lane, cx);
+    sum_zero(acc[0]);
     const Row rp[1] = {row_of(a, j - 1)};
-    int l = a.j0;
+    int l = a.j0, have = l, flush = l + kSumBlocks;
     while (l < j - 1) {
-      int upto = a.j0 + wait_rows(a, j, j - 1, j, j - 1, l - a.j0, sh);
-      if (upto > j - 1) upto = j - 1;
+      if (have <= l) have = a.j0 + wait_rows(a, j, j - 1, j, j - 1, l - a.j0, sh);
+      int upto = have < j - 1 ? have : j - 1;
+      if (upto > flush) upto = flush;
       flow_gemm<1, double, true>(a, acc, dacc, rp, rj, l, upto, lds);
       l = upto;
+      if (l == flush) {
+        sum_flush(acc[0], cx);
+        sum_flush(dacc, dc);
+        flush += kSumBlocks;
+      }
     }
+    block_sub(acc[0], cx);
   }
   // S's fragment t: minus X X^T when there is one, into LDS
   auto s_frag = [&](int t) {
@@ -787,7 +849,7 @@ __device__ __forceinline__ void task_diag(const FlowArgs& a, int j, double* lds,
       for (int e = 0; e < 16; ++e) dacc[t] = mfma_f64(Y[e * 64], X[e * 64], dacc[t]);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) Ls[blk16(bi, bj) + v * 64 + lane] = -dacc[t][v];
+    for (int v = 0; v < 4; ++v) Ls[blk16(bi, bj) + v * 64 + lane] = dc[t][v] - dacc[t][v];
   };
   if (chained) {
     fetch_inverse(a, j - 1, Xs, tid);
