@@ -512,7 +512,6 @@ __device__ __forceinline__ void flow_gemm(const FlowArgs& a, dx4 (&acc)[R][4], d
 }
 
 typedef __attribute__((address_space(1))) double gdouble;
-typedef __attribute__((address_space(1))) float gfloat;
 
 // The wave's 16 rows of a 64 x 64 block.
 template <class TA>

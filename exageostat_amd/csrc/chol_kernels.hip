@@ -103,9 +103,9 @@ void launch_trtri_tiles(const TileView& v, const double* dinv, double* xinv, hip
 // Tile pairs (m, n) with n in [col_lo, col_hi] and m in [n, mt), column by
 // column (consecutive pairs share the panel tile n).
 //
-// Persistent launch: gridDim.x work-groups (at most one per CU, fewer than
-// the CU count so the panel kernels of the critical path always find free
-// CUs) loop over the block list.  Work-groups are dispatched round-robin
+// Persistent launch: gridDim.x work-groups (one round of the whole chip, two
+// per CU; a panel on the other stream runs as they end) loop over the block
+// list.  Work-groups are dispatched round-robin
 // over the XCDs, so work-group w runs on XCD w % nx; each XCD gets a
 // contiguous slice of the block list and its work-groups walk it together,
 // which keeps the A/B row panels they share hot in that XCD's L2.

@@ -574,10 +574,10 @@ int tile_potrf(TileMatrix& A, CholWorkspace& ws, hipStream_t s1, hipStream_t s2,
     EXA_HIP(hipEventRecord(e, st));
     return e;
   };
-  // s1 carries the panel factorisations (one launch per tile column, on the
-  // CUs the persistent update leaves free); s2 carries the trailing updates: first
-  // the column that unblocks the next panel, then the rest, which overlaps
-  // with that panel on s1.
+  // s1 carries the panel factorisations (one launch per tile column); s2 carries
+  // the trailing updates: first the column that unblocks the next panel, then
+  // the rest, which overlaps with that panel on s1 as its work-groups find room
+  // between the persistent update's.
   // The FP64 factor's last kFlowBlocks block columns go into one dataflow
   // launch: its left-looking tasks reach 46-54 TFLOP/s against 60-70 of the
   // trailing update, but its chain costs 14 to 19 us per 64 columns where the tile

@@ -124,10 +124,8 @@ class CholWorkspace {
  public:
   ~CholWorkspace();
   void ensure(int mt, int ts);
-  double* dinv(int k) const { return dinv_ + (long)k * (ts_ / kNB) * 4096; }
   double* dinv_base() const { return dinv_; }
-  // Inverse of diagonal tile k (ts x ts, lower), filled by tile_potrf.
-  double* xinv(int k) const { return xinv_ + (long)k * ts_ * ts_; }
+  // Inverses of the diagonal tiles (ts x ts, lower), filled by tile_inverses.
   double* xinv_base() const { return xinv_; }
   // Partial results and zeroed flags of the triangular solves.
   double* tpart() const { return tpart_; }

@@ -472,47 +472,6 @@ __device__ __forceinline__ void acc_update(dx4 (&acc)[C::FM][C::FN], T* Cp, long
   }
 }
 
-// Cp[c + r*ldc] = acc(r, c): the block stored transposed.  Each lane keeps
-// one base address; the fragment offsets are uniform (a multiple of ldc plus
-// a constant), so the stores need no per-element address registers next to
-// the live accumulators.
-template <class C>
-__device__ __forceinline__ void acc_store_t(const dx4 (&acc)[C::FM][C::FN], double* Cp, long ldc) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = wave / C::WGN;
-  const int wn = wave - wm * C::WGN;
-  typedef __attribute__((address_space(1))) double gD;
-  gD* G = (gD*)(uintptr_t)(Cp + wn * C::WN + frag_col(lane) + (long)(wm * C::WM + frag_row(lane, 0)) * ldc);
-#pragma unroll
-  for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const long ro = (long)(i * 16 + 4 * v) * ldc;
-#pragma unroll
-      for (int j = 0; j < C::FN; ++j) G[ro + j * 16] = acc[i][j][v];
-    }
-}
-
-template <class C, class T = double>
-__device__ __forceinline__ void acc_load(dx4 (&acc)[C::FM][C::FN], const T* Cp, long ldc) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = wave / C::WGN;
-  const int wn = wave - wm * C::WGN;
-#pragma unroll
-  for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-    for (int j = 0; j < C::FN; ++j) {
-      const int c = wn * C::WN + j * 16 + frag_col(lane);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = wm * C::WM + i * 16 + frag_row(lane, v);
-        acc[i][j][v] = (double)Cp[r + (long)c * ldc];
-      }
-    }
-}
-
 // ---------------------------------------------------- FP32 matrix cores --
 // v_mfma_f32_16x16x4f32: operands as for the FP64 instruction (lane l
 // supplies A[l%16][l/16] and B[l/16][l%16]); result: lane l, element v holds

@@ -238,6 +238,8 @@ static void launch_class_bs(const TileView& v, int k, const int* pairs, long npa
     EXA_HIP(hipGetDevice(&dev));
     EXA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     EXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_update_class<CLS, BS>, ClassCfg<CLS, BS>::C::NT, 0));
+    // left free for the panel on the other stream; chosen when a panel was a
+    // chain of launches and not measured again for these tile sizes
     int reserve = 16;
     if (const char* e = getenv("EXAGEOSTAT_RESERVE_CUS")) reserve = atoi(e);
     if (reserve < 0 || reserve >= cus) reserve = 0;
