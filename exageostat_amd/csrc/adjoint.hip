@@ -95,7 +95,7 @@ void tile_potri_inplace(TileMatrix& A, CholWorkspace& ws, double* P, double* Q, 
                [&] { launch_takahashi_stage(v, k, P, Q, A.tile(k, k), 1, s, W, max_split, up, f32); });
     }
     profiled("potri_diag", 2.0 * below * rk * rk + rk * rk * rk / 3.0, 0.0, s,
-             [&] { launch_takahashi_stage(v, k, P, Q, A.tile(k, k), 2, s, nullptr, 1, up); });
+             [&] { launch_takahashi_stage(v, k, P, Q, A.tile(k, k), 2, s, nullptr, 1, up, f32); });
   }
   ws.factored = nullptr;
 }

@@ -224,19 +224,29 @@ __global__ void __launch_bounds__(256) k_sum_slabs(TileView v, int k, const doub
 // k_trmm_panel for the same reason (n = 12,000: 143 us a column
 // against 360 for all blocks of 192 x 192); without U
 // (Z_{k+i,k} read transposed) the register-staged core and its blocks.
+// full: the blocks above the diagonal too.  The recurrence keeps the rows of
+// Z consistent with L as they are computed; a lower triangle mirrored over the
+// upper one breaks that by the two sums' difference, which later columns
+// amplify.  With an FP32 column stage that difference is FP32 rounding: the
+// sweep's residual along z (bivariate kernel, tiles of 960) is 6.1e-6 with
+// both triangles and 1.4e-5 with a mirrored one at 40,000 rows, 1.6e-5 and
+// 5.1e-5 at 100,000, for the same time.  In FP64 (residual 1.15e-14 and
+// 1.30e-14, 12,000 rows, tiles of 192) the gradient shows no difference; its
+// sweep mirrors, and the inverse that the library returns is symmetric.
 template <class C, bool HAS_U>
 __global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(HAS_U ? 2 : 1)))
-    k_takahashi_diag(TileView v, int k, const double* P, double* Q, TileView U) {
+    k_takahashi_diag(TileView v, int k, const double* P, double* Q, TileView U, bool full) {
   __shared__ __attribute__((aligned(16))) double lds[HAS_U ? PipeLds<C, 2>::DOUBLES : C::LDS_DOUBLES];
   static_assert(C::BM == C::BN, "square blocks");
   const int qb = v.ts / C::BM;
-  const int per = qb * (qb + 1) / 2;
+  const int per = full ? qb * qb : qb * (qb + 1) / 2;
   const int i = (int)(blockIdx.x / per);
-  int bi, bj;
-  tri_decode(blockIdx.x - (long)i * per, bi, bj);
+  const int rem = (int)(blockIdx.x - (long)i * per);
+  int bi = rem % qb, bj = rem / qb;
+  if (!full) tri_decode(rem, bi, bj);
   const long ts = v.ts;
   const int j = k + i;
-  const long k0 = i == 0 ? (long)bi * C::BM : 0;
+  const long k0 = i == 0 ? (long)(bi > bj ? bi : bj) * C::BM : 0;
   const double* Pb = P + (long)j * ts * ts + bj * C::BN + k0 * ts;
   double* out = Q + (long)i * ts * ts + bi * C::BM + (long)bj * C::BN * ts;
   dx4 acc[C::FM][C::FN];
@@ -264,10 +274,11 @@ __global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(HAS_
 
 // Z_kk = sum_{i < cnt} Q_i (fixed order) from the sums' lower triangles, in
 // both triangles of out; one work-group per 64 x 64 block of the lower one.
-__global__ void __launch_bounds__(256) k_sum_diag(const double* Q, int cnt, int ts, double* out) {
+// full: from the whole sums, a work-group per block.
+__global__ void __launch_bounds__(256) k_sum_diag(const double* Q, int cnt, int ts, double* out, bool full) {
   __shared__ double blk[64][65];
-  int rb, cb;
-  tri_decode(blockIdx.x, rb, cb);
+  int rb = blockIdx.x % (ts / 64), cb = blockIdx.x / (ts / 64);
+  if (!full) tri_decode(blockIdx.x, rb, cb);
   const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
   const long len = (long)ts * ts;
   const double* q = Q + rb * 64 + lane + (long)(cb * 64 + grp * 16) * ts;
@@ -278,6 +289,11 @@ __global__ void __launch_bounds__(256) k_sum_diag(const double* Q, int cnt, int 
   for (int i = 0; i < cnt; ++i, q += len) {
 #pragma unroll
     for (int c = 0; c < 16; ++c) acc[c] += q[(long)c * ts];
+  }
+  if (full) {
+#pragma unroll
+    for (int c = 0; c < 16; ++c) out[rb * 64 + lane + (long)(cb * 64 + grp * 16 + c) * ts] = acc[c];
+    return;
   }
 #pragma unroll
   for (int c = 0; c < 16; ++c) blk[lane][grp * 16 + c] = acc[c];
@@ -488,12 +504,13 @@ static void takahashi_cfg(const TileView& v, int k, double* P, double* Q, double
     }
   }
   if (stage == 2) {
+    auto blocks = [&](int q) { return (unsigned)((below + 1) * (f32 ? q * q : q * (q + 1) / 2)); };
     if (U.ptr)
-      hipLaunchKernelGGL((k_takahashi_diag<CD, true>), dim3((unsigned)((below + 1) * (qd * (qd + 1) / 2))), dim3(CD::NT), 0, s,
-                         v, k, (const double*)P, Q, U);
+      hipLaunchKernelGGL((k_takahashi_diag<CD, true>), dim3(blocks(qd)), dim3(CD::NT), 0, s, v, k, (const double*)P, Q, U,
+                         f32);
     else
-      hipLaunchKernelGGL((k_takahashi_diag<C, false>), dim3((unsigned)((below + 1) * (qc * (qc + 1) / 2))), dim3(C::NT), 0, s,
-                         v, k, (const double*)P, Q, U);
+      hipLaunchKernelGGL((k_takahashi_diag<C, false>), dim3(blocks(qc)), dim3(C::NT), 0, s, v, k, (const double*)P, Q, U,
+                         f32);
   }
   EXA_HIP(hipGetLastError());
 }
@@ -535,8 +552,8 @@ void launch_takahashi_stage(const TileView& v, int k, double* P, double* Q, doub
   else takahashi_cfg<CT64, CT64, CT64>(v, k, P, Q, W, max_split, u, stage, s, f32);
   if (stage == 2) {
     const int q = v.ts / 64;
-    hipLaunchKernelGGL(k_sum_diag, dim3((unsigned)(q * (q + 1) / 2)), dim3(256), 0, s, (const double*)Q, v.mt - k, v.ts,
-                       Zkk);
+    hipLaunchKernelGGL(k_sum_diag, dim3((unsigned)(f32 ? q * q : q * (q + 1) / 2)), dim3(256), 0, s, (const double*)Q,
+                       v.mt - k, v.ts, Zkk, f32);
     EXA_HIP(hipGetLastError());
   }
 }
