@@ -263,8 +263,8 @@ double mixed_adjoint_loglik_grad(Context& ctx, KernelId kid, const double* theta
   }
   // The FP64 Sigma has served the refinement; it now receives the mixed
   // factor, whose Takahashi sweep gives the trace term.  With opt.grad_f32
-  // the sweep's column stage runs on the FP32 matrix cores: 0.74 against
-  // 1.01 s for l + gradient at n = 40,000 with a 0.01 nugget, the gradient
+  // the sweep's column stage runs on the FP32 matrix cores: 0.59 against
+  // 0.82 s for l + gradient at n = 40,000 with a 0.01 nugget, the gradient
   // as accurate as with the FP64 sweep there; on a worse-conditioned Sigma
   // (the parsimonious bivariate kernel at 50,000 locations) its rounding
   // error is 3.7e-3 of the largest component against 1.8e-4 from the mixed
